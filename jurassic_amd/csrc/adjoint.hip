@@ -100,7 +100,7 @@ __device__ __forceinline__ double u_vs(const float4 &r, double x, double &u) {
 }
 
 // FP32 path: col_eps_bis and col_u_bis with their slopes.
-__device__ __forceinline__ float col_eps_bis_vs(const float4 *col, int n, double x, float &s) {
+__device__ __forceinline__ float col_eps_bis_vs(Col col, int n, double x, float &s) {
   const float4 r0 = col[0];
   if (x < (double)r0.x) {
     s = fdiv(r0.y, r0.x);
@@ -119,7 +119,7 @@ __device__ __forceinline__ float col_eps_bis_vs(const float4 *col, int n, double
   return r.y + s * (float)(x - (double)r.x);
 }
 
-__device__ __forceinline__ double col_u_bis_vs(const float4 *col, int n, float x, float &s) {
+__device__ __forceinline__ double col_u_bis_vs(Col col, int n, float x, float &s) {
   const float4 r0 = col[0];
   if (x < r0.y) {
     s = fdiv(r0.x, r0.y);
@@ -138,7 +138,7 @@ __device__ __forceinline__ double col_u_bis_vs(const float4 *col, int n, float x
 }
 
 // EGA corner: eps(u(e_prev) + u_seg) with d/d e_prev and d/d u_seg.
-__device__ __forceinline__ void ega_corner(const float4 *col, int n, int mono, double ep, double useg,
+__device__ __forceinline__ void ega_corner(Col col, int n, int mono, double ep, double useg,
                                            int &g, double &e, double &dep, double &du) {
   float4 r, r2;
   int i;
@@ -155,7 +155,7 @@ __device__ __forceinline__ void ega_corner(const float4 *col, int n, int mono, d
 }
 
 // CGA corner: eps(U) and d/dU.
-__device__ __forceinline__ void cga_corner(const float4 *col, int n, int mono, double cu, int &g,
+__device__ __forceinline__ void cga_corner(Col col, int n, int mono, double cu, int &g,
                                            double &e, double &du) {
   float4 r;
   g = mono ? col_walk<0>(col, n, cu, g, r) : col_bisect<0>(col, n, cu, r);
@@ -217,12 +217,11 @@ __device__ __forceinline__ LkPart lookup_partials(const TabView &T, int tix, int
   const double cw[4] = {q0 * (1 - w0), q0 * w0, q1 * (1 - w1), q1 * w1};  // value
   const double tw[4] = {-q0 * s0, q0 * s0, -q1 * s1, q1 * s1};            // d/dT
   const double pw[4] = {-(1 - w0) * dwp, -w0 * dwp, (1 - w1) * dwp, w1 * dwp};  // d/dp
-  const float4 *base0 = T.rec + (c0 * T.TT + j0) * T.TU;
-  const float4 *base1 = T.rec + ((c0 + 1) * T.TT + j1) * T.TU;
+  const size_t col0 = c0 * T.TT + j0, col1 = (c0 + 1) * T.TT + j1;
   double en = 0;
 #pragma unroll
   for (int c = 0; c < 4; c++) {
-    const float4 *col = (c < 2 ? base0 : base1) + (c & 1) * T.TU;
+    const Col col = T.col((c < 2 ? col0 : col1) + (c & 1));
     double e, de, du;
     if (CGA) {
       cga_corner(col, nc[c], mono, x, gi[c], e, du);
@@ -289,13 +288,12 @@ __device__ __forceinline__ LkPart lookup_partials_f32(const TabView &T, int tix,
   const float cw[4] = {q0 * (1.f - w0), q0 * w0, q1 * (1.f - w1), q1 * w1};
   const float tw[4] = {-q0 * dt0, q0 * dt0, -q1 * dt1, q1 * dt1};
   const float pw[4] = {-(1.f - w0) * dwp, -w0 * dwp, (1.f - w1) * dwp, w1 * dwp};
-  const float4 *base0 = T.rec + (c0 * T.TT + j0) * T.TU;
-  const float4 *base1 = T.rec + ((c0 + 1) * T.TT + j1) * T.TU;
+  const size_t col0 = c0 * T.TT + j0, col1 = (c0 + 1) * T.TT + j1;
   float ec[4];
   float dep = 0.f, du = 0.f, dt = 0.f, dp = 0.f;
 #pragma unroll
   for (int c = 0; c < 4; c++) {
-    const float4 *col = (c < 2 ? base0 : base1) + (c & 1) * T.TU;
+    const Col col = T.col((c < 2 ? col0 : col1) + (c & 1));
     const int n = nc[c];
     float e, de, su, se;
     if (CGA) {
@@ -312,7 +310,7 @@ __device__ __forceinline__ LkPart lookup_partials_f32(const TabView &T, int tix,
       e = col_eps_bis_vs(col, n, u + x, se);
       de = se * su;
     } else {
-      e = ega_corner_f32_d(col, n, ep, x, gi[c], de, se);
+      e = ega_step_slow<true>(col, n, ep, x, gi[c], de, se);
     }
     ec[c] = e;
     dep += cw[c] * de;

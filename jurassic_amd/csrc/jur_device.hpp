@@ -115,7 +115,7 @@ template <int C>
 __device__ __forceinline__ float hi_of(const float4 &r) { return C == 0 ? r.z : r.w; }
 
 template <int C>
-__device__ __forceinline__ int col_walk(const float4 *col, int n, double x, int g, float4 &r) {
+__device__ __forceinline__ int col_walk(Col col, int n, double x, int g, float4 &r) {
   g = g < 0 ? 0 : (g > n - 2 ? n - 2 : g);
   r = col[g];
   if (g > 0 && (double)lo_of<C>(r) > x) {
@@ -164,7 +164,7 @@ __device__ __forceinline__ int col_walk(const float4 *col, int n, double x, int 
 // col_walk with the record at the start index already in hand (rg = col[g],
 // g in [0, n-2]): the common case, x still inside that bracket, loads nothing.
 template <int C>
-__device__ __forceinline__ int col_walk_r(const float4 *col, int n, double x, int g, const float4 &rg,
+__device__ __forceinline__ int col_walk_r(Col col, int n, double x, int g, const float4 &rg,
                                           float4 &r) {
   const bool left = g > 0 && (double)lo_of<C>(rg) > x;
   const bool right = g < n - 2 && (double)hi_of<C>(rg) <= x;
@@ -203,7 +203,7 @@ __device__ __forceinline__ double eps_from_rec(const float4 &r, double x) {
 // col_walk for a float key (the FP32 path): same end condition, float
 // comparisons.
 template <int C>
-__device__ __forceinline__ int col_walk_f(const float4 *col, int n, float x, int g, float4 &r) {
+__device__ __forceinline__ int col_walk_f(Col col, int n, float x, int g, float4 &r) {
   g = g < 0 ? 0 : (g > n - 2 ? n - 2 : g);
   r = col[g];
   if (g > 0 && lo_of<C>(r) > x) {
@@ -289,7 +289,7 @@ __device__ __forceinline__ float tanh_pos_f(float x) {
 
 // The reference bisection itself (for columns that are not monotone).
 template <int C>
-__device__ __forceinline__ int col_bisect(const float4 *col, int n, double x, float4 &r) {
+__device__ __forceinline__ int col_bisect(Col col, int n, double x, float4 &r) {
   int ilo = 0, ihi = n - 1, i;
   while (ihi > ilo + 1) {
     i = (ihi + ilo) >> 1;
@@ -307,147 +307,62 @@ __device__ __forceinline__ float eps_from_rec_f(const float4 &r, double x) {
   return r.y + fdiv(r.w - r.y, r.z - r.x) * (float)(x - (double)r.x);
 }
 
-// col_walk_f with the record at the (clamped) start index already in hand.
-template <int C>
-__device__ __forceinline__ int col_walk_f_r(const float4 *col, int n, float x, int g, const float4 &rg,
-                                            float4 &r) {
-  const bool left = g > 0 && lo_of<C>(rg) > x;
-  const bool right = g < n - 2 && hi_of<C>(rg) <= x;
-  if (!left && !right) {
-    r = rg;
-    return g;
-  }
-  return col_walk_f<C>(col, n, x, g, r);
-}
-
 // One EGA growth step on one table column, FP32 path: from the path
 // emissivity ep, u_eq = u(ep) (intpol_tbl_u, src/jurassic.c:3933-3967), then
-// eps(u_eq + u_seg) (intpol_tbl_eps, :3895-3929), both evaluated relative to
-// the knot of the inverse lookup's bracket r.
+// eps(u_eq + u_seg) (intpol_tbl_eps, :3895-3929).
 //
-// ega_step_fast covers the common case without branches: ep inside the eps
-// bracket of the record at the previous index (no walk, not below the first
-// or above the last knot) and u_eq + u_seg still inside its u bracket.
-// Otherwise slow is set and ega_step_slow gives the result.
-__device__ __forceinline__ void ega_step_fast(const float4 &r, float ep, float us, bool gt0, bool ltn2,
-                                              float &ec, bool &slow) {
-  const float du = r.z - r.x, de = r.w - r.y;
-  const float off = (ep - r.y) * fdiv(du, de) + us;
-  const bool walk = (gt0 && r.y > ep) || (ltn2 && r.w <= ep);
-  const bool outside = ep < r.y || ep > r.w;
-  slow = walk || outside || !(off < du);
-  ec = r.y + off * fdiv(de, du);
+// Both interpolations run on the same piecewise-linear curve through the
+// knots, so inside one bracket the step is ep + u_seg s with the bracket's
+// slope s = deps/du, and a step that leaves the bracket at its upper knot
+// (u_1, e_1) continues from there with the next slope: the part of u_seg
+// beyond the knot is (ep + u_seg s_0 - e_1)/s_0, hence e_1 + that s_1.  No
+// column density is formed, so nothing cancels and nothing needs FP64.
+//
+// ega_step_fast has the three knots k[0..2] from the previous step's bracket
+// g on in hand (a = k[0], k[1]; b = k[2]; g = -1: the bracket between the
+// origin and the first knot).  It covers ep in the bracket g or g + 1, the
+// grown emissivity in the same or (from g) the next one.  ok is false for
+// everything else (longer walks, beyond the last knot: the end marks' eps of
+// -1 fails the comparisons; flat or vertical brackets: NaN does) and
+// ega_step_slow gives the result.  g returns the inverse bracket.  With D,
+// dep = d eps / d ep and deu = d eps / d u_seg of the brackets used.
+template <bool D>
+__device__ __forceinline__ void ega_step_fast(const float4 &a, const float2 &b, float ep, float us, int &g,
+                                              float &ec, float &dep, float &deu, bool &ok) {
+  const float s0 = fdiv(a.w - a.y, a.z - a.x);
+  const float s1 = fdiv(b.y - a.w, b.x - a.z);
+  const float ratio = fdiv(s1, s0);
+  const bool up = ep >= a.w;
+  const float s = up ? s1 : s0;
+  const float x = ep + us * s;
+  const bool in = x < (up ? b.y : a.w);
+  const float y = a.w + (x - a.w) * ratio;
+  ok = a.y <= ep && (in || (!up && y < b.y));
+  ec = in ? x : y;
+  if (D) {
+    dep = in ? 1.f : ratio;
+    deu = in ? s : s1;
+  }
+  if (up) g++;
 }
 
-// The fast step with the records at g and g + 1 in hand (r0 = col[g], r1 =
-// col[min(g + 1, n - 2)]): it also covers the inverse bracket moving up by one
-// knot and the grown column crossing into the next u bracket, which is what a
-// growing path emissivity does every few segments.  Results are those of
-// ega_step_slow for the same inputs (same brackets, same formulas); slow is
-// set for everything else (walks of more than one knot, the extrapolation
-// branches below the first and above the last knot).  g returns the inverse
-// lookup's bracket index.
-__device__ __forceinline__ void ega_step_fast2(const float4 &r0, const float4 &r1, int n, float ep, float us,
-                                               double useg, int &g, float &ec, bool &slow) {
-  const bool top = g >= n - 2;
-  // inverse bracket: stay at g, or move to g + 1
-  const bool stay = (g == 0 || r0.y <= ep) && (top || r0.w > ep);
-  const bool up = !top && r0.w <= ep && (g + 1 >= n - 2 || r1.w > ep);
-  const float4 rb = stay ? r0 : r1;
-  const int b = stay ? g : g + 1;
-  bool ok = (stay || up) && !(ep < rb.y) && !(ep > rb.w);
-  const float du = rb.z - rb.x, de = rb.w - rb.y;
-  const float off = (ep - rb.y) * fdiv(du, de) + us;
-  const float e_in = rb.y + off * fdiv(de, du);
-  // forward bracket when off leaves the inverse bracket: the record after b
-  // (only r1 is in hand, so only from b == g), or b itself where rounding of
-  // du left arg below its upper knot
-  const double arg = (double)rb.x + (double)off;
-  const bool cross = !(off < du);
-  const bool b_top = b >= n - 2;
-  const bool inb = b_top ? !(arg > (double)rb.z) : !((double)rb.z <= arg);
-  const bool nxt = stay && !top && (double)r0.z <= arg && (g + 1 >= n - 2 ? !(arg > (double)r1.z) : (double)r1.z > arg);
-  const float4 rf = inb ? rb : r1;
-  const float e_x = rf.y + fdiv(rf.w - rf.y, rf.z - rf.x) * (float)(arg - (double)rf.x);
-  ok = ok && (!cross || inb || nxt);
-  ec = cross ? e_x : e_in;
-  // above the last knot (paths that have grown past a column's last
-  // emissivity, e.g. a limb path climbing into thin layers)
-  const bool above = (stay || up) && b_top && ep > rb.w;
-  if (above) ec = 1.f - (1.f - ep) * __expf(fdiv(__logf(1.f - rb.w), rb.z) * us);
-  ok = ok || above;
-  slow = !ok;
-  g = ok ? b : g;
+// Above the last knot (a = the bracket that ends at it, b = an end mark;
+// paths that have grown past a column's last emissivity, e.g. a limb path
+// climbing into thin layers): eps(u) = 1 - exp(c u), c = log(1 - eps_last) /
+// u_last, so eps(u_eq + u_seg) = 1 - (1 - ep) exp(c u_seg).
+__device__ __forceinline__ bool ega_above(const float4 &a, const float2 &b, float ep) {
+  return b.y < 0.f && a.w >= 0.f && ep > a.w;
 }
-
-// ega_step_fast2 with the partials of the step: dep = d eps / d ep and
-// deu = d eps / d u_seg, the slopes of the brackets used (as the FP32
-// lookup evaluates them: reciprocal-multiply float slopes).
-__device__ __forceinline__ void ega_step_fast2_d(const float4 &r0, const float4 &r1, int n, float ep, float us,
-                                                 int &g, float &ec, float &dep, float &deu, bool &slow) {
-  const bool top = g >= n - 2;
-  const bool stay = (g == 0 || r0.y <= ep) && (top || r0.w > ep);
-  const bool up = !top && r0.w <= ep && (g + 1 >= n - 2 || r1.w > ep);
-  const float4 rb = stay ? r0 : r1;
-  const int b = stay ? g : g + 1;
-  bool ok = (stay || up) && !(ep < rb.y) && !(ep > rb.w);
-  const float du = rb.z - rb.x, de = rb.w - rb.y;
-  const float su = fdiv(du, de);
-  const float off = (ep - rb.y) * su + us;
-  const float se_in = fdiv(de, du);
-  const float e_in = rb.y + off * se_in;
-  const double arg = (double)rb.x + (double)off;
-  const bool cross = !(off < du);
-  const bool b_top = b >= n - 2;
-  const bool inb = b_top ? !(arg > (double)rb.z) : !((double)rb.z <= arg);
-  const bool nxt = stay && !top && (double)r0.z <= arg && (g + 1 >= n - 2 ? !(arg > (double)r1.z) : (double)r1.z > arg);
-  const float4 rf = inb ? rb : r1;
-  const float sf = fdiv(rf.w - rf.y, rf.z - rf.x);
-  const float e_x = rf.y + sf * (float)(arg - (double)rf.x);
-  ok = ok && (!cross || inb || nxt);
-  ec = cross ? e_x : e_in;
-  deu = cross ? sf : se_in;
-  dep = deu * su;
-  const bool above = (stay || up) && b_top && ep > rb.w;
-  if (above) {
-    const float a = fdiv(__logf(1.f - rb.w), rb.z);
-    const float ex = __expf(a * us);
-    ec = 1.f - (1.f - ep) * ex;
-    deu = ex > 0.f ? -a * (1.f - ep) * ex : 0.f;
+template <bool D>
+__device__ __forceinline__ float ega_step_above(float u_last, float e_last, float ep, float us, float &dep,
+                                                float &deu) {
+  const float c = fdiv(__logf(1.f - e_last), u_last);
+  const float ex = __expf(c * us);
+  if (D) {
+    deu = ex > 0.f ? -c * (1.f - ep) * ex : 0.f;
     dep = ex;
   }
-  ok = ok || above;
-  slow = !ok;
-  g = ok ? b : g;
-}
-
-// The general step, starting the inverse search at g (record rg = col[g] in
-// hand); g returns the inverse lookup's bracket index.
-__device__ __forceinline__ float ega_step_slow(const float4 *col, int n, float ep, double useg, int &g,
-                                               const float4 &rg) {
-  float4 r;
-  const int i = col_walk_f_r<1>(col, n, ep, g, rg, r);
-  g = i;
-  if (ep < r.y) {
-    // below the first knot: u_eq = ep u_0 / eps_0 (small), absolute
-    const double arg = (double)(fdiv(r.x, r.y) * ep) + useg;
-    float4 r2;
-    col_walk_r<0>(col, n, arg, i, r, r2);
-    return eps_from_rec_f(r2, arg);
-  }
-  if (ep > r.w) {
-    // above the last knot: eps(u) = 1 - exp(a u), a = log(1 - eps_last) /
-    // u_last, so eps(u_eq + u_seg) = 1 - (1 - ep) exp(a u_seg)
-    const float a = fdiv(__logf(1.f - r.w), r.z);
-    return 1.f - (1.f - ep) * __expf(a * (float)useg);
-  }
-  const float du = r.z - r.x, de = r.w - r.y;
-  const float off = (ep - r.y) * fdiv(du, de) + (float)useg;
-  if (off < du) return r.y + off * fdiv(de, du);
-  const double arg = (double)r.x + (double)off;
-  float4 r2;
-  col_walk_r<0>(col, n, arg, i, r, r2);
-  return eps_from_rec_f(r2, arg);
+  return 1.f - (1.f - ep) * ex;
 }
 
 // FP32 path: eps_from_rec_f with its slope.
@@ -466,49 +381,41 @@ __device__ __forceinline__ float eps_rec_f_vs(const float4 &r, double x, float &
   return r.y + s * (float)(x - (double)r.x);
 }
 
-// General FP32 EGA step on one monotone column (ega_step_slow) with its
-// partials de = d eps / d ep and se = d eps / d u_seg; the inverse search
-// starts at g and g returns its bracket.
-__device__ __forceinline__ float ega_corner_f32_d(const float4 *col, int n, float ep, double x, int &g,
-                                                  float &de, float &se) {
-  float4 r;
+// The general step on one monotone column of n knots; the inverse search
+// starts at g and g returns its bracket (-1 below the first knot).
+template <bool D>
+__device__ __forceinline__ float ega_step_slow(Col col, int n, float ep, double useg, int &g, float &dep,
+                                               float &deu) {
+  float4 r, r2;
   const int i = col_walk_f<1>(col, n, ep, g, r);
-  g = i;
-  float e, su;
-  if (ep < r.y) {
-    su = fdiv(r.x, r.y);
-    const double arg = (double)(su * ep) + x;
-    float4 r2;
-    col_walk_r<0>(col, n, arg, i, r, r2);
-    e = eps_rec_f_vs(r2, arg, se);
-    de = se * su;
-  } else if (ep > r.w) {
-    // e = 1 - (1 - ep) exp(a u_seg), as ega_step_slow evaluates it
-    const float a = fdiv(__logf(1.f - r.w), r.z);
-    const float ex = __expf(a * (float)x);
-    e = 1.f - (1.f - ep) * ex;
-    se = ex > 0.f ? -a * (1.f - ep) * ex : 0.f;
-    de = ex;
-  } else {
-    const float dur = r.z - r.x, der = r.w - r.y;
-    su = fdiv(dur, der);
-    const float off = (ep - r.y) * su + (float)x;
-    if (off < dur) {
-      se = fdiv(der, dur);
-      e = r.y + off * se;
-    } else {
-      const double arg = (double)r.x + (double)off;
-      float4 r2;
-      col_walk_r<0>(col, n, arg, i, r, r2);
-      e = eps_rec_f_vs(r2, arg, se);
+  g = ep < r.y ? -1 : i;
+  if (ep > r.w) return ega_step_above<D>(r.z, r.w, ep, (float)useg, dep, deu);
+  // the bracket of ep: through the origin below the first knot
+  const float x0 = ep < r.y ? 0.f : r.x, y0 = ep < r.y ? 0.f : r.y;
+  const float dx = (ep < r.y ? r.x : r.z) - x0, dy = (ep < r.y ? r.y : r.w) - y0;
+  const float su = fdiv(dx, dy);
+  const float off = (ep - y0) * su + (float)useg;
+  if (off < dx) {
+    const float se = fdiv(dy, dx);
+    if (D) {
+      dep = 1.f;
+      deu = se;
     }
-    de = se * su;
+    return ep + (float)useg * se;
+  }
+  const double arg = (double)x0 + (double)off;
+  float se;
+  col_walk_r<0>(col, n, arg, i, r, r2);
+  const float e = eps_rec_f_vs(r2, arg, se);
+  if (D) {
+    deu = se;
+    dep = se * su;
   }
   return e;
 }
 
 // Reference-order lookups for columns that are not monotone (bisection).
-__device__ __forceinline__ float col_eps_bis(const float4 *col, int n, double x) {
+__device__ __forceinline__ float col_eps_bis(Col col, int n, double x) {
   const float4 r0 = col[0];
   if (x < (double)r0.x) return fdiv(r0.y, r0.x) * (float)x;
   const float4 rl = col[n - 1];
@@ -518,7 +425,7 @@ __device__ __forceinline__ float col_eps_bis(const float4 *col, int n, double x)
   return r.y + fdiv(r.w - r.y, r.z - r.x) * (float)(x - (double)r.x);
 }
 
-__device__ __forceinline__ double col_u_bis(const float4 *col, int n, float x) {
+__device__ __forceinline__ double col_u_bis(Col col, int n, float x) {
   const float4 r0 = col[0];
   if (x < r0.y) return (double)(fdiv(r0.x, r0.y) * x);
   const float4 rl = col[n - 1];
@@ -534,7 +441,7 @@ __device__ __forceinline__ double col_u_bis(const float4 *col, int n, float x) {
 // knot can only leave the walk at record 0, which holds (u_0, eps_0), and x
 // above the last knot only at record n-2, which holds (u_{n-1}, eps_{n-1}).
 // Branch conditions and arithmetic are those of the reference.
-__device__ __forceinline__ double col_eps(const float4 *col, int n, double x, int mono, int &g) {
+__device__ __forceinline__ double col_eps(Col col, int n, double x, int mono, int &g) {
   JUR_FP_EXACT
   float4 r;
   if (mono) {
@@ -558,7 +465,7 @@ __device__ __forceinline__ double col_eps(const float4 *col, int n, double x, in
 }
 
 // intpol_tbl_u on one column (src/jurassic.c:3933-3967), same scheme.
-__device__ __forceinline__ double col_u(const float4 *col, int n, double x, int mono, int &g) {
+__device__ __forceinline__ double col_u(Col col, int n, double x, int mono, int &g) {
   JUR_FP_EXACT
   float4 r;
   if (mono) {
@@ -615,6 +522,62 @@ __device__ __forceinline__ Cell locate_cell(const TabView &T, int tix, int npt, 
     c.tb1 = tg1[c.it1 + 1];
   }
   return c;
+}
+
+// One EGA growth step on one table column, FP64 path: eps(u(x) + u_seg) with
+// the reference's operations (u_from_rec and eps_from_rec; below the first
+// knot their LIN through the origin is the bracket of the column's origin).
+//
+// ega_step64 has the four knots from the previous step's bracket g on in hand
+// (k01, k23; g = -1: the bracket between the origin and the first knot).  It
+// covers x in the bracket g or g + 1 and the grown column in the same or the
+// next one; ok is false for everything else (longer walks, beyond the last
+// knot, whose end marks fail the comparisons) and ega_slow64 gives the
+// result.  g returns the inverse bracket.
+__device__ __forceinline__ double ega_step64(const float4 &k01, const float4 &k23, double x, double useg, int &g,
+                                             bool &ok) {
+  JUR_FP_EXACT
+  const bool up = x >= (double)k01.w;
+  const float u0 = up ? k01.z : k01.x, e0 = up ? k01.w : k01.y;
+  const float u1 = up ? k23.x : k01.z, e1 = up ? k23.y : k01.w;
+  const float u2 = up ? k23.z : k23.x, e2 = up ? k23.w : k23.y;
+  const double arg = lin_f(e0, u0, e1, u1, x) + useg;
+  const bool inb = arg < (double)u1;
+  ok = (double)e0 <= x && x < (double)e1 && (double)u0 <= arg && (inb || arg < (double)u2);
+  if (up) g++;
+  const float ua = inb ? u0 : u1, ea = inb ? e0 : e1, ub = inb ? u1 : u2, eb = inb ? e1 : e2;
+  return lin_f(ua, ea, ub, eb, arg);
+}
+
+__device__ __forceinline__ double ega_slow64(Col col, int n, double x, double useg, int &g) {
+  JUR_FP_EXACT
+  float4 r, r2;
+  const int i = col_walk<1>(col, n, x, g, r);
+  g = x < (double)r.y ? -1 : i;
+  const double arg = u_from_rec(r, x) + useg;
+  col_walk_r<0>(col, n, arg, i, r, r2);
+  return eps_from_rec(r2, arg);
+}
+
+// Values of the lanes of a quad (lanes 4k..4k+3) by DPP: of lane K, and of
+// the lane that differs in the bits X of its number.
+template <int CTRL>
+__device__ __forceinline__ int quad_dpp(int v) {
+  return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xf, 0xf, true);
+}
+template <int CTRL>
+__device__ __forceinline__ float quad_dpp(float v) {
+  return __int_as_float(quad_dpp<CTRL>(__float_as_int(v)));
+}
+template <int CTRL>
+__device__ __forceinline__ double quad_dpp(double v) {
+  return __hiloint2double(quad_dpp<CTRL>(__double2hiint(v)), quad_dpp<CTRL>(__double2loint(v)));
+}
+template <int K, typename V>
+__device__ __forceinline__ V quad_lane(V v) { return quad_dpp<K * 0x55>(v); }
+template <int X, typename V>
+__device__ __forceinline__ V quad_xor(V v) {
+  return quad_dpp<(0 ^ X) | (1 ^ X) << 2 | (2 ^ X) << 4 | (3 ^ X) << 6>(v);
 }
 
 // Per-(channel, emitter) table constants, loaded once per wavefront.

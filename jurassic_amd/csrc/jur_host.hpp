@@ -252,8 +252,8 @@ struct jur_ctx {
   // tables
   jur::DevBuf<int> d_np, d_nt, d_nu, d_mono, d_pdir;
   jur::DevBuf<double> d_p, d_t;
-  jur::DevBuf<float4> d_rec;
-  int TP = 2, TT = 2, TU = 2;
+  jur::DevBuf<float2> d_kn;
+  int TP = 2, TT = 2, TU = 2, TS = 4;
   int shared = 0, ref_tix = 0, all_mono = 1;
   size_t table_bytes = 0;
   // model constants

@@ -2,6 +2,7 @@
 // libjurassic_gpu.so.  Plain structs only; device pointers are raw.
 #pragma once
 
+#include <hip/hip_runtime.h>
 #include <stdint.h>
 
 #include "../../include/jurassic_gpu.h"
@@ -25,19 +26,39 @@ constexpr int WAVE = 64;
 
 // ------------------------------------------------------------------
 // Emissivity tables in HBM, laid out [gas][channel][p][T][u].
-// Each (p, T) column of nu knots is stored as nu records
-//   rec[i] = (u_i, eps_i, u_{i+1}, eps_{i+1})   (last: (u_n-1, e_n-1, same))
-// so that one aligned 16-byte load holds a whole interpolation bracket.
+// Each (p, T) column of nu knots (u_i, eps_i) is stored in TS = TU + 2 slots:
+//   (0, 0), knot 0, ..., knot nu-1, end marks (0, -1) up to the next column
+// The origin before knot 0 makes the interpolation below the first knot
+// (intpol_tbl_eps and intpol_tbl_u: through the origin) a bracket like any
+// other, and an end mark, below every emissivity, fails every comparison of
+// the FP32 step beyond the last knot.  A 16-byte load at knot i (8-byte
+// aligned) holds the bracket (u_i, eps_i, u_{i+1}, eps_{i+1}).
 // ------------------------------------------------------------------
+// A 16-byte load at 8-byte alignment.
+struct alignas(8) Knots2 {
+  float x, y, z, w;
+};
+
+// One (p, T) column: col[i] = (u_i, eps_i, u_{i+1}, eps_{i+1}), i >= -1; of
+// col[nu-1] only the first two are a knot.
+struct Col {
+  const float2 *k;
+  __host__ __device__ __forceinline__ float4 operator[](int i) const {
+    const Knots2 v = *(const Knots2 *)(k + i);
+    return make_float4(v.x, v.y, v.z, v.w);
+  }
+};
+
 struct TabView {
   int nd, ng;
   int TP, TT, TU;          // padded capacities of p, T, u
+  int TS;                  // slots of a column (TU + 2)
   const int *np;           // [ng][nd]           (-1: missing table)
   const int *nt;           // [ng][nd][TP]
   const int *nu;           // [ng][nd][TP][TT]
   const double *p;         // [ng][nd][TP]
   const double *t;         // [ng][nd][TP][TT]
-  const float4 *rec;       // [ng][nd][TP][TT][TU]
+  const float2 *kn;        // [ng][nd][TP][TT][TS]
   const int *mono;         // [ng][nd]: 1 if every column is non-decreasing
                            // in u and eps (search by local walk), 0 otherwise
                            // (search by the reference bisection)
@@ -48,6 +69,8 @@ struct TabView {
                            // T-grid sizes and T grids (one cell search per
                            // segment serves all of them)
   int ref_tix;             // a table holding the shared grids
+  // column c = (table * TP + p) * TT + T
+  __device__ __forceinline__ Col col(size_t c) const { return Col{kn + c * TS + 1}; }
 };
 
 // ------------------------------------------------------------------

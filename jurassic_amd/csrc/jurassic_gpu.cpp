@@ -57,8 +57,8 @@ void launch_finalize(double *, int, int, const ChanInfo *, int, const unsigned c
                      hipStream_t);
 void launch_block_np(const RayInfo *, int, int, int, int *, hipStream_t);
 void launch_zero(void *, size_t, hipStream_t);
-void launch_pack_tables(int, int, int, int, int, const int *, const int *, const int *, int, int, int,
-                        const float *, const float *, float4 *, int *, hipStream_t);
+void launch_pack_tables(int, int, int, int, int, size_t, const int *, const int *, const int *, int, int, int,
+                        const float *, const float *, float2 *, int *, hipStream_t);
 
 // ------------------------------------------------------------------
 // Errors.
@@ -305,6 +305,10 @@ static int p_direction(const double *p, int np) {
   return (np >= 2 && asc) ? 1 : ((np >= 2 && desc) ? -1 : 0);
 }
 
+// Knot slots of ntab tables, with the spare ones that a 24-byte load at the
+// last column's last slot reaches into.
+static size_t table_slots(size_t ntab, int TP, int TT, int TS) { return ntab * TP * TT * TS + 4; }
+
 static int build_tables(jur_ctx *c) {
   const Setup &s = c->s;
   const int nd = s.nd, ng = s.ng;
@@ -324,11 +328,14 @@ static int build_tables(jur_ctx *c) {
   c->TP = TP;
   c->TT = TT;
   c->TU = TU;
+  c->TS = TU + 2;
   const size_t ntab = (size_t)nd * ng;
   std::vector<int> h_np(ntab + 1, -1), h_nt(ntab * TP + 1, 0), h_nu(ntab * TP * TT + 1, 0),
       h_mono(ntab + 1, 1), h_pdir(ntab + 1, 0);
   std::vector<double> h_p(ntab * TP + 1, 0.0), h_t(ntab * TP * TT + 1, 0.0);
-  std::vector<float4> h_rec(ntab * TP * TT * TU + 1, make_float4(0, 0, 0, 0));
+  const int TS = c->TS;
+  std::vector<float2> h_kn(table_slots(ntab, TP, TT, TS), make_float2(0, -1));
+  for (size_t q = 0; q < ntab * TP * TT; q++) h_kn[q * TS] = make_float2(0, 0);
   c->all_mono = 1;
   for (size_t k = 0; k < ntab; k++) {
     const HostTable &tb = tabs[k];
@@ -341,10 +348,10 @@ static int build_tables(jur_ctx *c) {
         h_t[(k * TP + ip) * TT + it] = tb.t[ip][it];
         const int n = tb.nu[ip][it];
         h_nu[(k * TP + ip) * TT + it] = n;
-        float4 *col = &h_rec[((k * TP + ip) * TT + it) * TU];
+        float2 *col = &h_kn[((k * TP + ip) * TT + it) * TS + 1];
         for (int i = 0; i < n; i++) {
           const int j = (i + 1 < n) ? i + 1 : i;
-          col[i] = make_float4(tb.u[ip][it][i], tb.eps[ip][it][i], tb.u[ip][it][j], tb.eps[ip][it][j]);
+          col[i] = make_float2(tb.u[ip][it][i], tb.eps[ip][it][i]);
           if (i + 1 < n && (!(tb.u[ip][it][j] >= tb.u[ip][it][i]) ||
                             !(tb.eps[ip][it][j] >= tb.eps[ip][it][i])))
             mono = 0;
@@ -363,8 +370,8 @@ static int build_tables(jur_ctx *c) {
   if ((rc = c->d_pdir.upload(h_pdir.data(), h_pdir.size()))) return rc;
   if ((rc = c->d_p.upload(h_p.data(), h_p.size()))) return rc;
   if ((rc = c->d_t.upload(h_t.data(), h_t.size()))) return rc;
-  if ((rc = c->d_rec.upload(h_rec.data(), h_rec.size()))) return rc;
-  c->table_bytes = h_rec.size() * sizeof(float4);
+  if ((rc = c->d_kn.upload(h_kn.data(), h_kn.size()))) return rc;
+  c->table_bytes = h_kn.size() * sizeof(float2);
   detect_shared(c, h_np, h_nt, h_p, h_t);
   return JUR_OK;
 }
@@ -409,6 +416,7 @@ static int build_tables_device(jur_ctx *c, const jur_dtables_t *d) {
   c->TP = TP;
   c->TT = TT;
   c->TU = TU;
+  c->TS = TU + 2;
   // the library's order: table k = ig * nd + id
   std::vector<int> h_np(ntab + 1, -1), h_nt(ntab * TP + 1, 0), h_nu(ntab * TP * TT + 1, 0),
       h_mono(ntab + 1, 1), h_pdir(ntab + 1, 0);
@@ -437,11 +445,11 @@ static int build_tables_device(jur_ctx *c, const jur_dtables_t *d) {
   if ((rc = c->d_pdir.upload(h_pdir.data(), h_pdir.size()))) return rc;
   if ((rc = c->d_p.upload(h_p.data(), h_p.size()))) return rc;
   if ((rc = c->d_t.upload(h_t.data(), h_t.size()))) return rc;
-  const size_t nrec = ntab * TP * TT * TU + 1;
-  if ((rc = c->d_rec.reserve(nrec))) return rc;
-  c->table_bytes = nrec * sizeof(float4);
-  launch_pack_tables(nd, ng, TP, TT, TU, c->d_np.p, c->d_nt.p, c->d_nu.p, tp, tt, tu, d->u, d->eps,
-                     c->d_rec.p, c->d_mono.p, 0);
+  const size_t nkn = table_slots(ntab, TP, TT, c->TS);
+  if ((rc = c->d_kn.reserve(nkn))) return rc;
+  c->table_bytes = nkn * sizeof(float2);
+  launch_pack_tables(nd, ng, TP, TT, c->TS, nkn, c->d_np.p, c->d_nt.p, c->d_nu.p, tp, tt, tu, d->u, d->eps,
+                     c->d_kn.p, c->d_mono.p, 0);
   HIPCHK(hipGetLastError());
   HIPCHK(hipDeviceSynchronize());
   HIPCHK(hipMemcpy(h_mono.data(), c->d_mono.p, ntab * sizeof(int), hipMemcpyDeviceToHost));
@@ -584,12 +592,13 @@ static ModelView model_view(const jur_ctx *c) {
   T.TP = c->TP;
   T.TT = c->TT;
   T.TU = c->TU;
+  T.TS = c->TS;
   T.np = c->d_np.p;
   T.nt = c->d_nt.p;
   T.nu = c->d_nu.p;
   T.p = c->d_p.p;
   T.t = c->d_t.p;
-  T.rec = c->d_rec.p;
+  T.kn = c->d_kn.p;
   T.mono = c->d_mono.p;
   T.pdir = c->d_pdir.p;
   T.shared = c->shared;

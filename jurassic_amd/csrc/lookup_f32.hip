@@ -8,11 +8,13 @@
 //    no accumulated rounding, and small emissivities keep full relative
 //    precision in float where 1 - tau_path would not.
 //  * The emissivity-growth step u_eq = u(eps_path), eps00 = eps(u_eq + u_seg)
-//    is evaluated relative to the knot u_i of the inverse lookup's bracket:
-//    off = (eps_path - eps_i) du/deps + u_seg is a small float with no
-//    cancellation against u_i, and eps00 = eps_i + off deps/du while off stays
-//    inside the bracket (the common case; otherwise the forward bracket is
-//    searched on the absolute column density in FP64).
+//    runs along the column's piecewise-linear curve (ega_step_fast): inside a
+//    bracket eps00 = eps_path + u_seg deps/du, and across its upper knot it
+//    continues with the next slope, so no column density is formed.  (Before,
+//    both lookups were evaluated one after the other, relative to the
+//    bracket's knot: 62.7 ms per 4096 x 32 x 12 limb batch of three emitters
+//    against 51 ms, 27.2 against 19.4 ms for 1000 nadir paths of 256 channels
+//    and eight emitters.)
 //  * Output is the path emissivity eps_path after each segment (the radiance
 //    kernel forms the segment emissivity (eps_i - eps_{i-1}) / (1 - eps_{i-1});
 //    the adjoint restarts any segment from eps_{i-1}); 1 marks an opaque
@@ -74,13 +76,24 @@ __global__ __launch_bounds__(WAVE) void k_lookup_f32(ModelView M, BatchView B, L
   const size_t tcols = (size_t)T.TP * T.TT;  // (p, T) columns per table
   const double *tgb = T.t + (size_t)tix * tcols;
   const int *nub = T.nu + (size_t)tix * tcols;
-  const float4 *recb = T.rec + (size_t)tix * tcols * T.TU;
+  const float2 *knb = T.kn + (size_t)tix * tcols * T.TS;
 
   float ep = 0.f;
   double cu = 0, cp = 0, ct = 0;
   int gi[4];
 #pragma unroll
-  for (int c = 0; c < 4; c++) gi[c] = T.TU / 2;
+  for (int c = 0; c < 4; c++) gi[c] = CGA || !mono ? T.TU / 2 : -1;
+  // the three knots from bracket g of the column with knot 0 at ko on: one
+  // 24-byte stretch; g is brought into the column's slots
+  const int gtop = T.TU - 2;
+  auto load_knots = [&](unsigned ko, int &g, float4 &a, float2 &b) {
+    g = g < -1 ? -1 : (g > gtop ? gtop : g);
+    const unsigned k = ko + g;
+    const char *at = (const char *)knb + (size_t)(k * (unsigned)sizeof(float2));
+    const Knots2 v = *(const Knots2 *)at;
+    a = make_float4(v.x, v.y, v.z, v.w);
+    b = *(const float2 *)(at + 16);
+  };
 
   // cached cell
   int ipr = -1, it0 = -1, it1 = -1;
@@ -191,34 +204,35 @@ __global__ __launch_bounds__(WAVE) void k_lookup_f32(ModelView M, BatchView B, L
         n11 = ld32(nub, tq0 + T.TT + it1 + 1);
       }
       if (n00 >= 2 && n01 >= 2 && n10 >= 2 && n11 >= 2) {
-        // first record of each corner column in the table
+        // knot 0 of each corner column in the table
         unsigned ko[4];
-        ko[0] = (tq0 + it0) * T.TU;
-        ko[1] = ko[0] + T.TU;
-        ko[2] = (tq0 + T.TT + it1) * T.TU;
-        ko[3] = ko[2] + T.TU;
-        const float4 *kc[4] = {recb + ko[0], recb + ko[1], recb + ko[2], recb + ko[3]};
+        ko[0] = (tq0 + it0) * T.TS + 1;
+        ko[1] = ko[0] + T.TS;
+        ko[2] = (tq0 + T.TT + it1) * T.TS + 1;
+        ko[3] = ko[2] + T.TS;
         const int nc[4] = {n00, n01, n10, n11};
         const float us = (float)useg;
         float ec[4], dep[4] = {0.f, 0.f, 0.f, 0.f}, deu[4] = {0.f, 0.f, 0.f, 0.f};
         if (CGA || !mono) {
           if (RL > 1 && !mono) {
             const int c = sub;
-            const float4 *kcc = c == 0 ? kc[0] : (c == 1 ? kc[1] : (c == 2 ? kc[2] : kc[3]));
+            const Col kcc{knb + (c == 0 ? ko[0] : (c == 1 ? ko[1] : (c == 2 ? ko[2] : ko[3])))};
             const int ncc = c == 0 ? nc[0] : (c == 1 ? nc[1] : (c == 2 ? nc[2] : nc[3]));
             const float e = col_eps_bis(kcc, ncc, col_u_bis(kcc, ncc, ep) + useg);
 #pragma unroll
             for (int k = 0; k < 4; k++) ec[k] = __shfl(e, k, RL);
           } else if (!mono) {
 #pragma unroll 1
-            for (int c = 0; c < 4; c++)
-              ec[c] = CGA ? col_eps_bis(kc[c], nc[c], cu)
-                          : col_eps_bis(kc[c], nc[c], col_u_bis(kc[c], nc[c], ep) + useg);
+            for (int c = 0; c < 4; c++) {
+              const Col kcc{knb + ko[c]};
+              ec[c] = CGA ? col_eps_bis(kcc, nc[c], cu)
+                          : col_eps_bis(kcc, nc[c], col_u_bis(kcc, nc[c], ep) + useg);
+            }
           } else {
 #pragma unroll
             for (int c = 0; c < 4; c++) {
               float4 r;
-              gi[c] = col_walk<0>(kc[c], nc[c], cu, gi[c], r);
+              gi[c] = col_walk<0>(Col{knb + ko[c]}, nc[c], cu, gi[c], r);
               ec[c] = eps_from_rec_f(r, cu);
             }
           }
@@ -226,29 +240,26 @@ __global__ __launch_bounds__(WAVE) void k_lookup_f32(ModelView M, BatchView B, L
           tn = LOSR(F_T, ipn);
           un = LOSR(L.f_u + ig, ipn);
         } else if constexpr (RL > 1) {
-          // the lane's corner: its bracket records, the step, and the
+          // the lane's corner: its bracket's knots, the step, and the
           // corners' results gathered from the quad
           const int c = sub;
-          const float4 *kcc = c == 0 ? kc[0] : (c == 1 ? kc[1] : (c == 2 ? kc[2] : kc[3]));
           const int ncc = c == 0 ? nc[0] : (c == 1 ? nc[1] : (c == 2 ? nc[2] : nc[3]));
           const unsigned koc = c == 0 ? ko[0] : (c == 1 ? ko[1] : (c == 2 ? ko[2] : ko[3]));
           int g = c == 0 ? gi[0] : (c == 1 ? gi[1] : (c == 2 ? gi[2] : gi[3]));
-          g = g < 0 ? 0 : (g > ncc - 2 ? ncc - 2 : g);
-          const float4 r = ld32(recb, koc + g);
-          const float4 rn = ld32(recb, koc + (g + 1 < ncc - 2 ? g + 1 : ncc - 2));
+          float4 ka;
+          float2 kb;
+          load_knots(koc, g, ka, kb);
           __builtin_amdgcn_sched_barrier(0);
           pn = LOSR(F_P, ipn);
           tn = LOSR(F_T, ipn);
           un = LOSR(L.f_u + ig, ipn);
           __builtin_amdgcn_sched_barrier(0);
           float e, de = 0.f, du = 0.f;
-          bool slow;
-          if constexpr (PART) {
-            ega_step_fast2_d(r, rn, ncc, ep, us, g, e, de, du, slow);
-            if (slow) e = ega_corner_f32_d(kcc, ncc, ep, useg, g, de, du);
-          } else {
-            ega_step_fast2(r, rn, ncc, ep, us, useg, g, e, slow);
-            if (slow) e = ega_step_slow(kcc, ncc, ep, useg, g, r);
+          bool ok;
+          ega_step_fast<PART>(ka, kb, ep, us, g, e, de, du, ok);
+          if (!ok) {
+            if (ega_above(ka, kb, ep)) e = ega_step_above<PART>(ka.z, ka.w, ep, us, de, du);
+            else e = ega_step_slow<PART>(Col{knb + koc}, ncc, ep, useg, g, de, du);
           }
 #pragma unroll
           for (int k = 0; k < 4; k++) {
@@ -260,42 +271,26 @@ __global__ __launch_bounds__(WAVE) void k_lookup_f32(ModelView M, BatchView B, L
             }
           }
         } else {
-          // the bracket records at the previous segment's index and the next
-          float4 r[4], rn[4];
+          // the knots from the previous segment's brackets on
+          float4 ka[4];
+          float2 kb[4];
 #pragma unroll
-          for (int c = 0; c < 4; c++) {
-            int g = gi[c];
-            g = g < 0 ? 0 : (g > nc[c] - 2 ? nc[c] - 2 : g);
-            gi[c] = g;
-            r[c] = ld32(recb, ko[c] + g);
-            rn[c] = ld32(recb, ko[c] + (g + 1 < nc[c] - 2 ? g + 1 : nc[c] - 2));
-          }
+          for (int c = 0; c < 4; c++) load_knots(ko[c], gi[c], ka[c], kb[c]);
           __builtin_amdgcn_sched_barrier(0);
           pn = LOSR(F_P, ipn);
           tn = LOSR(F_T, ipn);
           un = LOSR(L.f_u + ig, ipn);
           __builtin_amdgcn_sched_barrier(0);
-          // common case: the inverse and forward brackets are those records
-          bool slow[4];
-          if constexpr (PART) {
+          bool ok[4];
 #pragma unroll
-            for (int c = 0; c < 4; c++) {
-              int gg = gi[c];
-              ega_step_fast2_d(r[c], rn[c], nc[c], ep, us, gg, ec[c], dep[c], deu[c], slow[c]);
-              gi[c] = gg;
+          for (int c = 0; c < 4; c++)
+            ega_step_fast<PART>(ka[c], kb[c], ep, us, gi[c], ec[c], dep[c], deu[c], ok[c]);
+#pragma unroll
+          for (int c = 0; c < 4; c++)
+            if (!ok[c]) {
+              if (ega_above(ka[c], kb[c], ep)) ec[c] = ega_step_above<PART>(ka[c].z, ka[c].w, ep, us, dep[c], deu[c]);
+              else ec[c] = ega_step_slow<PART>(Col{knb + ko[c]}, nc[c], ep, useg, gi[c], dep[c], deu[c]);
             }
-#pragma unroll
-            for (int c = 0; c < 4; c++) {
-              if (slow[c]) ec[c] = ega_corner_f32_d(kc[c], nc[c], ep, useg, gi[c], dep[c], deu[c]);
-            }
-          } else {
-#pragma unroll
-            for (int c = 0; c < 4; c++) ega_step_fast2(r[c], rn[c], nc[c], ep, us, useg, gi[c], ec[c], slow[c]);
-#pragma unroll
-            for (int c = 0; c < 4; c++) {
-              if (slow[c]) ec[c] = ega_step_slow(kc[c], nc[c], ep, useg, gi[c], r[c]);
-            }
-          }
         }
         const float w0 = (tq - ta0) * dt0;
         const float w1 = (tq - ta1) * dt1;

@@ -12,14 +12,23 @@
 // A lane keeps tau_path, its table cell and, per corner, the bracket of the
 // inverse lookup u(1 - tau_path).  Along a ray consecutive segments mostly
 // stay in the same cell and bracket, so:
-//  * cell data (pressure bracket, temperature grids, column sizes) are
-//    reloaded only when the cell changes;
-//  * each inverse lookup starts from the previous segment's bracket;
-//  * the forward lookup eps(u + u_seg) starts from the inverse lookup's
-//    bracket record, already in registers (u lies in that bracket and
-//    u_seg >= 0).
+//  * cell data (pressure bracket, temperature grids and their reciprocal
+//    spacings, column sizes) are reloaded only when the cell changes, and a
+//    column that the cell keeps takes its bracket along;
+//  * a corner's four knots from the previous segment's bracket on are loaded
+//    first, and cover the inverse lookup moving up one knot and the grown
+//    column the next one (ega_step64); the next point's LOS values are loaded
+//    behind them, so that waiting for the knots does not wait for HBM.
 // Every search returns the reference bisection's index and the arithmetic is
-// the reference's (built with -ffp-contract=off).
+// the reference's (built with -ffp-contract=off), except that the cell's
+// weights multiply by reciprocals kept with the cell where LIN divides (an
+// ulp or so).
+// Large batches are bound by instruction issue (512 x 32 x 12 limb paths of
+// three emitters: 10.3 ms, 14.9 ms with one walk per lookup and LIN's
+// divisions), small ones by the latency of a point: its LOS load, its knots
+// and its eight float quotients in series took 4.25 us; with the loads ahead
+// and a quad's lanes sharing the quotients it is 0.84 us (10 nadir rays, 2
+// channels, 805 points: 3.43 -> 0.67 ms).
 #include "jur_device.hpp"
 
 namespace jur {
@@ -28,18 +37,27 @@ namespace jur {
 
 // PATH: store the path transmittance tau_path after each segment instead of
 // the segment emissivity (the Jacobian restarts any segment from it).
-template <bool CGA, bool PATH>
+// RL lanes per chain, as in the FP32 lookups: RL = 4 (small batches, where a
+// wavefront's chain is the kernel's duration; EGA): each lane of a quad takes
+// one corner of the cell, exchanged by DPP; the same operations on the same
+// values, so the same bits.  A wavefront then covers a quarter of a block.
+template <bool CGA, bool PATH, int RL = 1>
 __global__ __launch_bounds__(WAVE) void k_lookup_f64(ModelView M, BatchView B, LosView L,
                                                      EpsView E, const RayInfo *info, int blk0,
                                                      int nblk) {
   JUR_FP_EXACT
+  static_assert(RL == 1 || !CGA, "the four-lane chains are the EGA ones");
   const int nd = M.nd, ng = M.ng;
   int bl, rem;
-  if (!xcd_block_map(blockIdx.x, nd * ng, nblk, bl, rem)) return;
+  if (!xcd_block_map(blockIdx.x, nd * ng * RL, nblk, bl, rem)) return;
+  const int qtr = rem % RL;
+  rem /= RL;
   const int id = rem / ng;
   const int ig = rem - id * ng;
   const int lane = threadIdx.x;
-  const int ir = (blk0 + bl) * WAVE + lane;
+  const int sub = lane % RL;  // the lane's corner (RL = 4)
+  const int ln = RL == 1 ? lane : qtr * (WAVE / RL) + lane / RL;  // the ray's lane in its block
+  const int ir = (blk0 + bl) * WAVE + ln;
   if (ir >= B.nray) return;
   const TabView &T = M.tab;
   const int tix = ig * nd + id;
@@ -48,41 +66,51 @@ __global__ __launch_bounds__(WAVE) void k_lookup_f64(ModelView M, BatchView B, L
   const RayInfo R = info[ir];
   if (R.status != JUR_OK) return;
 
-  const double *los = L.los + (size_t)bl * L.cap * L.nfield * WAVE + lane;
+  const double *los = L.los + (size_t)bl * L.cap * L.nfield * WAVE + ln;
   const int npb = E.npb[bl];
-  double *out = (double *)E.eps + E.off[bl] + ((size_t)id * ng + ig) * npb * WAVE + lane;
+  double *out = (double *)E.eps + E.off[bl] + ((size_t)id * ng + ig) * npb * WAVE + ln;
   const int mono = T.mono[tix];
   const int pdir = T.pdir[tix];
   const double *pg = T.p + (size_t)tix * T.TP;
   const int *ntp = T.nt + (size_t)tix * T.TP;
+  const double *tgb = T.t + (size_t)tix * T.TP * T.TT;
+  const int *nub = T.nu + (size_t)tix * T.TP * T.TT;
+  const float2 *knb = T.kn + (size_t)tix * T.TP * T.TT * T.TS + 1;
+  const int gtop = T.TU - 2;
 
+  constexpr int NC = RL == 1 ? 4 : 1;  // the lane's corners
   double tp = 1, cu = 0, cp = 0, ct = 0;
-  int gi[4];
+  int gi[NC];
 #pragma unroll
-  for (int c = 0; c < 4; c++) gi[c] = T.TU / 2;
+  for (int c = 0; c < NC; c++) gi[c] = CGA || !mono ? T.TU / 2 : -1;
 
   // cached cell
   int ipr = -1, it0 = -1, it1 = -1;
-  double pa = 0, pb = 0, g00 = 0, g01 = 0, g10 = 0, g11 = 0;   // p[ipr..], T-grid starts
-  double ta0 = 0, tb0 = 0, ta1 = 0, tb1 = 0;
-  int nt0 = 0, nt1 = 0, n00 = 0, n01 = 0, n10 = 0, n11 = 0;
-  const double *tg0 = nullptr;
+  double pa = 0, pb = 0, rp = 0, g00 = 0, r0 = 0, g10 = 0, r1 = 0;  // p bracket, T-grid starts and 1/spacings
+  double ta0 = 0, rt0 = 0, ta1 = 0, rt1 = 0;
+  int nt0 = 0, nt1 = 0;
+  int tq0 = 0;          // first T-grid entry of p row ipr
+  bool full = false;    // every corner column has two knots
 
+  double p = 0, t = 0, useg = 0;
+  if (R.np > 0) {
+    p = LOSR(F_P, 0);
+    t = LOSR(F_T, 0);
+    useg = LOSR(L.f_u + ig, 0);
+  }
   for (int ip = 0; ip < R.np; ip++) {
-    const double p = LOSR(F_P, ip);
-    const double t = LOSR(F_T, ip);
-    const double useg = LOSR(L.f_u + ig, ip);
+    const int ipn = ip + 1 < R.np ? ip + 1 : ip;
     if (CGA) {
       cu = cu + useg;
       cp = cp + useg * p;
       ct = ct + useg * t;
     }
-    double eps;
-    if (tp < 1e-9) {
-      eps = 1;
-    } else {
-      const double pq = CGA ? cp / cu : p;
-      const double tq = CGA ? ct / cu : t;
+    const bool opaque = tp < 1e-9;
+    const double pq = CGA ? cp / cu : p;
+    const double tq = CGA ? ct / cu : t;
+    bool cell = false;
+    float4 ka[NC], kb[NC];
+    if (!opaque) {
       // pressure bracket (locate_irr): keep the cached one while it holds
       bool keep = false;
       if (ipr >= 0 && pdir != 0) {
@@ -92,96 +120,181 @@ __global__ __launch_bounds__(WAVE) void k_lookup_f64(ModelView M, BatchView B, L
           keep = (ipr == 0 || !(pa <= pq)) && (ipr == npt - 2 || pb <= pq);
       }
       if (!keep) {
+        const int iprev = ipr;
         ipr = (pdir != 0 && ipr >= 0) ? irr_walk(pg, npt, pq, ipr, pdir) : locate_irr(pg, npt, pq);
+        // a column that the cell keeps takes its bracket along, a new one
+        // extrapolates from the pair
+        const bool fwd = ipr == iprev + 1, bwd = ipr == iprev - 1;
+        if (fwd || bwd) {
+          if constexpr (RL == 1) {
+#pragma unroll
+            for (int c = 0; c < 2; c++) {
+              const int lo = gi[c], hi = gi[c + 2];
+              gi[c] = fwd ? hi : 2 * lo - hi;
+              gi[c + 2] = fwd ? 2 * hi - lo : lo;
+            }
+          } else {
+            const int o = quad_xor<2>(gi[0]);
+            gi[0] = (sub < 2) == fwd ? o : 2 * gi[0] - o;
+          }
+        }
         pa = pg[ipr];
         pb = pg[ipr + 1];
+        rp = 1 / (pb - pa);
         nt0 = ntp[ipr];
         nt1 = ntp[ipr + 1];
-        tg0 = T.t + ((size_t)tix * T.TP + ipr) * T.TT;
-        g00 = tg0[0];
-        g01 = tg0[1];
-        g10 = tg0[T.TT];
-        g11 = tg0[T.TT + 1];
-        it0 = it1 = -1;
+        tq0 = ipr * T.TT;
+        g00 = tgb[tq0];
+        r0 = 1 / (tgb[tq0 + 1] - g00);
+        g10 = tgb[tq0 + T.TT];
+        r1 = 1 / (tgb[tq0 + T.TT + 1] - g10);
+        it0 = it1 = -2;
       }
-      if (nt0 < 2 || nt1 < 2) {
-        eps = 0;
-      } else {
+      cell = nt0 >= 2 && nt1 >= 2;
+      if (cell) {
         // locate_reg on the two temperature rows
-        int j0 = (int)((tq - g00) / (g01 - g00));
+        int j0 = (int)((tq - g00) * r0);
         j0 = j0 < 0 ? 0 : (j0 > nt0 - 2 ? nt0 - 2 : j0);
-        int j1 = (int)((tq - g10) / (g11 - g10));
+        int j1 = (int)((tq - g10) * r1);
         j1 = j1 < 0 ? 0 : (j1 > nt1 - 2 ? nt1 - 2 : j1);
-        const size_t c0 = (size_t)tix * T.TP + ipr;
-        if (j0 != it0) {
+        if (j0 != it0 || j1 != it1) {
+          const int d0 = j0 - it0, d1 = j1 - it1;
+          if constexpr (RL == 1) {
+            const int lo0 = gi[0], hi0 = gi[1], lo1 = gi[2], hi1 = gi[3];
+            if (d0 == 1) { gi[0] = hi0; gi[1] = 2 * hi0 - lo0; }
+            if (d0 == -1) { gi[1] = lo0; gi[0] = 2 * lo0 - hi0; }
+            if (d1 == 1) { gi[2] = hi1; gi[3] = 2 * hi1 - lo1; }
+            if (d1 == -1) { gi[3] = lo1; gi[2] = 2 * lo1 - hi1; }
+          } else {
+            const int o = quad_xor<1>(gi[0]);
+            const int d = sub < 2 ? d0 : d1;
+            if (d == 1) gi[0] = (sub & 1) ? 2 * gi[0] - o : o;
+            if (d == -1) gi[0] = (sub & 1) ? o : 2 * gi[0] - o;
+          }
           it0 = j0;
-          ta0 = tg0[it0];
-          tb0 = tg0[it0 + 1];
-          n00 = T.nu[c0 * T.TT + it0];
-          n01 = T.nu[c0 * T.TT + it0 + 1];
-        }
-        if (j1 != it1) {
           it1 = j1;
-          ta1 = tg0[T.TT + it1];
-          tb1 = tg0[T.TT + it1 + 1];
-          n10 = T.nu[(c0 + 1) * T.TT + it1];
-          n11 = T.nu[(c0 + 1) * T.TT + it1 + 1];
+          ta0 = tgb[tq0 + it0];
+          rt0 = 1 / (tgb[tq0 + it0 + 1] - ta0);
+          ta1 = tgb[tq0 + T.TT + it1];
+          rt1 = 1 / (tgb[tq0 + T.TT + it1 + 1] - ta1);
+          full = nub[tq0 + it0] >= 2 && nub[tq0 + it0 + 1] >= 2 && nub[tq0 + T.TT + it1] >= 2 &&
+                 nub[tq0 + T.TT + it1 + 1] >= 2;
         }
-        if (n00 < 2 || n01 < 2 || n10 < 2 || n11 < 2) {
-          eps = 0;
+        cell = full;
+      }
+    }
+    // the corner's column of the table
+    auto column = [&](int c) {
+      return (c < 2 ? tq0 + it0 : tq0 + T.TT + it1) + (c & 1);
+    };
+    if (cell && !CGA && mono) {
+#pragma unroll
+      for (int c = 0; c < NC; c++) {
+        gi[c] = gi[c] < -1 ? -1 : (gi[c] > gtop ? gtop : gi[c]);
+        const Col k{knb + (size_t)column(RL == 1 ? c : sub) * T.TS};
+        ka[c] = k[gi[c]];
+        kb[c] = k[gi[c] + 2];
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    const double pn = LOSR(F_P, ipn), tn = LOSR(F_T, ipn), un = LOSR(L.f_u + ig, ipn);
+    __builtin_amdgcn_sched_barrier(0);
+    double eps = opaque ? 1 : 0;
+    if (cell) {
+      double e[4] = {0, 0, 0, 0};
+      if (!CGA && mono) {
+        const double x = 1 - tp;
+        double ec[NC];
+        int bad = 0;
+#pragma unroll
+        for (int c = 0; c < NC; c++) {
+          bool ok;
+          ec[c] = ega_step64(ka[c], kb[c], x, useg, gi[c], ok);
+          bad |= ok ? 0 : 1 << c;
+        }
+        // the corners left, one at a time for each lane
+        while (bad) {
+          int c = 0, g = gi[0];
+          if constexpr (RL == 1) {
+            c = __ffs(bad) - 1;
+            g = c == 0 ? gi[0] : (c == 1 ? gi[1] : (c == 2 ? gi[2] : gi[3]));
+          }
+          const int q = column(RL == 1 ? c : sub);
+          const double v = ega_slow64(Col{knb + (size_t)q * T.TS}, nub[q], x, useg, g);
+#pragma unroll
+          for (int k = 0; k < NC; k++)
+            if (k == c) {
+              ec[k] = v;
+              gi[k] = g;
+            }
+          bad &= bad - 1;
+        }
+        if constexpr (RL == 1) {
+#pragma unroll
+          for (int c = 0; c < 4; c++) e[c] = ec[c];
         } else {
-          const float4 *kc[4];
-          kc[0] = T.rec + (c0 * T.TT + it0) * T.TU;
-          kc[1] = kc[0] + T.TU;
-          kc[2] = T.rec + ((c0 + 1) * T.TT + it1) * T.TU;
-          kc[3] = kc[2] + T.TU;
-          const int nc[4] = {n00, n01, n10, n11};
-          double e[4];
+          e[0] = quad_lane<0>(ec[0]);
+          e[1] = quad_lane<1>(ec[0]);
+          e[2] = quad_lane<2>(ec[0]);
+          e[3] = quad_lane<3>(ec[0]);
+        }
+      } else {
+        if constexpr (CGA) {
           if (mono) {
 #pragma unroll
             for (int c = 0; c < 4; c++) {
+              const int q = column(c);
               float4 r;
-              if (CGA) {
-                gi[c] = col_walk<0>(kc[c], nc[c], cu, gi[c], r);
-                e[c] = eps_from_rec(r, cu);
-              } else {
-                const double x = 1 - tp;
-                const int i = col_walk<1>(kc[c], nc[c], x, gi[c], r);
-                gi[c] = i;
-                const double arg = u_from_rec(r, x) + useg;
-                float4 r2;
-                col_walk_r<0>(kc[c], nc[c], arg, i, r, r2);
-                e[c] = eps_from_rec(r2, arg);
-              }
+              gi[c] = col_walk<0>(Col{knb + (size_t)q * T.TS}, nub[q], cu, gi[c], r);
+              e[c] = eps_from_rec(r, cu);
             }
-          } else {
-            int g2 = 0;
-#pragma unroll
-            for (int c = 0; c < 4; c++)
-              e[c] = CGA ? col_eps(kc[c], nc[c], cu, 0, g2)
-                         : col_eps(kc[c], nc[c], col_u(kc[c], nc[c], 1 - tp, 0, g2) + useg, 0, g2);
           }
-          double e00 = lin(ta0, e[0], tb0, e[1], tq);
-          const double e11 = lin(ta1, e[2], tb1, e[3], tq);
-          e00 = CGA ? logx(pa, e00, pb, e11, pq) : lin(pa, e00, pb, e11, pq);
-          e00 = (e00 < 1) ? e00 : 1;  // MAX(MIN(eps00, 1), 0)
-          e00 = (e00 > 0) ? e00 : 0;
-          eps = 1 - (1 - e00) / tp;
+        }
+        if (!mono) {
+#pragma unroll 1
+          for (int c = 0; c < 4; c++) {
+            const int q = column(c), n = nub[q];
+            const Col k{knb + (size_t)q * T.TS};
+            int g2 = 0;
+            const double v = CGA ? col_eps(k, n, cu, 0, g2)
+                                 : col_eps(k, n, col_u(k, n, 1 - tp, 0, g2) + useg, 0, g2);
+            e[0] = c == 0 ? v : e[0];
+            e[1] = c == 1 ? v : e[1];
+            e[2] = c == 2 ? v : e[2];
+            e[3] = c == 3 ? v : e[3];
+          }
         }
       }
+      const double w0 = (tq - ta0) * rt0, w1 = (tq - ta1) * rt1;
+      double e00 = e[0] + (e[1] - e[0]) * w0;
+      const double e11 = e[2] + (e[3] - e[2]) * w1;
+      e00 = CGA ? logx(pa, e00, pb, e11, pq) : e00 + (e11 - e00) * ((pq - pa) * rp);
+      e00 = (e00 < 1) ? e00 : 1;  // MAX(MIN(eps00, 1), 0)
+      e00 = (e00 > 0) ? e00 : 0;
+      eps = 1 - (1 - e00) / tp;
     }
     tp *= (1 - eps);
-    out[(size_t)ip * WAVE] = PATH ? tp : eps;
+    if (sub == 0) out[(size_t)ip * WAVE] = PATH ? tp : eps;
+    p = pn;
+    t = tn;
+    useg = un;
   }
 }
 
 void launch_lookup_f64(const ModelView &M, const BatchView &B, const LosView &L, const EpsView &E,
                        const RayInfo *info, int blk0, int nblk, bool path, hipStream_t s) {
   if (M.nd * M.ng == 0) return;
-  const dim3 grid(padded_blocks(nblk) * M.nd * M.ng), blk(WAVE);
+  const size_t chains = (size_t)padded_blocks(nblk) * M.nd * M.ng;
+  const dim3 grid(chains), blk(WAVE);
   if (M.formod == 0) {
     if (path) hipLaunchKernelGGL((k_lookup_f64<true, true>), grid, blk, 0, s, M, B, L, E, info, blk0, nblk);
     else hipLaunchKernelGGL((k_lookup_f64<true, false>), grid, blk, 0, s, M, B, L, E, info, blk0, nblk);
+  } else if (chains * 4 <= 4096) {
+    // small batches: four lanes per chain while that stays within the four
+    // wavefronts per SIMD its registers allow
+    const dim3 g4(chains * 4);
+    if (path) hipLaunchKernelGGL((k_lookup_f64<false, true, 4>), g4, blk, 0, s, M, B, L, E, info, blk0, nblk);
+    else hipLaunchKernelGGL((k_lookup_f64<false, false, 4>), g4, blk, 0, s, M, B, L, E, info, blk0, nblk);
   } else {
     if (path) hipLaunchKernelGGL((k_lookup_f64<false, true>), grid, blk, 0, s, M, B, L, E, info, blk0, nblk);
     else hipLaunchKernelGGL((k_lookup_f64<false, false>), grid, blk, 0, s, M, B, L, E, info, blk0, nblk);

@@ -13,6 +13,7 @@ All calls go through the C-ABI.
 import ctypes as C
 import os
 import shutil
+import struct
 
 import numpy as np
 import pytest
@@ -238,3 +239,45 @@ def test_device_tables_capacity_errors(gpu):
     with pytest.raises(gpu.JurassicError) as e:
         gpu.Context.from_device_tables(ctl, [ctl.nu[i] for i in range(ctl.nd)], tabs)
     assert "pressure levels" in str(e.value)
+
+
+def _ragged_tables(ctl):
+    """Cut every table's columns to different ranges: columns of two and
+    three knots, columns that start far up (paths start below their first
+    knot) or end early (paths grow past their last knot), a repeated
+    emissivity, and full ones."""
+    for id_ in range(ctl.nd):
+        for ig in range(ctl.ng):
+            fn = scenes.table_name(ctl.tblbase.decode(), ctl.nu[id_], ctl.emitter[ig].value.decode(), 2)
+            pg, ts, cols = scenes.read_table_bin(fn)
+            with open(fn, "wb") as f:
+                f.write(struct.pack("<i", len(pg)) + np.asarray(pg, "<f8").tobytes())
+                for ip in range(len(pg)):
+                    f.write(struct.pack("<i", len(ts[ip])) + np.asarray(ts[ip], "<f8").tobytes())
+                    for it, (u, e) in enumerate(cols[ip]):
+                        k = (3 * ip + 5 * it + 7 * id_ + ig) % 6
+                        i = [np.arange(len(u)), np.arange(40, len(u)), np.arange(0, 130), np.array([60, 110]),
+                             np.array([0, 90, 199]), np.arange(25, 150, 4)][k]
+                        e = e[i].copy()
+                        if k == 5:
+                            e[12] = e[13]
+                        f.write(struct.pack("<i", len(i)) + u[i].astype("<f4").tobytes() + e.astype("<f4").tobytes())
+
+
+def test_ragged_columns(gpu, tmp_path):
+    """Columns of very different lengths and ranges (see _ragged_tables):
+    the oracle's radiances from files and from device memory, and the same
+    bits from a batch large enough for one lane per chain (40 ray blocks x 36
+    chains) as from a small one (four lanes)."""
+    torch = pytest.importorskip("torch")
+    ctl = _scene_copy(tmp_path, scenes.limb_3gas_ctl(), "ragged")
+    _ragged_tables(ctl)
+    _same_as_files(gpu, ctl, torch)
+    ctx = gpu.Context(ctl)
+    try:
+        for prec in (abi.JUR_FP64, abi.JUR_FP32):
+            out = [_forward(ctx, ctl, _limb_batch(ctl, torch, n), prec, torch)[0].reshape(-1, n, ctl.nd)[:, :3]
+                   for n in (3, 320)]
+            assert np.array_equal(out[0], out[1]), prec
+    finally:
+        ctx.close()
