@@ -33,6 +33,8 @@ namespace jur {
 size_t ray_tail_bytes();
 void launch_raytrace(const ModelView &, const BatchView &, const LosView &, RayInfo *, void *, int, int,
                      hipStream_t);
+void launch_ray_points(const ModelView &, const BatchView &, const LosView &, const RayInfo *, const void *, int, int,
+                       int, hipStream_t);
 void launch_hydrostatic(atm_t *, int, double, int, hipStream_t);
 void launch_lookup_f64(const ModelView &, const BatchView &, const LosView &, const EpsView &,
                        const RayInfo *, int, int, bool, hipStream_t);
@@ -791,6 +793,10 @@ int forward_pass(jur_ctx *c, const BatchView &B, int precision, const unsigned c
         if (Ls.losf) Ls.losf = L.losf + (size_t)s0 * L.cap * L.nfield * WAVE;
         EpsView E{d_eps, d_eoff, d_npb + s0, d_part};
         const int bs = b0 + s0;
+        const int maxnp = *std::max_element(npb.begin() + s0, npb.begin() + s1);
+        HIPCHK(hipEventRecord(c->ev[0], st));
+        launch_ray_points(M, B, Ls, d_info, d_tail, bs, ns, maxnp, st);
+        HIPCHK(hipGetLastError());
         HIPCHK(hipEventRecord(c->ev[1], st));
         if (precision == JUR_FP32) launch_lookup_f32(M, B, Ls, E, d_info, bs, ns, st);
         else launch_lookup_f64(M, B, Ls, E, d_info, bs, ns, jac != nullptr, st);
@@ -807,7 +813,6 @@ int forward_pass(jur_ctx *c, const BatchView &B, int precision, const unsigned c
           launch_zero(d_kt, (size_t)ns * s.nd * jac->ncol * WAVE, st);
           JacView J{jac->xmap, jac->nmap, jac->prof_map, jac->ncol, d_kt, d_scr, d_soff, nscr, d_nef,
                     dpath ? nscr0 : -1, d_pco};
-          const int maxnp = *std::max_element(npb.begin() + s0, npb.begin() + s1);
           launch_adjoint(M, B, Ls, E, d_info, d_tail, bs, ns, maxnp, J, precision == JUR_FP32, d_rad, d_tau, st);
           HIPCHK(hipGetLastError());
           launch_jac_store(d_kt, s.nd, jac->ncol, bs, ns, B.nray, d_rad, c->d_chan.p, s.write_bbt, d_mask,
@@ -820,7 +825,7 @@ int forward_pass(jur_ctx *c, const BatchView &B, int precision, const unsigned c
         HIPCHK(hipGetLastError());
         HIPCHK(hipEventRecord(c->ev[3], st));
         HIPCHK(hipEventSynchronize(c->ev[3]));
-        for (int k = 1; k < 3; k++) {
+        for (int k = 0; k < 3; k++) {
           float a = 0;
           HIPCHK(hipEventElapsedTime(&a, c->ev[k], c->ev[k + 1]));
           ms[k] += a;

@@ -581,3 +581,29 @@ def test_lookup_lanes_per_chain_jacobian_agree(gpu):
     assert np.array_equal(r0, r1)
     assert np.isfinite(k0).all() and np.abs(k0).max() > 0
     np.testing.assert_allclose(k1, k0, rtol=1e-13, atol=1e-13 * np.abs(k0).max())
+
+
+@pytest.mark.parametrize("nlev,up,refrac", [(2, True, 1), (8, False, 1), (9, True, 0), (10, True, 1), (17, False, 1)])
+def test_level_grids(gpu, oracle, nlev, up, refrac):
+    """Level counts around the rounds of eight of the march's altitude scan,
+    ascending and descending grids, with and without refraction: the
+    oracle's radiances and tangent points of limb and nadir rays.
+    Transmittances to 1e-10 relative or 1e-30: that of a path of optical
+    depth x carries x times the rounding of the depth, which is summed over
+    about 1000 segments (up to 1e-12), so 1e-10 need not hold beyond x = 70."""
+    z = np.linspace(0.0, 80.0, nlev)
+    ctl, _, obs = scenes.limb_3gas(0, nrays=7)
+    ctl.refrac = refrac
+    atm = scenes.make_profile_atm(["CO2", "H2O", "O3"], z=z, perturb=False)
+    if not up:
+        rows = [atm.z, atm.p, atm.t] + [atm.q[g] for g in range(3)]
+        for a in rows:
+            v = abi.np_view(a)
+            v[:nlev] = v[:nlev][::-1].copy()
+    for o in (obs, scenes.make_obs(scenes.nadir_geometry(705.0, [0.0, 30.0, 55.0]))):
+        (_, oc), (_, og) = _run_both(gpu, oracle, ctl, atm, o)
+        r1, t1 = abi.obs_arrays(og, ctl)
+        r0, t0 = abi.obs_arrays(oc, ctl)
+        _cmp(r1, r0, RTOL64, "rad")
+        _cmp(t1, t0, RTOL64, "tau", atol=1e-30)
+        _cmp(abi.np_view(og.tpz)[:o.nr], abi.np_view(oc.tpz)[:o.nr], 1e-11, "tpz", atol=1e-9)
