@@ -390,19 +390,33 @@ __device__ __forceinline__ float ega_step_slow(Col col, int n, float ep, double 
   const int i = col_walk_f<1>(col, n, ep, g, r);
   g = ep < r.y ? -1 : i;
   if (ep > r.w) return ega_step_above<D>(r.z, r.w, ep, (float)useg, dep, deu);
-  // the bracket of ep: through the origin below the first knot
-  const float x0 = ep < r.y ? 0.f : r.x, y0 = ep < r.y ? 0.f : r.y;
-  const float dx = (ep < r.y ? r.x : r.z) - x0, dy = (ep < r.y ? r.y : r.w) - y0;
-  const float su = fdiv(dx, dy);
-  const float off = (ep - y0) * su + (float)useg;
-  if (off < dx) {
-    const float se = fdiv(dy, dx);
+  // the bracket of ep (through the origin below the first knot) and the knot
+  // after it: inside the bracket and up to that knot the operations of
+  // ega_step_fast, so the result does not depend on where the search started
+  const bool below = ep < r.y;
+  const float2 k2 = below ? make_float2(r.z, r.w) : col.k[i + 2];
+  const float x0 = below ? 0.f : r.x, y0 = below ? 0.f : r.y, x1 = below ? r.x : r.z, y1 = below ? r.y : r.w;
+  const float s0 = fdiv(y1 - y0, x1 - x0), s1 = fdiv(k2.y - y1, k2.x - x1);
+  const float x = ep + (float)useg * s0;
+  if (x < y1) {
     if (D) {
       dep = 1.f;
-      deu = se;
+      deu = s0;
     }
-    return ep + (float)useg * se;
+    return x;
   }
+  const float ratio = fdiv(s1, s0);
+  const float y = y1 + (x - y1) * ratio;
+  if (y < k2.y) {
+    if (D) {
+      dep = ratio;
+      deu = s1;
+    }
+    return y;
+  }
+  // further up: by the column density
+  const float su = fdiv(x1 - x0, y1 - y0);
+  const float off = (ep - y0) * su + (float)useg;
   const double arg = (double)x0 + (double)off;
   float se;
   col_walk_r<0>(col, n, arg, i, r, r2);

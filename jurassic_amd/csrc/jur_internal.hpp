@@ -69,6 +69,10 @@ struct TabView {
                            // T-grid sizes and T grids (one cell search per
                            // segment serves all of them)
   int ref_tix;             // a table holding the shared grids
+  int cells;               // 1 if the tables are shared and all_mono, on a strictly
+                           // monotone p grid, and every row and column of them has
+                           // two entries: a cell is then the same for all of them
+                           // and never without data
   // column c = (table * TP + p) * TT + T
   __device__ __forceinline__ Col col(size_t c) const { return Col{kn + c * TS + 1}; }
 };
@@ -101,6 +105,12 @@ struct LosView {
   float *losf;  // FP32 forward pass: the fields rounded to float, same layout
                 // (the FP32 radiance kernel rounds every field it reads);
                 // null otherwise
+  float4 *cell; // FP32 EGA over tables of one grid (TabView::cells): per point
+                // ncell records, layout [block][cap][lane][ncell]: (columns
+                // c00 | c10 << 16 of the cell's two temperature brackets,
+                // weights in T on its two pressures, weight in p) and for the
+                // Jacobian (their slopes in T, T and p, 0); null otherwise
+  int ncell;
   int f_xe;     // Jacobian pass with refraction: first of six fields holding
                 // the point's Cartesian position and the march direction
                 // leaving it (x0 x1 x2 e0 e1 e2); -1 otherwise

@@ -273,10 +273,11 @@ namespace jur {
 // and T grids as the first such table (one cell search per segment then
 // serves all of them).
 static void detect_shared(jur_ctx *c, const std::vector<int> &h_np, const std::vector<int> &h_nt,
+                          const std::vector<int> &h_nu, const std::vector<int> &h_pdir,
                           const std::vector<double> &h_p, const std::vector<double> &h_t) {
   const size_t ntab = (size_t)c->s.nd * c->s.ng;
   const int TP = c->TP, TT = c->TT;
-  c->shared = 0;
+  c->shared = c->cells = 0;
   c->ref_tix = 0;
   int ref = -1;
   for (size_t k = 0; k < ntab; k++)
@@ -294,6 +295,17 @@ static void detect_shared(jur_ctx *c, const std::vector<int> &h_np, const std::v
   }
   c->shared = same ? 1 : 0;
   c->ref_tix = ref;
+  // cells located once for all tables: none without data, columns in 16 bits
+  c->cells = same && c->all_mono && h_pdir[ref] != 0 && TP * TT <= 65536;
+  for (size_t k = 0; k < ntab && c->cells; k++) {
+    if (h_np[k] < 30) continue;
+    for (int ip = 0; ip < h_np[k]; ip++) {
+      const size_t row = k * TP + ip;
+      if (h_nt[row] < 2) c->cells = 0;
+      for (int it = 0; it < h_nt[row]; it++)
+        if (h_nu[row * TT + it] < 2) c->cells = 0;
+    }
+  }
 }
 
 // Direction of a table's pressure grid: +1 strictly ascending, -1 strictly
@@ -374,7 +386,7 @@ static int build_tables(jur_ctx *c) {
   if ((rc = c->d_t.upload(h_t.data(), h_t.size()))) return rc;
   if ((rc = c->d_kn.upload(h_kn.data(), h_kn.size()))) return rc;
   c->table_bytes = h_kn.size() * sizeof(float2);
-  detect_shared(c, h_np, h_nt, h_p, h_t);
+  detect_shared(c, h_np, h_nt, h_nu, h_pdir, h_p, h_t);
   return JUR_OK;
 }
 
@@ -458,7 +470,7 @@ static int build_tables_device(jur_ctx *c, const jur_dtables_t *d) {
   c->all_mono = 1;
   for (size_t k = 0; k < ntab; k++)
     if (h_np[k] >= 30 && !h_mono[k]) c->all_mono = 0;
-  detect_shared(c, h_np, h_nt, h_p, h_t);
+  detect_shared(c, h_np, h_nt, h_nu, h_pdir, h_p, h_t);
   return JUR_OK;
 }
 
@@ -606,6 +618,7 @@ static ModelView model_view(const jur_ctx *c) {
   T.shared = c->shared;
   T.ref_tix = c->ref_tix;
   T.all_mono = c->all_mono;
+  T.cells = c->cells;
   return M;
 }
 
@@ -696,7 +709,11 @@ int forward_pass(jur_ctx *c, const BatchView &B, int precision, const unsigned c
     // the FP32 forward pass also keeps the fields rounded to float (what its
     // radiance kernel reads)
     const bool losf = precision == JUR_FP32 && !jac;
-    const size_t los_blk = (size_t)L.nfield * L.cap * WAVE * (sizeof(double) + (losf ? sizeof(float) : 0));
+    // FP32 EGA over tables of one grid: each point's cell, located once
+    const bool cells = precision == JUR_FP32 && M.formod != 0 && M.tab.cells;
+    L.ncell = part ? 2 : 1;
+    const size_t los_blk = (size_t)L.nfield * L.cap * WAVE * (sizeof(double) + (losf ? sizeof(float) : 0)) +
+                           (cells ? (size_t)L.ncell * L.cap * WAVE * sizeof(float4) : 0);
     const size_t pt_blk = (size_t)s.nd * s.ng * WAVE * (esz + (part ? sizeof(float4) : 0)) +
                           (jac ? (size_t)s.nd * nscr * WAVE * sizeof(double) : 0) +
                           (dpath ? (size_t)JUR_NPCO * WAVE * sizeof(double) : 0);
@@ -717,6 +734,7 @@ int forward_pass(jur_ctx *c, const BatchView &B, int precision, const unsigned c
       if (kind != c->pass_kind) {
         c->d_los.release();
         c->d_losf.release();
+        c->d_cell.release();
         c->d_eps.release();
         c->d_part.release();
         c->d_kt.release();
@@ -726,7 +744,8 @@ int forward_pass(jur_ctx *c, const BatchView &B, int precision, const unsigned c
       }
       size_t fr = 0, tot = 0;
       HIPCHK(hipMemGetInfo(&fr, &tot));
-      fr += c->d_los.n * sizeof(double) + c->d_losf.n * sizeof(float) + c->d_eps.n + c->d_part.n * sizeof(float4) +
+      fr += c->d_los.n * sizeof(double) + c->d_losf.n * sizeof(float) + c->d_eps.n +
+            (c->d_part.n + c->d_cell.n) * sizeof(float4) +
             (c->d_kt.n + c->d_scr.n + c->d_pco.n) * sizeof(double);
       budget = std::min(fr / 2, (size_t)96 << 30);
     }
@@ -744,10 +763,13 @@ int forward_pass(jur_ctx *c, const BatchView &B, int precision, const unsigned c
     if (jac && (rc = pm.get(c->d_soff, chunk, &d_soff))) return rc;
     if ((rc = pm.get(c->d_los, (size_t)L.nfield * L.cap * WAVE * chunk, &d_los))) return rc;
     if (losf && (rc = pm.get(c->d_losf, (size_t)L.nfield * L.cap * WAVE * chunk, &d_losf))) return rc;
+    float4 *d_cell = nullptr;
+    if (cells && (rc = pm.get(c->d_cell, (size_t)L.ncell * L.cap * WAVE * chunk, &d_cell))) return rc;
     if (pm.base) rest = pm.cap - pm.used;
     const size_t mark1 = pm.used;
     L.los = d_los;
     L.losf = d_losf;
+    L.cell = d_cell;
     std::vector<int> npb(chunk);
     std::vector<size_t> eoff(chunk), soff(chunk);
     float ms[3] = {0, 0, 0};
@@ -791,6 +813,7 @@ int forward_pass(jur_ctx *c, const BatchView &B, int precision, const unsigned c
         LosView Ls = L;
         Ls.los = L.los + (size_t)s0 * L.cap * L.nfield * WAVE;
         if (Ls.losf) Ls.losf = L.losf + (size_t)s0 * L.cap * L.nfield * WAVE;
+        if (Ls.cell) Ls.cell = L.cell + (size_t)s0 * L.cap * L.ncell * WAVE;
         EpsView E{d_eps, d_eoff, d_npb + s0, d_part};
         const int bs = b0 + s0;
         const int maxnp = *std::max_element(npb.begin() + s0, npb.begin() + s1);

@@ -558,6 +558,48 @@ __global__ __launch_bounds__(WAVE) void k_ray_points(ModelView M, BatchView B, L
   extern __shared__ double lvl[];
 #define LV(f) lvl[(f) * WAVE + lane]
   LevelCache lc;
+  // the tables' cell of a point (LosView::cell): the pressure bracket and,
+  // on its two pressures, the temperature brackets and weights, with the
+  // arithmetic of the FP32 lookups (float, reciprocal spacings)
+  const TabView &T = M.tab;
+  float4 *cell = L.cell ? L.cell + ((size_t)bl * L.cap * WAVE + lane) * L.ncell : nullptr;
+  const double *pg = T.p + (size_t)T.ref_tix * T.TP;
+  const double *tgb = T.t + (size_t)T.ref_tix * T.TP * T.TT;
+  const int *ntp = T.nt + (size_t)T.ref_tix * T.TP;
+  const int npt = cell ? T.np[T.ref_tix] : 0, pdir = cell ? T.pdir[T.ref_tix] : 0;
+  int ipr = -1;
+  double pa = 0, pb = 0;
+  float rwp = 0, g00 = 0, gi0 = 0, g10 = 0, gi1 = 0;
+  int nt0 = 0, nt1 = 0;
+  auto put_cell = [&](double p, double t, int ip) {
+    const bool keep = ipr >= 0 && (pdir > 0 ? (ipr == 0 || !(pa > p)) && (ipr == npt - 2 || pb > p)
+                                            : (ipr == 0 || !(pa <= p)) && (ipr == npt - 2 || pb <= p));
+    if (!keep) {
+      ipr = ipr >= 0 ? irr_walk(pg, npt, p, ipr, pdir) : locate_irr(pg, npt, p);
+      pa = pg[ipr];
+      pb = pg[ipr + 1];
+      rwp = frcp((float)(pb - pa));
+      nt0 = ntp[ipr];
+      nt1 = ntp[ipr + 1];
+      const double *tg = tgb + (size_t)ipr * T.TT;
+      g00 = (float)tg[0];
+      gi0 = frcp((float)(tg[1] - tg[0]));
+      g10 = (float)tg[T.TT];
+      gi1 = frcp((float)(tg[T.TT + 1] - tg[T.TT]));
+    }
+    const float tq = (float)t;
+    int j0 = (int)((tq - g00) * gi0);
+    j0 = j0 < 0 ? 0 : (j0 > nt0 - 2 ? nt0 - 2 : j0);
+    int j1 = (int)((tq - g10) * gi1);
+    j1 = j1 < 0 ? 0 : (j1 > nt1 - 2 ? nt1 - 2 : j1);
+    const int c00 = ipr * T.TT + j0, c10 = (ipr + 1) * T.TT + j1;
+    const double ta0 = tgb[c00], ta1 = tgb[c10];
+    const float dt0 = frcp((float)(tgb[c00 + 1] - ta0)), dt1 = frcp((float)(tgb[c10 + 1] - ta1));
+    float4 *o = cell + (size_t)ip * WAVE * L.ncell;
+    o[0] = make_float4(__int_as_float(c00 | c10 << 16), (tq - (float)ta0) * dt0, (tq - (float)ta1) * dt1,
+                       (float)(p - pa) * rwp);
+    if (L.ncell > 1) o[1] = make_float4(dt0, dt1, rwp, 0.f);
+  };
   double z = LOSW(F_Z, i0), ds = LOSW(F_DS, i0);
   for (int ip = i0; ip < i1; ip++) {
     const int ipn = ip + 1 < i1 ? ip + 1 : ip;
@@ -588,8 +630,13 @@ __global__ __launch_bounds__(WAVE) void k_ray_points(ModelView M, BatchView B, L
       if (basef) LOS_AT(basef, L, f, ip) = (float)v;
       else LOSW(f, ip) = v;
     };
-    LOSW(F_P, ip) = p;
-    LOSW(F_T, ip) = t;
+    if (cell) {
+      put_cell(p, t, ip);
+    }
+    if (!cell || !basef) {
+      LOSW(F_P, ip) = p;
+      LOSW(F_T, ip) = t;
+    }
     if (basef) {
       put(F_P, p);
       put(F_T, t);

@@ -281,3 +281,29 @@ def test_ragged_columns(gpu, tmp_path):
             assert np.array_equal(out[0], out[1]), prec
     finally:
         ctx.close()
+
+
+@pytest.mark.parametrize("nprof", [3, 320])
+def test_cells_equal_general(gpu, tmp_path, nprof):
+    """FP32 EGA on tables that share their grids (each point's cell located
+    once, with the ray) and on the same tables beside one that has a
+    pressure more (each chain locates its own): the same bits in the other
+    channels, with four lanes per chain (3 atmospheres) and with one."""
+    torch = pytest.importorskip("torch")
+    ctl = scenes.limb_3gas_ctl()
+    other = _scene_copy(tmp_path, ctl, "grid")
+    fn = scenes.table_name(other.tblbase.decode(), ctl.nu[0], "H2O", 2)
+    pg, ts, cols = scenes.read_table_bin(fn)
+    eps = np.array([[cols[ip][it][1] for it in range(len(ts[ip]))] for ip in range(len(pg))], dtype=np.float32)
+    scenes.write_table_bin(fn, np.append(pg, 1.1 * pg[-1]), ts[0], cols[0][0][0], np.append(eps, eps[-1:], axis=0))
+    batch = _limb_batch(ctl, torch, nprof)
+    out = []
+    for c in (ctl, other):
+        ctx = gpu.Context(c)
+        try:
+            out.append(_forward(ctx, c, batch, abi.JUR_FP32, torch))
+        finally:
+            ctx.close()
+    assert np.array_equal(out[0][0][:, 1:], out[1][0][:, 1:])
+    assert np.array_equal(out[0][1][:, 1:], out[1][1][:, 1:])
+    np.testing.assert_allclose(out[1][0][:, 0], out[0][0][:, 0], rtol=1e-5)
