@@ -6,6 +6,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "jur_internal.hpp"
 
 namespace jur {
@@ -802,6 +804,52 @@ __device__ __forceinline__ int xcd_remap(int wg, int nwg) {
   if (k < per) return x * per + (x < rem ? x : rem) + k;
   // tail ids (k == per) exist only for x < rem
   return x * per + x + k;
+}
+
+// ------------------------------------------------------------------
+// Sums along a path in chunks of RAD_CH points (the FP32 radiance kernel): each
+// chunk's radiance, transmittance and down-welling sum as if it began the
+// path, joined in path order.  The chunks do not depend on each other, so a
+// small batch, whose duration is one path's, takes them on the PW waves of a
+// workgroup (32 points: a few rounds of 16 waves for the ~800 to 1500 points
+// of a path, against a join of three operations); a large one in one wave.
+// Both join the same chunks in the same order, so the sums are the same bits.
+// ------------------------------------------------------------------
+constexpr int RAD_CH = 32;
+
+struct PathSum {
+  double rad = 0, tau = 1, drefl = 0;
+  __device__ __forceinline__ void append(const PathSum &c) {
+    JUR_FP_EXACT
+    rad = rad + tau * c.rad;
+    drefl = drefl * c.tau + c.drefl;
+    tau = tau * c.tau;
+  }
+  // sum: the path up to this round's PW chunks, c: the wave's chunk
+  template <int PW>
+  static __device__ __forceinline__ void join(PathSum &sum, double (*part)[3][WAVE], int wv, int lane,
+                                              const PathSum &c) {
+    if constexpr (PW == 1) {
+      sum.append(c);
+    } else {
+      part[wv][0][lane] = c.rad;
+      part[wv][1][lane] = c.tau;
+      part[wv][2][lane] = c.drefl;
+      __syncthreads();
+      if (wv == 0)
+        for (int k = 0; k < PW; k++) sum.append(PathSum{part[k][0][lane], part[k][1][lane], part[k][2][lane]});
+      __syncthreads();
+    }
+  }
+};
+
+// Runs a kernel of g workgroups with the most waves each, TOP, 4 or 1, that
+// stay within `all` waves (what runs at once).
+template <int TOP, typename F>
+void launch_paths(unsigned g, unsigned all, F run) {
+  if (g <= all / TOP) run(std::integral_constant<int, TOP>{});
+  else if (g <= all / 4) run(std::integral_constant<int, 4>{});
+  else run(std::integral_constant<int, 1>{});
 }
 
 // ------------------------------------------------------------------

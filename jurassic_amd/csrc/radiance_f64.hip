@@ -4,8 +4,15 @@
 // src/jurassic.c:3233-3334).
 //
 // One wavefront per (block of 64 rays, channel), lane = ray.  Every segment
-// field is read with one coalesced access per wavefront; the work per segment
-// is a few FP64 operations, so the kernel streams.
+// field is read with one coalesced access per wavefront.
+//
+// The segments' emissivities and source functions do not depend on each
+// other, only the sums do.  A small batch, whose duration is one path's, forms
+// them on the PW = 8 waves of a workgroup, RAD64_PT points each per round, and
+// adds them in path order on the first wave: the same operations in the same
+// order as on one wave, so the same bits (0.63 -> 0.1 ms for 10 nadir rays of
+// 805 points; joining the sums of chunks, as the FP32 kernel does, would
+// round differently from the reference).
 //
 // Built with -ffp-contract=off; operation order follows the reference,
 // except that the per-segment continua and source function multiply by
@@ -17,20 +24,27 @@
 
 namespace jur {
 
+constexpr int RAD64_PT = 8;
+
 #define LOSR(f, ip) LOS_AT(los, L, f, ip)
 
-__global__ __launch_bounds__(WAVE) void k_radiance_f64(ModelView M, BatchView B, LosView L,
+template <int PW>
+__global__ __launch_bounds__(WAVE *PW) void k_radiance_f64(ModelView M, BatchView B, LosView L,
                                                        EpsView E, const RayInfo *info, int blk0,
                                                        int nblk, double *rad_out, double *tau_out) {
   JUR_FP_EXACT
   const int nd = M.nd, ng = M.ng;
   int bl, id;
   if (!xcd_block_map(blockIdx.x, nd, nblk, bl, id)) return;
-  const int lane = threadIdx.x;
-  const int ir = (blk0 + bl) * WAVE + lane;
-  if (ir >= B.nray) return;
-  const RayInfo R = info[ir];
-  if (R.status != JUR_OK) return;
+  const int lane = threadIdx.x % WAVE;
+  const int wv = PW == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+  // lanes without a ray follow the last one (the waves meet at barriers) and
+  // write nothing
+  const bool live = (blk0 + bl) * WAVE + lane < B.nray;
+  const int ir = live ? (blk0 + bl) * WAVE + lane : B.nray - 1;
+  RayInfo R = info[ir];
+  const bool write = live && R.status == JUR_OK && wv == 0;
+  if (!live || R.status != JUR_OK) R.np = 0;
 
   const atm_t *atm = &B.atm[B.ray_prof[ir]];
   const ChanInfo C = M.chan[id];
@@ -50,18 +64,33 @@ __global__ __launch_bounds__(WAVE) void k_radiance_f64(ModelView M, BatchView B,
   const bool has_k = C.window < M.nw;
   const CtmChan K = ctm_chan(M.ctm, nu);
 
-  double rad = 0, tau = 1, drefl = 0, tau_refl = 1;
-  for (int ip = 0; ip < R.np; ip++) {
-    const double p = LOSR(F_P, ip);
-    const double t = LOSR(F_T, ip);
-    const double ds = LOSR(F_DS, ip);
+  // emitters with a table (the others have eps = 0)
+  unsigned gmask = 0;
+  for (int g = 0; g < ng; g++)
+    if (M.tab.np[g * nd + id] >= 30) gmask |= 1u << g;
+  struct Point {
+    double p, t, ds, e[4];
+  };
+  // what a point's arithmetic begins with: p, t, ds and its first four emitters
+  auto load = [&](int ip) {
+    Point x;
+    x.p = LOSR(F_P, ip);
+    x.t = LOSR(F_T, ip);
+    x.ds = LOSR(F_DS, ip);
+#pragma unroll
+    for (int g = 0; g < 4; g++) x.e[g] = g < ng && (gmask >> g & 1u) ? eps_g[((size_t)g * npb + ip) * WAVE] : 0.0;
+    return x;
+  };
 
+  // a = src eps and s = 1 - eps of a segment (0 and 1 for one that adds nothing)
+  auto segment = [&](int ip, const Point &x, double &a, double &s) {
+    const double p = x.p, t = x.t, ds = x.ds;
     // tau_seg = prod_g (1 - eps_g), emitter order (intpol_tbl_ega)
     double tau_gas = 1;
-    for (int g = 0; g < ng; g++) {
-      const double eps = (M.tab.np[g * nd + id] < 30) ? 0.0 : eps_g[((size_t)g * npb + ip) * WAVE];
-      tau_gas *= (1 - eps);
-    }
+#pragma unroll
+    for (int g = 0; g < 4; g++) tau_gas *= (1 - x.e[g]);
+    for (int g = 4; g < ng; g++)
+      if (gmask >> g & 1u) tau_gas *= (1 - eps_g[((size_t)g * npb + ip) * WAVE]);
 
     // formod_continua (src/jurassic.c:3075-3117)
     const double rt = 1 / t, rds = 1 / ds;
@@ -74,18 +103,57 @@ __global__ __launch_bounds__(WAVE) void k_radiance_f64(ModelView M, BatchView B,
     if (M.ctm_o2) beta += ctmo2_seg(K, p, rt);
 
     const double src = srcfunc_u(M.st, inv_dst, sr_col, t);
-
+    a = 0;
+    s = 1;
     if (tau_gas > 0) {
       const double eps = 1 - tau_gas * exp(-beta * ds);
-      rad += src * eps * tau;
-      tau *= (1 - eps);
-      // down-welling sum of the reflection term, accumulated forward:
-      // D = sum_i src_i eps_i prod_{k>i} (1 - eps_k)
-      drefl = drefl * (1 - eps) + src * eps;
-      tau_refl *= (1 - eps);
+      a = src * eps;
+      s = 1 - eps;
+    }
+  };
+
+  double rad = 0, tau = 1, drefl = 0;
+  // the down-welling sum of the reflection term is accumulated forward:
+  // D = sum_i src_i eps_i prod_{k>i} (1 - eps_k)
+  auto add = [&](double a, double s) {
+    rad += a * tau;
+    tau *= s;
+    drefl = drefl * s + a;
+  };
+  if constexpr (PW == 1) {
+    for (int ip = 0; ip < R.np; ip++) {
+      double a, s;
+      segment(ip, load(ip), a, s);
+      add(a, s);
+    }
+  } else {
+    extern __shared__ double2 seg[];  // [points of a round][lane]
+    constexpr int RP = PW * RAD64_PT;
+    for (int r0 = 0; r0 < npb; r0 += RP) {
+      const int i0 = r0 + wv * RAD64_PT;
+      const int i1 = i0 + RAD64_PT < R.np ? i0 + RAD64_PT : R.np;
+      Point nx{};
+      if (i0 < i1) nx = load(i0);
+      for (int ip = i0; ip < i1; ip++) {
+        const Point x = nx;
+        nx = load(ip + 1 < i1 ? ip + 1 : ip);
+        double2 v;
+        segment(ip, x, v.x, v.y);
+        seg[(ip - r0) * WAVE + lane] = v;
+      }
+      __syncthreads();
+      if (wv == 0) {
+        const int n = R.np - r0 < RP ? R.np - r0 : RP;
+        for (int k = 0; k < n; k++) {
+          const double2 v = seg[k * WAVE + lane];
+          add(v.x, v.y);
+        }
+      }
+      __syncthreads();
     }
   }
 
+  if (!write) return;
   // surface emission, reflection and solar term (src/jurassic.c:3262-3328)
   if (M.sftype >= 1 && R.sft > 0) {
     const double src_sf = srcfunc(M.st, sr_col, R.sft);
@@ -93,7 +161,7 @@ __global__ __launch_bounds__(WAVE) void k_radiance_f64(ModelView M, BatchView B,
     if (M.sftype >= 2 && sfeps < 1) {
       rad += drefl * tau * (1 - sfeps);
       if (M.sftype >= 3 && R.pad > 0)
-        rad += 6.764e-5 / (2. * JUR_PI) * C.planck_sun * tau_refl * (1 - sfeps) * tau * R.rcos;
+        rad += 6.764e-5 / (2. * JUR_PI) * C.planck_sun * tau * (1 - sfeps) * tau * R.rcos;
     }
   }
   rad_out[(size_t)ir * nd + id] = rad;
@@ -104,8 +172,14 @@ void launch_radiance_f64(const ModelView &M, const BatchView &B, const LosView &
                          const RayInfo *info, int blk0, int nblk, double *rad, double *tau,
                          hipStream_t s) {
   if (M.nd == 0) return;
-  hipLaunchKernelGGL(k_radiance_f64, dim3(padded_blocks(nblk) * M.nd), dim3(WAVE), 0, s, M, B, L, E, info, blk0,
-                     nblk, rad, tau);
+  const unsigned g = (unsigned)padded_blocks(nblk) * M.nd;
+  // eight waves a path while all workgroups run at once (one per CU, whose LDS
+  // and registers hold two)
+  if (g <= 512)
+    hipLaunchKernelGGL(k_radiance_f64<8>, dim3(g), dim3(8 * WAVE), 8 * RAD64_PT * WAVE * sizeof(double2), s, M, B, L, E,
+                       info, blk0, nblk, rad, tau);
+  else
+    hipLaunchKernelGGL(k_radiance_f64<1>, dim3(g), dim3(WAVE), 0, s, M, B, L, E, info, blk0, nblk, rad, tau);
 }
 
 }  // namespace jur

@@ -607,3 +607,29 @@ def test_level_grids(gpu, oracle, nlev, up, refrac):
         _cmp(r1, r0, RTOL64, "rad")
         _cmp(t1, t0, RTOL64, "tau", atol=1e-30)
         _cmp(abi.np_view(og.tpz)[:o.nr], abi.np_view(oc.tpz)[:o.nr], 1e-11, "tpz", atol=1e-9)
+
+
+@pytest.mark.parametrize("nr", [1, 63, 65])
+def test_radiance_waves_per_path_agree(gpu, nr):
+    """A small batch forms a path's segments on several waves (16 or 8 per
+    path), a large one on one: the same bits for one package of 1, 63 or 65
+    rays (a block with one lane, one short, two blocks) and for it among
+    copies of itself that fill more blocks than the small launches take."""
+    ctl = scenes.limb_3gas_ctl()
+    ctl.sftype = 2
+    atm = scenes.make_profile_atm(["CO2", "H2O", "O3"], iprof=2)
+    geom = scenes.limb_geometry(800.0, np.linspace(-5.0, 60.0, nr) if nr > 1 else np.array([11.0]))
+    n = -(-5000 // nr) if nr > 1 else 5000
+    for prec in (abi.JUR_FP64, abi.JUR_FP32):
+        one = scenes.make_obs(geom)
+        gpu.formod(ctl, abi.copy_struct(atm), one, prec)
+        atms, obss = (abi.atm_t * n)(), (abi.obs_t * n)()
+        for k in range(n):
+            atms[k] = atm
+            obss[k] = scenes.make_obs(geom)
+        gpu.formod_batch(ctl, atms, obss, prec)
+        r0, t0 = abi.obs_arrays(one, ctl)
+        assert np.isfinite(r0).all() and (r0 > 0).any()
+        for k in (0, n // 2, n - 1):
+            r1, t1 = abi.obs_arrays(obss[k], ctl)
+            assert np.array_equal(r0, r1) and np.array_equal(t0, t1), (prec, k)
