@@ -31,15 +31,13 @@ __device__ __forceinline__ int atm_level(const atm_t *atm, int anp, int zdir, do
 // the ray stays between the same levels gives bit-identical values.
 struct LevelCache {
   int ip = -1;
-  double z0 = 0, z1 = 0, p0 = 0, pq = 0, t0 = 0, tq = 0;
+  // the altitudes [lo, hi) for which a walk from this pair returns it: its
+  // levels', open at the ends of the grid; empty for a grid that is not
+  // strictly monotone (search by bisection)
+  double lo = 1, hi = 0;
+  double z0 = 0, dz = 0, p0 = 0, pq = 0, t0 = 0, tq = 0;
   bool plog = false;
-  // the walk from this pair returns it for z
-  __device__ __forceinline__ bool holds(int anp, int zdir, double z) const {
-    if (ip < 0) return false;
-    if (zdir > 0) return (ip == 0 || !(z0 > z)) && (ip == anp - 2 || z1 > z);
-    if (zdir < 0) return (ip == 0 || !(z0 <= z)) && (ip == anp - 2 || z1 <= z);
-    return false;
-  }
+  __device__ __forceinline__ bool holds(double z) const { return lo <= z && z < hi; }
   __device__ __forceinline__ void enter(const atm_t *atm, int anp, int zdir, double z) {
     JUR_FP_EXACT
     int g = ip;
@@ -48,17 +46,24 @@ struct LevelCache {
     ip = l;
     const double x0 = atm->z[l], x1 = atm->z[l + 1];
     const double y0 = atm->p[l], y1 = atm->p[l + 1];
+    if (zdir != 0) {
+      lo = l == (zdir > 0 ? 0 : anp - 2) ? -INFINITY : (zdir > 0 ? x0 : x1);
+      hi = l == (zdir > 0 ? anp - 2 : 0) ? INFINITY : (zdir > 0 ? x1 : x0);
+    }
     z0 = x0;
-    z1 = x1;
+    dz = x1 - x0;
     p0 = y0;
     plog = (y1 / y0 > 0);
-    pq = plog ? log(y1 / y0) / (x1 - x0) : (y1 - y0) / (x1 - x0);
+    pq = plog ? log(y1 / y0) / dz : (y1 - y0) / dz;
     t0 = atm->t[l];
-    tq = (atm->t[l + 1] - t0) / (x1 - x0);
+    tq = (atm->t[l + 1] - t0) / dz;
   }
   __device__ __forceinline__ double p(double z) const {
     JUR_FP_EXACT
-    return plog ? p0 * exp(pq * (z - z0)) : p0 + pq * (z - z0);
+    // (the exponential is taken in either case: without the branch the
+    // evaluations at several altitudes overlap)
+    const double x = pq * (z - z0), e = exp(plog ? x : 0);
+    return plog ? p0 * e : p0 + x;
   }
   __device__ __forceinline__ double t(double z) const {
     JUR_FP_EXACT
@@ -233,15 +238,15 @@ __global__ __launch_bounds__(WAVE) void k_raytrace(ModelView M, BatchView B, Los
   // same x gives the values the reference stores per point.  (A NaN altitude
   // never leaves the range, so its ray ends at the capacity below and has no
   // tangent point.)
-  double zprev = 0, xprev[3] = {0, 0, 0}, xfirst[3] = {0, 0, 0}, xb[3] = {0, 0, 0}, xa[3] = {0, 0, 0};
+  double zprev = 0, xprev[3] = {0, 0, 0}, xb[3] = {0, 0, 0}, xa[3] = {0, 0, 0};
   double zlow = 0, ds_imin = 0, ds_imin1 = 0;
   int imin = 0;
   bool after_pending = false;
-  double dscut = 0;
   double ds1 = 0, ds2 = 0;  // raw step lengths of the last two points written
   // the level pairs of the point and of its midpoint probes: a point mostly
   // enters the pair that the probes before it were in
   LevelCache lp, lc;
+  const double xfirst[3] = {x[0], x[1], x[2]};
   // the lane's probe (RL = 4): the displacements by h along the axes before
   // its own are made and undone as in the serial order below, x + hp - hm
   const int sub = RL == 1 ? 0 : lane % RL;
@@ -249,8 +254,9 @@ __global__ __launch_bounds__(WAVE) void k_raytrace(ModelView M, BatchView B, Los
   const double hm[3] = {sub >= 2 ? h : 0.0, sub >= 3 ? h : 0.0, 0.0};
   double *w = base;
   const size_t wstep = (size_t)L.nfield * WAVE;
+  double ds;
   for (;;) {
-    double ds = M.rayds;
+    ds = M.rayds;
     const double radius = sqrt_mid(x[0] * x[0] + x[1] * x[1] + x[2] * x[2]);
     if (M.raydz > 0) {
       const double rn = div_mid(1, radius);
@@ -261,24 +267,7 @@ __global__ __launch_bounds__(WAVE) void k_raytrace(ModelView M, BatchView B, Los
 
     z = radius - JUR_RE;  // the z output of cart2geo
 
-    if (z < zmin || z > zmax) {
-      // The step left the altitude range: k_ray_finish clips it to the
-      // range and writes the last point (its cart2geo/geo2cart would hold
-      // registers for the whole march here).  With no point written yet
-      // the entry search ended outside the range, so there is no previous
-      // point to clip to (the reference would read los->z[-1]): the ray has
-      // no LOS points.
-      dscut = ds;
-      break;
-    }
-
-    if (np >= L.cap) {
-      // capacity exceeded: the reference limit NLOS -> error, a smaller
-      // working capacity -> the host retries with NLOS
-      R.status = (L.cap >= NLOS) ? JUR_ERR_LOS : 100;
-      if (wr) info[ir] = R;
-      return;
-    }
+    if (z < zmin || z > zmax || np >= L.cap) break;
     // the trapezoid segment length of the point (src/jurassic.c:4410-4411)
     // from its raw step length ds and the previous point's: 0.5 (ds_prev +
     // ds), the first point 0.5 ds (the clip of the last step changes the last
@@ -308,71 +297,69 @@ __global__ __launch_bounds__(WAVE) void k_raytrace(ModelView M, BatchView B, Los
     }
     ds2 = ds1;
     ds1 = ds;
-    if (np == 0)
-      for (int i = 0; i < 3; i++) xfirst[i] = x[i];
     for (int i = 0; i < 3; i++) xprev[i] = x[i];
     zprev = z;
     np++;
 
-    const bool bend = M.refrac && z <= zrefrac;
-    if (bend) {
-      if (!lp.holds(anp, zdir, z)) {
-        if (lc.holds(anp, zdir, z)) lp = lc;
-        else lp.enter(atm, anp, zdir, z);
-      }
-      n = 1 + div_mid(7.753e-05 * lp.p(z), lp.t(z));
-    } else
-      n = 1;
-
-    for (int i = 0; i < 3; i++) ex1[i] = ex0[i] * n;
-
-    if (bend) {
+    if (M.refrac && z <= zrefrac) {
+      // the refractivity at the point, and at the midpoint and the three
+      // probes displaced by h along each axis, in the reference's order (each
+      // displacement is undone by subtracting h before the next axis moves);
+      // with RL = 4 each lane has its own probe.  The level pairs come first,
+      // so that the evaluations overlap.
+      constexpr int NQ = RL == 4 ? 1 : 4;
+      double zq[NQ], rq[NQ];
       for (int i = 0; i < 3; i++) xh[i] = x[i] + 0.5 * ds * ex0[i];
       if constexpr (RL == 4) {
-        // lane sub's probe: the midpoint (0) or the midpoint displaced by h
-        // along axis sub - 1
         for (int i = 0; i < 3; i++) xh[i] = xh[i] + hp[i] - hm[i];
-        const double zq = cart2z(xh);
-        if (!lc.holds(anp, zdir, zq)) lc.enter(atm, anp, zdir, zq);
-        const double rq = div_mid(7.753e-05 * lc.p(zq), lc.t(zq));
-        n = quad_lane<0>(rq);
-        ngr[0] = (quad_lane<1>(rq) - n) * (1 / h);
-        ngr[1] = (quad_lane<2>(rq) - n) * (1 / h);
-        ngr[2] = (quad_lane<3>(rq) - n) * (1 / h);
+        zq[0] = cart2z(xh);
       } else {
-        // the refractivity at the midpoint and at the three probes displaced
-        // by h along each axis, in the reference's order (each displacement
-        // is undone by subtracting h before the next axis moves)
-        double zq[4], rq[4];
         zq[0] = cart2z(xh);
         for (int i = 0; i < 3; i++) {
           xh[i] += h;
           zq[i + 1] = cart2z(xh);
           xh[i] -= h;
         }
-        // all four in the cached pair: side by side; otherwise probe by probe
-        // (not unrolled)
-        bool all = true;
-        for (int k = 0; k < 4; k++) all = all && lc.holds(anp, zdir, zq[k]);
-        if (all) {
-          for (int k = 0; k < 4; k++) rq[k] = div_mid(7.753e-05 * lc.p(zq[k]), lc.t(zq[k]));
-        } else {
-#pragma unroll 1
-          for (int k = 0; k < 4; k++) {
-            const double zk = k == 0 ? zq[0] : (k == 1 ? zq[1] : (k == 2 ? zq[2] : zq[3]));
-            if (!lc.holds(anp, zdir, zk)) lc.enter(atm, anp, zdir, zk);
-            const double v = div_mid(7.753e-05 * lc.p(zk), lc.t(zk));
-            rq[0] = k == 0 ? v : rq[0];
-            rq[1] = k == 1 ? v : rq[1];
-            rq[2] = k == 2 ? v : rq[2];
-            rq[3] = k == 3 ? v : rq[3];
-          }
-        }
-        n = rq[0];
-        for (int i = 0; i < 3; i++) ngr[i] = (rq[i + 1] - n) * (1 / h);
       }
-    } else
-      for (int i = 0; i < 3; i++) ngr[i] = 0;
+      bool all = true;  // the probes are in their cached pair
+      for (int k = 0; k < NQ; k++) all &= lc.holds(zq[k]);
+      if (!lp.holds(z)) {
+        if (lc.holds(z)) lp = lc;
+        else lp.enter(atm, anp, zdir, z);
+      }
+      if (RL == 4 && !all) lc.enter(atm, anp, zdir, zq[0]);
+      if (RL == 4 || all) {
+        for (int k = 0; k < NQ; k++) rq[k] = div_mid(7.753e-05 * lc.p(zq[k]), lc.t(zq[k]));
+      } else {
+        // probe by probe (not unrolled)
+#pragma unroll 1
+        for (int k = 0; k < NQ; k++) {
+          const double zk = k == 0 ? zq[0] : (k == 1 ? zq[1 % NQ] : (k == 2 ? zq[2 % NQ] : zq[3 % NQ]));
+          if (!lc.holds(zk)) lc.enter(atm, anp, zdir, zk);
+          const double v = div_mid(7.753e-05 * lc.p(zk), lc.t(zk));
+          rq[0] = k == 0 ? v : rq[0];
+          rq[1 % NQ] = k == 1 ? v : rq[1 % NQ];
+          rq[2 % NQ] = k == 2 ? v : rq[2 % NQ];
+          rq[3 % NQ] = k == 3 ? v : rq[3 % NQ];
+        }
+      }
+      n = 1 + div_mid(7.753e-05 * lp.p(z), lp.t(z));
+      for (int i = 0; i < 3; i++) ex1[i] = ex0[i] * n;
+      if constexpr (RL == 4) {
+        n = quad_lane<0>(rq[0]);
+        ngr[0] = (quad_lane<1>(rq[0]) - n) * (1 / h);
+        ngr[1] = (quad_lane<2>(rq[0]) - n) * (1 / h);
+        ngr[2] = (quad_lane<3>(rq[0]) - n) * (1 / h);
+      } else {
+        n = rq[0];
+        for (int i = 0; i < 3; i++) ngr[i] = (rq[(i + 1) % NQ] - n) * (1 / h);
+      }
+    } else {
+      for (int i = 0; i < 3; i++) {
+        ex1[i] = ex0[i];
+        ngr[i] = 0;
+      }
+    }
 
     for (int i = 0; i < 3; i++) ex1[i] += ds * ngr[i];
     const double rn1 = div_mid(1, sqrt_mid(ex1[0] * ex1[0] + ex1[1] * ex1[1] + ex1[2] * ex1[2]));
@@ -380,8 +367,20 @@ __global__ __launch_bounds__(WAVE) void k_raytrace(ModelView M, BatchView B, Los
     for (int i = 0; i < 3; i++) x[i] += 0.5 * ds * (ex0[i] + ex1[i]);
     for (int i = 0; i < 3; i++) ex0[i] = ex1[i];
   }
-  R.np = np;
   if (!wr) return;
+  if (!(z < zmin || z > zmax)) {
+    // capacity exceeded: the reference limit NLOS -> error, a smaller
+    // working capacity -> the host retries with NLOS
+    R.status = (L.cap >= NLOS) ? JUR_ERR_LOS : 100;
+    info[ir] = R;
+    return;
+  }
+  // The last step left the altitude range: k_ray_finish clips it to the range
+  // and writes the last point (its cart2geo/geo2cart would hold registers for
+  // the whole march here).  With no point written the entry search ended
+  // outside the range, so there is no previous point to clip to (the reference
+  // would read los->z[-1]): the ray has no LOS points.
+  R.np = np;
   RayTail *tl = tail + ir;
   if (np > 0) {
     for (int i = 0; i < 3; i++) {
@@ -394,7 +393,7 @@ __global__ __launch_bounds__(WAVE) void k_raytrace(ModelView M, BatchView B, Los
     }
     tl->zprev = zprev;
     tl->zcut = z;
-    tl->dscut = dscut;
+    tl->dscut = ds;
     tl->zmin = zmin;
     tl->zmax = zmax;
     tl->ds1 = ds1;
@@ -604,12 +603,12 @@ __global__ __launch_bounds__(WAVE) void k_ray_points(ModelView M, BatchView B, L
   for (int ip = i0; ip < i1; ip++) {
     const int ipn = ip + 1 < i1 ? ip + 1 : ip;
     const double zn = LOSW(F_Z, ipn), dsn = LOSW(F_DS, ipn);
-    if (!lc.holds(anp, zdir, z)) {
+    if (!lc.holds(z)) {
       const int old = lc.ip;
       lc.enter(atm, anp, zdir, z);
       const int l = lc.ip;
       if (l != old) {
-        const double dx = lc.z1 - lc.z0;
+        const double dx = lc.dz;
         for (int ig = 0; ig < M.ng; ig++) {
           const double q0 = atm->q[ig][l];
           LV(ig) = q0;
