@@ -24,6 +24,12 @@ __device__ __forceinline__ int atm_level(const atm_t *atm, int anp, int zdir, do
   return g;
 }
 
+// A level (index ip) loaded ahead.
+struct LevelAhead {
+  int ip = -1;
+  double z = 0, p = 0, t = 0;
+};
+
 // Pressure and temperature interpolation of intpol_atm
 // (src/jurassic.c:3685-3706) with the level-pair coefficients cached: LOGY
 // evaluates y0 exp(log(y1/y0)/(x1-x0) (x-x0)) and LIN y0 + (y1-y0)/(x1-x0)
@@ -37,26 +43,61 @@ struct LevelCache {
   double lo = 1, hi = 0;
   double z0 = 0, dz = 0, p0 = 0, pq = 0, t0 = 0, tq = 0;
   bool plog = false;
+  double z1 = 0, p1 = 0, t1 = 0;
   __device__ __forceinline__ bool holds(double z) const { return lo <= z && z < hi; }
-  __device__ __forceinline__ void enter(const atm_t *atm, int anp, int zdir, double z) {
+  __device__ __forceinline__ void range(int anp, int zdir) {
+    lo = ip == (zdir > 0 ? 0 : anp - 2) ? -INFINITY : (zdir > 0 ? z0 : z1);
+    hi = ip == (zdir > 0 ? anp - 2 : 0) ? INFINITY : (zdir > 0 ? z1 : z0);
+  }
+  // To the pair of z, not held by this one.  A path leaves a pair into its
+  // neighbour: that takes one level, loaded ahead when the pair before was
+  // entered (a search reads a level at a time, each a round trip to memory
+  // behind the march's stores).
+  __device__ __forceinline__ void enter(const atm_t *atm, int anp, int zdir, double z, LevelAhead &ah) {
     JUR_FP_EXACT
-    int g = ip;
-    const int l = atm_level(atm, anp, zdir, z, g);
-    if (l == ip) return;
-    ip = l;
-    const double x0 = atm->z[l], x1 = atm->z[l + 1];
-    const double y0 = atm->p[l], y1 = atm->p[l + 1];
-    if (zdir != 0) {
-      lo = l == (zdir > 0 ? 0 : anp - 2) ? -INFINITY : (zdir > 0 ? x0 : x1);
-      hi = l == (zdir > 0 ? anp - 2 : 0) ? INFINITY : (zdir > 0 ? x1 : x0);
+    bool found = false, up = false;
+    if (ip >= 0 && zdir != 0) {
+      up = (z >= hi) == (zdir > 0);
+      const int f = up ? ip + 2 : ip - 1;
+      if (f >= 0 && f < anp) {
+        double zf = ah.z, pf = ah.p, tf = ah.t;
+        if (ah.ip != f) {
+          zf = atm->z[f];
+          pf = atm->p[f];
+          tf = atm->t[f];
+        }
+        ip = up ? ip + 1 : ip - 1;
+        const double zs = up ? z1 : z0, ps = up ? p1 : p0, ts = up ? t1 : t0;
+        z0 = up ? zs : zf;
+        p0 = up ? ps : pf;
+        t0 = up ? ts : tf;
+        z1 = up ? zf : zs;
+        p1 = up ? pf : ps;
+        t1 = up ? tf : ts;
+        range(anp, zdir);
+        found = holds(z);
+      }
     }
-    z0 = x0;
-    dz = x1 - x0;
-    p0 = y0;
-    plog = (y1 / y0 > 0);
-    pq = plog ? log(y1 / y0) / dz : (y1 - y0) / dz;
-    t0 = atm->t[l];
-    tq = (atm->t[l + 1] - t0) / dz;
+    if (!found) {
+      int g = ip;
+      ip = atm_level(atm, anp, zdir, z, g);
+      z0 = atm->z[ip];
+      z1 = atm->z[ip + 1];
+      p0 = atm->p[ip];
+      p1 = atm->p[ip + 1];
+      t0 = atm->t[ip];
+      t1 = atm->t[ip + 1];
+      if (zdir != 0) range(anp, zdir);
+    }
+    const int f = up ? ip + 2 : ip - 1;
+    ah.ip = f >= 0 && f < anp ? f : ip;
+    ah.z = atm->z[ah.ip];
+    ah.p = atm->p[ah.ip];
+    ah.t = atm->t[ah.ip];
+    dz = z1 - z0;
+    plog = (p1 / p0 > 0);
+    pq = plog ? log(p1 / p0) / dz : (p1 - p0) / dz;
+    tq = (t1 - t0) / dz;
   }
   __device__ __forceinline__ double p(double z) const {
     JUR_FP_EXACT
@@ -246,6 +287,7 @@ __global__ __launch_bounds__(WAVE) void k_raytrace(ModelView M, BatchView B, Los
   // the level pairs of the point and of its midpoint probes: a point mostly
   // enters the pair that the probes before it were in
   LevelCache lp, lc;
+  LevelAhead ahead;
   const double xfirst[3] = {x[0], x[1], x[2]};
   // the lane's probe (RL = 4): the displacements by h along the axes before
   // its own are made and undone as in the serial order below, x + hp - hm
@@ -325,9 +367,9 @@ __global__ __launch_bounds__(WAVE) void k_raytrace(ModelView M, BatchView B, Los
       for (int k = 0; k < NQ; k++) all &= lc.holds(zq[k]);
       if (!lp.holds(z)) {
         if (lc.holds(z)) lp = lc;
-        else lp.enter(atm, anp, zdir, z);
+        else lp.enter(atm, anp, zdir, z, ahead);
       }
-      if (RL == 4 && !all) lc.enter(atm, anp, zdir, zq[0]);
+      if (RL == 4 && !all) lc.enter(atm, anp, zdir, zq[0], ahead);
       if (RL == 4 || all) {
         for (int k = 0; k < NQ; k++) rq[k] = div_mid(7.753e-05 * lc.p(zq[k]), lc.t(zq[k]));
       } else {
@@ -335,7 +377,7 @@ __global__ __launch_bounds__(WAVE) void k_raytrace(ModelView M, BatchView B, Los
 #pragma unroll 1
         for (int k = 0; k < NQ; k++) {
           const double zk = k == 0 ? zq[0] : (k == 1 ? zq[1 % NQ] : (k == 2 ? zq[2 % NQ] : zq[3 % NQ]));
-          if (!lc.holds(zk)) lc.enter(atm, anp, zdir, zk);
+          if (!lc.holds(zk)) lc.enter(atm, anp, zdir, zk, ahead);
           const double v = div_mid(7.753e-05 * lc.p(zk), lc.t(zk));
           rq[0] = k == 0 ? v : rq[0];
           rq[1 % NQ] = k == 1 ? v : rq[1 % NQ];
@@ -446,7 +488,8 @@ __global__ __launch_bounds__(WAVE) void k_ray_finish(ModelView M, BatchView B, L
   }
   // the temperature at the clipped point (intpol_atm), for the surface
   LevelCache lc;
-  lc.enter(atm, atm->np, T.zdir, z);
+  LevelAhead ahead;
+  lc.enter(atm, atm->np, T.zdir, z, ahead);
   double t = lc.t(z);
   // trapezoid segment lengths (src/jurassic.c:4410-4411) of the last point
   // written, from its clipped raw length, and of this one (raw length 0);
@@ -557,6 +600,7 @@ __global__ __launch_bounds__(WAVE) void k_ray_points(ModelView M, BatchView B, L
   extern __shared__ double lvl[];
 #define LV(f) lvl[(f) * WAVE + lane]
   LevelCache lc;
+  LevelAhead ahead;
   // the tables' cell of a point (LosView::cell): the pressure bracket and,
   // on its two pressures, the temperature brackets and weights, with the
   // arithmetic of the FP32 lookups (float, reciprocal spacings)
@@ -605,7 +649,7 @@ __global__ __launch_bounds__(WAVE) void k_ray_points(ModelView M, BatchView B, L
     const double zn = LOSW(F_Z, ipn), dsn = LOSW(F_DS, ipn);
     if (!lc.holds(z)) {
       const int old = lc.ip;
-      lc.enter(atm, anp, zdir, z);
+      lc.enter(atm, anp, zdir, z, ahead);
       const int l = lc.ip;
       if (l != old) {
         const double dx = lc.dz;
