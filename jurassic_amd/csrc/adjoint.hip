@@ -504,6 +504,14 @@ __device__ __forceinline__ int level_of(const atm_t *atm, double z, int lev, dou
   return lev;
 }
 
+// A product as rounded, kept out of the multiply-adds it would be contracted
+// into: the row kernel hands the segment transmittance from wave to wave, and
+// the large batches' kernel gives the same radiances.
+__device__ __forceinline__ double rounded(double v) {
+  asm("" : "+v"(v));
+  return v;
+}
+
 // Sums of point adjoints of the current level pair (wa, wa+1) for NQ level
 // quantities (JUR_XMAP_LEV quantity index qi[q], -1 = none); flushed into the
 // lane's tile row when the pair changes.
@@ -1105,10 +1113,7 @@ __device__ __forceinline__ void point_forms(const double *e, double f, double c[
   }
 }
 
-// LM (lane-major, for the small-batch sweep that stages each lane's step in
-// LDS): step k of lane l at ((k 64 + l) JUR_NPCO + f); otherwise
-// coefficient-major, (k JUR_NPCO + f) 64 + l.
-template <bool LM>
+// Coefficient f of step k of lane l at (k JUR_NPCO + f) 64 + l.
 __global__ __launch_bounds__(WAVE) void k_path_coef(ModelView M, BatchView B, LosView L, const RayInfo *info,
                                                     int blk0, int nblk, int nchunk, JacView J) {
   int bl, chk;
@@ -1123,7 +1128,7 @@ __global__ __launch_bounds__(WAVE) void k_path_coef(ModelView M, BatchView B, Lo
   if (k0 >= k1) return;
   const atm_t *atm = &B.atm[B.ray_prof[ir]];
   const double *los = L.los + (size_t)bl * L.cap * L.nfield * WAVE + lane;
-  double *pc = J.pco + J.soff[bl] / ((size_t)M.nd * J.nscr) * JUR_NPCO + (LM ? (size_t)lane * JUR_NPCO : lane);
+  double *pc = J.pco + J.soff[bl] / ((size_t)M.nd * J.nscr) * JUR_NPCO + lane;
   int hint = -1;
   for (int k = k0; k < k1; k++) {
     double x[3], e[3];
@@ -1134,7 +1139,7 @@ __global__ __launch_bounds__(WAVE) void k_path_coef(ModelView M, BatchView B, Lo
     MarchStep S;
     march_step(M, atm, x, e, hint, S);
     double *o = pc + (size_t)k * JUR_NPCO * WAVE;
-#define PCW(f, v) o[LM ? (size_t)(f) : (size_t)(f) * WAVE] = (v)
+#define PCW(f, v) o[(size_t)(f) * WAVE] = (v)
     PCW(PC_HDS, 0.5 * S.ds);
     PCW(PC_RNV, 1 / S.nv);
     PCW(PC_N, S.n);
@@ -1237,7 +1242,8 @@ __global__ __launch_bounds__(WAVE) void k_path_coef(ModelView M, BatchView B, Lo
 // of the state, the level window, and the clip of the last step.  Level sums
 // are kept for a window of three levels (the step's LB and the two above)
 // per channel and added to the K tile when the window moves.
-template <int CH>
+// ATOM: atomic adds, where another wave adds to the same tile row meanwhile.
+template <int CH, bool ATOM = false>
 struct PathRev {
   const int *xm;
   int nlev, nc;
@@ -1291,6 +1297,11 @@ struct PathRev {
     }
   }
 
+  static __device__ __forceinline__ void tile_add(double *kt, int col, double v) {
+    if (ATOM) unsafeAtomicAdd(&kt[(size_t)col * WAVE], v);
+    else kt[(size_t)col * WAVE] += v;
+  }
+
   __device__ __forceinline__ void flush_level(int j) {
     const int l = wb + j;
     if (l >= nlev) return;
@@ -1299,19 +1310,18 @@ struct PathRev {
     for (int c = 0; c < CH; c++) {
       if (c >= nc) continue;
       double *kt = kt0 + (size_t)c * ktstride;
-      if (ct >= 0) kt[(size_t)ct * WAVE] += Tw[c][j];
-      if (cp >= 0) kt[(size_t)cp * WAVE] += Pw[c][j];
+      if (ct >= 0) tile_add(kt, ct, Tw[c][j]);
+      if (cp >= 0) tile_add(kt, cp, Pw[c][j]);
     }
   }
 
   // The reverse of march step k (of N points) with its coefficients cf and
   // the channels' point values gz = d rad / d z_k, gd = d rad / d ds_k.
-  // LAY 0: coefficient f at cf[f]; LAY 1 (a lane's coefficients staged in
-  // LDS by 16 B direct-to-LDS loads, pair i at i KiB + lane 16 B): at
-  // cf[(f / 2) 128 + f % 2] with cf at the lane's first pair.
+  // LAY 0: coefficient f at cf[f]; LAY 1 (a step's block staged in LDS,
+  // coefficient-major): at cf[64 f] with cf at the lane's first.
   template <int LAY = 0>
   __device__ __forceinline__ void step(int k, int N, const double *cf, const double *gzv, const double *gdv) {
-#define PCR(f) (LAY == 0 ? cf[f] : cf[((f) >> 1) * 128 + ((f) & 1)])
+#define PCR(f) (LAY == 0 ? cf[f] : cf[(f) * WAVE])
     const double hds = PCR(PC_HDS), rnv = PCR(PC_RNV), n = PCR(PC_N), sk = PCR(PC_SK);
     double e[3], e1[3], ngm[3], xh[3], a[3], b[3], mx[9];
 #pragma unroll
@@ -1410,10 +1420,10 @@ struct PathRev {
           const double g = q == 0 ? e[0] * V[c][0] + e[1] * V[c][1] + e[2] * V[c][2]
                                   : (q == 1 ? -f * (V[c][0] + V[c][1] + V[c][2]) : f * V[c][q >= 2 ? q - 2 : 0]);
           double *kt = kt0 + (size_t)c * ktstride;
-          if (t0 >= 0) kt[(size_t)t0 * WAVE] += g * w0;
-          if (t1 >= 0) kt[(size_t)t1 * WAVE] += g * w1;
-          if (p0 >= 0) kt[(size_t)p0 * WAVE] += g * w2;
-          if (p1 >= 0) kt[(size_t)p1 * WAVE] += g * w3;
+          if (t0 >= 0) tile_add(kt, t0, g * w0);
+          if (t1 >= 0) tile_add(kt, t1, g * w1);
+          if (p0 >= 0) tile_add(kt, p0, g * w2);
+          if (p1 >= 0) tile_add(kt, p1, g * w3);
         }
       }
     }
@@ -1428,7 +1438,7 @@ struct PathRev {
     for (int c = 0; c < CH; c++)
       for (int i = 0; i < 3; i++) {
         const int f = PC_XH + i;
-        X[c][i] += Xp[c][i] + gzp[c] * (LAY == 0 ? cf[f] : cf[(f >> 1) * 128 + (f & 1)]);
+        X[c][i] += Xp[c][i] + gzp[c] * (LAY == 0 ? cf[f] : cf[f * WAVE]);
       }
   }
 
@@ -1449,15 +1459,7 @@ struct PathStepIn {
 // rad, tau, H_i (scratch), the number of points before the first opaque
 // segment, and the K entries of continua, source function, window
 // extinction, clouds and surface.
-// EMF > 0 (FP32 EGA with stored partials, ng <= EMF): the reverse sweep also
-// runs the emitter chains of the row, point by point, as k_adj_chains_f32
-// does; H_i is used where it is formed, and the chains' T, p and q adjoints
-// join the accumulation's in one level window.  PFU (with PATH): it also
-// runs the reverse march of the refracted path (PathRev, one channel) point
-// by point from the stored step coefficients, so that the row's whole
-// reverse sweep is one pass over the path: the form for small batches,
-// where each kernel lasts as long as one wavefront's sweep.
-template <typename SF, bool PATH, int EMF = 0, bool PFU = false>
+template <typename SF, bool PATH>
 __global__ __launch_bounds__(WAVE) void k_adj_acc(ModelView M, BatchView B, LosView L, EpsView E,
                                                   const RayInfo *info, const RayTail *tail, int blk0, int nblk,
                                                   JacView J, double *rad_out, double *tau_out) {
@@ -1526,7 +1528,7 @@ __global__ __launch_bounds__(WAVE) void k_adj_acc(ModelView M, BatchView B, LosV
       rp = rcp_d(p);
       beta = beta_grad_f(M, K, KF, nu, p, t, rt, rp, rcp_d(ds), q_h2o, u_co2, u_h2o, kwin, clx, bg);
       src = srcfunc_du(M.st, inv_dst, sr_col, t, dsrc);
-      return tg * (double)__expf((float)(-beta * ds));
+      return rounded(tg * (double)__expf((float)(-beta * ds)));
     } else {
       rt = 1 / t;
       rp = 1 / p;
@@ -1642,94 +1644,18 @@ __global__ __launch_bounds__(WAVE) void k_adj_acc(ModelView M, BatchView B, LosV
   // H_i replaces tau_i in the scratch; continua, source function, window
   // extinction and clouds contribute here, the emitter chains below.
   double clz_bar = 0, cldz_bar = 0, clk_bar = 0;
-  // the surface temperature taken from the last LOS point's T: its slope
-  // moves d rad / d z of that point (added here where the path adjoint runs
-  // in this sweep, after the sweep otherwise)
-  double gz_sft = 0;
-  if (PFU && M.sftype >= 1 && R.sft > 0 && !(M.nsf > 0 && atm->sft > 0) && R.np > 0 && R.np - 1 < nef) {
-    double w;
-    const int lv = level_of(atm, LOSR(F_Z, R.np - 1), -1, w);
-    gz_sft = sft_bar * (atm->t[lv + 1] - atm->t[lv]) / (atm->z[lv + 1] - atm->z[lv]);
-  }
   {
-    // level quantities: T, p, the window's extinction, then CO2 and H2O, or
-    // with the chains every emitter's q
-    constexpr int NQW = EMF > 0 ? 3 + EMF : 5;
-    int qi[NQW];
-    qi[0] = 1;
-    qi[1] = 0;
-    qi[2] = has_k ? 2 + NG + C.window : -1;
-    if constexpr (EMF > 0) {
-#pragma unroll
-      for (int g = 0; g < EMF; g++) qi[3 + g] = g < ng ? 2 + g : -1;
-    } else {
-      qi[3] = M.ig_co2 >= 0 ? 2 + M.ig_co2 : -1;
-      qi[4] = M.ig_h2o >= 0 ? 2 + M.ig_h2o : -1;
-    }
+    // level quantities: T, p, the window's extinction, CO2 and H2O
+    constexpr int NQW = 5;
+    const int qi[NQW] = {1, 0, has_k ? 2 + NG + C.window : -1, M.ig_co2 >= 0 ? 2 + M.ig_co2 : -1,
+                         M.ig_h2o >= 0 ? 2 + M.ig_h2o : -1};
     LevelWindow<NQW, (1u << NQW) - 1u, F32, PATH> W;
     // the path adjoint's point values d rad / d z_i, d rad / d ds_i: zero
     // beyond the first opaque segment, the emitter chains add theirs
-    if (PATH && !PFU)
+    if (PATH)
       for (int ip = nef; ip < R.np; ip++) SCR(J.kz, ip) = SCR(J.kz + 1, ip) = 0.0;
     int lev = -1;
     double qi_cur = nef > 0 ? qprod(nef - 1) : 1;
-    // the chains' state: Lambda carry, the path transmittance after the
-    // point (as the float the chain divides by), the point's stored partials
-    // (dep, dp, dT, du) and column density, loaded one point ahead
-    constexpr int EC = EMF > 0 ? EMF : 1;
-    bool on[EC];
-    double carry[EC], ucur[EC], unx[EC];
-    float trc[EC];
-    float4 dcur[EC], dnx[EC];
-    const float4 *pab = EMF > 0 ? E.part + E.off[bl] + (size_t)id * ng * npb * WAVE + lane : nullptr;
-#pragma unroll
-    for (int g = 0; g < EC; g++) {
-      on[g] = EMF > 0 && g < ng && (gm >> g & 1u);
-      carry[g] = ucur[g] = unx[g] = 0;
-      trc[g] = (on[g] && nef > 0) ? (float)trans_of(EPS_AT(g, nef - 1)) : 1.f;
-      dcur[g] = dnx[g] = make_float4(0.f, 0.f, 0.f, 0.f);
-    }
-    double Hn = 0;
-    // the path's reverse march (PFU): its state, the held values of the last
-    // point, and the next step's coefficients loaded one point ahead
-    const int N = R.np;
-    PathRev<1> P;
-    bool pstart = false;
-    double gz_last = 0, gd_last = 0;
-    // the next step's coefficients are staged in LDS (one wavefront per
-    // workgroup: 27 KiB), copied by the wavefront's direct-to-LDS loads
-    // while the next point's accumulation runs, instead of in registers
-    const char *pcg = nullptr;
-    double *pcs = nullptr;
-    // (lane-major coefficients: each lane copies its own step's 432 B; the
-    // lanes of a wavefront are at different steps)
-    auto pc_fetch = [&](int k) {
-      if constexpr (PFU) {
-        // the reads of the last step's coefficients have completed before
-        // the copy overwrites them; the memory clobber keeps the compiler
-        // from moving those reads below the copy, whose LDS write it does
-        // not see
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-        const char *g = pcg + ((size_t)k * WAVE + lane) * JUR_NPCO * sizeof(double);
-#pragma unroll
-        for (int i = 0; i < JUR_NPCO / 2; i++)
-          __builtin_amdgcn_global_load_lds((const void *)(g + i * 16),
-                                           (__attribute__((address_space(3))) void *)((char *)pcs + i * 1024),
-                                           16, 0, 0);
-      }
-    };
-    if constexpr (PFU) {
-      __shared__ double pc_lds[JUR_NPCO * WAVE];
-      pcs = pc_lds;
-      P.xm = xm;
-      P.nlev = atm->np;
-      P.nc = 1;
-      P.kt0 = kt;
-      P.ktstride = (size_t)J.ncol * WAVE;
-      pcg = (const char *)(J.pco + J.soff[bl] / ((size_t)nd * J.nscr) * JUR_NPCO);
-      const int k0 = nef - 1 < N - 2 ? nef - 1 : N - 2;
-      if (k0 >= 0) pc_fetch(k0);
-    }
     // point ip's inputs and scratch, and the emitters' values at ip - 1,
     // loaded one iteration ahead
     double sc0n = 0, sc1n = 0;
@@ -1738,27 +1664,12 @@ __global__ __launch_bounds__(WAVE) void k_adj_acc(ModelView M, BatchView B, LosV
       sc0n = SCR(0, ip);
       sc1n = J.nscr > 1 ? SCR(1, ip) : 0.0;
       if (ip > 0) ld_eps(ip - 1);
-      if constexpr (EMF > 0) {
-#pragma unroll
-        for (int g = 0; g < EMF; g++)
-          if (on[g]) {
-            dnx[g] = pab[((size_t)g * npb + ip) * WAVE];
-            unx[g] = LOSR(L.f_u + g, ip);
-          }
-      }
     };
     if (nef > 0) ld_rev(nef - 1);
     for (int ip = nef - 1; ip >= 0; ip--) {
       const PtIn cu = nx;
       const double tau_i = sc0n, dr_i = sc1n;
       const double qm = ip > 0 ? prod_en() : 1;
-      float em1[EC];  // the emitters' path emissivities before point ip
-#pragma unroll
-      for (int g = 0; g < EC; g++) {
-        em1[g] = EMF > 0 ? (float)en[g] : 0.f;
-        dcur[g] = dnx[g];
-        ucur[g] = unx[g];
-      }
       if (ip > 0) ld_rev(ip - 1);
       const double tg = F32 ? qi_cur * rcp_d(qm) : qi_cur / qm;
       qi_cur = qm;
@@ -1776,7 +1687,7 @@ __global__ __launch_bounds__(WAVE) void k_adj_acc(ModelView M, BatchView B, LosV
       tb = src * (1 - s) + tb * s;
       db = db * s;
       const double H = G * s;
-      if (EMF == 0) SCR(0, ip) = H;
+      SCR(0, ip) = H;
       const double beta_bar = -H * ds;
 
       // u = 10 q p / (kB T) ds
@@ -1788,35 +1699,8 @@ __global__ __launch_bounds__(WAVE) void k_adj_acc(ModelView M, BatchView B, LosV
       v[1] = beta_bar * bg.dp + (F32 ? uu * rp : uu / p);                   // p
       v[2] = beta_bar;                                                                  // k
       const double vco2 = uc_bar * ucoef, vh2o = uh_bar * ucoef + beta_bar * bg.dq_h2o;
-      double gu = 0;  // the chains' sum of u_bar u_seg (d rad / d ds_i through u)
-      if constexpr (EMF > 0) {
-        // the chains (as k_adj_chains_f32: float reciprocals of T, p and the
-        // transmittance, whose 1e-7 is far below the FP32 lookups')
-        const double rtf = (double)frcp((float)t), rpf = (double)frcp((float)p);
-        const double ucf = 10 * p * rtf * ds * (1 / JUR_KB);
-        double vt = 0, vp = 0;
-#pragma unroll
-        for (int g = 0; g < EMF; g++) {
-          double vq = (g == M.ig_co2 ? vco2 : 0.0) + (g == M.ig_h2o ? vh2o : 0.0);
-          if (on[g]) {
-            const double lam = (Hn - H) * (double)frcp(trc[g]) + carry[g];
-            const double u_bar = lam * dcur[g].w;
-            carry[g] = lam * dcur[g].x;
-            vt += lam * dcur[g].z - u_bar * ucur[g] * rtf;
-            vp += lam * dcur[g].y + u_bar * ucur[g] * rpf;
-            vq += u_bar * ucf;
-            gu += u_bar * ucur[g];
-            trc[g] = ip > 0 ? (float)(1.0 - (double)em1[g]) : 1.f;
-          }
-          v[3 + g] = vq;
-        }
-        v[0] += vt;
-        v[1] += vp;
-        Hn = H;
-      } else {
-        v[3] = vco2;  // q_co2
-        v[4] = vh2o;  // q_h2o
-      }
+      v[3] = vco2;  // q_co2
+      v[4] = vh2o;  // q_h2o
       const double gz = W.add(atm, z, lev, v, 1, p, xm, qi, kt);
       if (PATH) {
         // altitude: the level quantities' slopes and the cloud profile's;
@@ -1825,36 +1709,8 @@ __global__ __launch_bounds__(WAVE) void k_adj_acc(ModelView M, BatchView B, LosV
         // densities' part comes from the emitter chains
         double gzc = gz;
         if (cloud && atm->cldz > 0) gzc -= beta_bar * kcl * aux * (z - atm->clz) / (atm->cldz * atm->cldz);
-        const double gdc = EMF > 0 ? -H * beta + gu * rcp_d(ds) : -H * beta;
-        if constexpr (PFU) {
-          if (ip == N - 1) {
-            gz_last = gzc + gz_sft;
-            gd_last = gdc;
-          } else {
-            if (!pstart) {
-              // the first step reached: the clip of the last step, with
-              // point N-2's d rad / d ds where this is that point
-              double xl[3];
-              for (int i = 0; i < 3; i++) xl[i] = LOSR(L.f_xe + i, N - 1);
-              const double gdm = ip == N - 2 ? gdc : 0.0;
-              P.init(M, tail[ir], xl, &gz_last, &gd_last, &gdm);
-              pstart = true;
-            }
-            // the copy of this step's coefficients has landed in LDS: the
-            // direct-to-LDS loads count as vector memory loads, which the
-            // compiler does not track for LDS reads (the memory clobber
-            // keeps the reads below the wait)
-            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-            P.template step<1>(ip, N, pcs + 2 * lane, &gzc, &gdc);
-            if (ip == N - 2) P.template join_clip<1>(pcs + 2 * lane);
-            // the next step's coefficients, in flight during the next
-            // point's accumulation
-            if (ip > 0) pc_fetch(ip - 1);
-          }
-        } else {
-          SCR(J.kz, ip) = gzc;
-          SCR(J.kz + 1, ip) = gdc;
-        }
+        SCR(J.kz, ip) = gzc;
+        SCR(J.kz + 1, ip) = -H * beta;
       }
 
       if (cloud) {
@@ -1867,7 +1723,6 @@ __global__ __launch_bounds__(WAVE) void k_adj_acc(ModelView M, BatchView B, LosV
         }
       }
     }
-    if (PFU && pstart) P.finish();
     W.flush(xm, qi, kt);
   }
 
@@ -1883,7 +1738,7 @@ __global__ __launch_bounds__(WAVE) void k_adj_acc(ModelView M, BatchView B, LosV
       int c;
       if ((c = xm[JUR_XMAP_LEV(1, lv)]) >= 0) KT(c) += (1 - w) * sft_bar;
       if ((c = xm[JUR_XMAP_LEV(1, lv + 1)]) >= 0) KT(c) += w * sft_bar;
-      if (PATH && !PFU && R.np - 1 < nef)
+      if (PATH && R.np - 1 < nef)
         SCR(J.kz, R.np - 1) += sft_bar * (atm->t[lv + 1] - atm->t[lv]) / (atm->z[lv + 1] - atm->z[lv]);
     }
     if (M.nsf > 0) {
@@ -1902,6 +1757,469 @@ __global__ __launch_bounds__(WAVE) void k_adj_acc(ModelView M, BatchView B, LosV
 #undef EPS_AT
 #undef SCR
 #undef KT
+}
+
+// A whole row (64 rays, channel) in one workgroup of four waves, for small
+// batches of the FP32 EGA Jacobian, which last as long as one path's sweeps:
+// the work of k_adj_acc, k_adj_chains_f32 and k_adj_path as a pipeline over
+// the points (same formulas).
+//   forward: all four waves form the segments' s and src (they do not depend
+//     on each other), wave 0 the running tau, D and radiance;
+//   reverse, in rounds of ROW_RP points, each stage a round behind the one
+//     before: waves 2 and 3 the segment's terms and gradients, wave 0 the
+//     accumulation's adjoint, the emitter chains and the level sums, wave 1
+//     the reverse march of the refracted path, whose coefficients it copies
+//     into LDS a step ahead.
+// All lanes of the workgroup are at the same point (a lane begins at its own
+// last one), so a step's coefficients are one contiguous copy.  Wave 1 adds
+// to the T and p columns that wave 0 adds to: both add atomically.
+// One wave ran the two sweeps with everything in the reverse one before: 512
+// registers, 1140 vector instructions per point of one wave in series.
+constexpr int ROW_RP = 2;  // points per round: one per producing wave
+constexpr int ROW_TERMS = 8;
+constexpr int ROW_FP = 8;  // points per wave and round of the forward sweep
+
+template <int EM, bool PATH>
+__global__ __launch_bounds__(4 * WAVE, 2) void k_adj_row(ModelView M, BatchView B, LosView L, EpsView E,
+                                                         const RayInfo *info, const RayTail *tail, int blk0, int nblk,
+                                                         JacView J, double *rad_out, double *tau_out) {
+  const int nd = M.nd, ng = M.ng;
+  int bl, id;
+  if (!xcd_block_map(blockIdx.x, nd, nblk, bl, id)) return;
+  const int lane = threadIdx.x % WAVE;
+  const int role = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+  // lanes without a ray keep the barriers and do nothing
+  const bool live = (blk0 + bl) * WAVE + lane < B.nray;
+  const int ir = live ? (blk0 + bl) * WAVE + lane : B.nray - 1;
+  const RayInfo R = info[ir];
+  const bool ok = live && R.status == JUR_OK;
+  const int N = ok ? R.np : 0;
+  const int ipf = ok ? B.ray_prof[ir] : 0;
+  const int im = ok ? J.prof_map[ipf] : -1;
+  const bool map = im >= 0 && im < J.nmap;  // no state map: the K row stays zero
+  const int *xm = J.xmap + (size_t)(map ? im : 0) * JUR_XMAP_LEN;
+  const atm_t *atm = &B.atm[ipf];
+  const ChanInfo C = M.chan[id];
+  const double nu = C.nu;
+  const double *los = L.los + (size_t)bl * L.cap * L.nfield * WAVE + lane;
+  const int npb = E.npb[bl];
+  const float *epsb = (const float *)E.eps + E.off[bl] + (size_t)id * ng * npb * WAVE + lane;
+  const float4 *pab = E.part + E.off[bl] + (size_t)id * ng * npb * WAVE + lane;
+#define EPS_AT(g, ip) epsb[((size_t)(g) * npb + (ip)) * WAVE]
+  double *sc = J.scr + J.soff[bl] + (size_t)id * npb * J.nscr * WAVE + lane;
+#define SCR(k, ip) sc[((size_t)(ip) * J.nscr + (k)) * WAVE]
+  double *kt = J.kt + ((size_t)bl * nd + id) * J.ncol * WAVE + lane;
+#define KT(col) kt[(size_t)(col) * WAVE]
+  const double *sr_col = M.sr + (size_t)id * TBLNS;
+  const double inv_dst = 1 / (M.st[1] - M.st[0]);
+
+  // LDS: the forward sweep's segments; then the terms [buffer][point][term],
+  // the point values [buffer][point][z, ds] and two steps' coefficients
+  constexpr int N_TERM = 2 * ROW_RP * ROW_TERMS, N_GZ = 2 * ROW_RP * 2, N_PC = PATH ? 2 * JUR_NPCO : 0;
+  constexpr int N_FWD = 4 * ROW_FP * 2;
+  __shared__ double lds[(N_TERM + N_GZ + N_PC > N_FWD ? N_TERM + N_GZ + N_PC : N_FWD) * WAVE];
+  __shared__ int s_nef[WAVE];
+#define LD(i) lds[(i) * WAVE + lane]
+
+  bool on[EM];  // emitters with a table for this channel
+#pragma unroll
+  for (int g = 0; g < EM; g++) on[g] = g < ng && M.tab.np[g * nd + id] >= 30;
+
+  double kcl = 0, wcl = 0;
+  const bool cloud = L.f_cl >= 0 && M.ncl > 0;
+  if (cloud) {
+    const double x0 = M.clnu[C.icl], x1 = M.clnu[C.icl + 1];
+    kcl = lin(x0, atm->clk[C.icl], x1, atm->clk[C.icl + 1], nu);
+    wcl = (nu - x0) / (x1 - x0);
+  }
+  const bool has_k = C.window < M.nw;
+  const CtmChan K = ctm_chan(M.ctm, nu);
+  const CtmChanF KF = ctm_chan_f(K, nu);
+  const bool co2 = M.ig_co2 >= 0, h2o = M.ig_h2o >= 0;
+
+  // Point inputs (absent fields read F_DS in their place and are not used).
+  struct PtIn {
+    double p, t, ds, qh, uc, uh, kw, cl;
+    float e[EM], em[EM];  // the emitters' path emissivities after and before the point
+  };
+  const int f_qh = h2o ? F_Q0 + M.ig_h2o : F_DS, f_uc = co2 ? L.f_u + M.ig_co2 : F_DS;
+  const int f_uh = h2o ? L.f_u + M.ig_h2o : F_DS, f_kw = has_k ? L.f_k + C.window : F_DS;
+  const int f_cl = cloud ? L.f_cl : F_DS;
+  auto ld_pt = [&](int ip) {
+    PtIn x;
+    x.p = LOSR(F_P, ip);
+    x.t = LOSR(F_T, ip);
+    x.ds = LOSR(F_DS, ip);
+    x.qh = LOSR(f_qh, ip);
+    x.uc = LOSR(f_uc, ip);
+    x.uh = LOSR(f_uh, ip);
+    x.kw = LOSR(f_kw, ip);
+    x.cl = LOSR(f_cl, ip);
+#pragma unroll
+    for (int g = 0; g < EM; g++) {
+      x.e[g] = on[g] ? EPS_AT(g, ip) : 0.f;
+      x.em[g] = on[g] && ip > 0 ? EPS_AT(g, ip - 1) : 0.f;
+    }
+    return x;
+  };
+  auto qprod = [&](const float *e) {
+    double q = 1;
+#pragma unroll
+    for (int g = 0; g < EM; g++)
+      if (on[g]) q *= trans_of(e[g]);
+    return q;
+  };
+  // a segment's terms (as k_adj_acc's in FP32); q: its gas transmittance's
+  // numerator, qprod(x.e) > 0
+  struct Seg {
+    double s, src, dsrc, rt, rp, beta;
+    BetaGrad bg;
+  };
+  auto segment = [&](const PtIn &x, double q) {
+    Seg v;
+    const double tg = q * rcp_d(qprod(x.em));
+    v.rt = rcp_d(x.t);
+    v.rp = rcp_d(x.p);
+    v.beta = beta_grad_f(M, K, KF, nu, x.p, x.t, v.rt, v.rp, rcp_d(x.ds), h2o ? x.qh : 0.0, co2 ? x.uc : 0.0,
+                         h2o ? x.uh : 0.0, has_k ? x.kw : 0.0, cloud ? x.cl * kcl : 0.0, v.bg);
+    v.src = srcfunc_du(M.st, inv_dst, sr_col, x.t, v.dsrc);
+    v.s = rounded(tg * (double)__expf((float)(-v.beta * x.ds)));
+    return v;
+  };
+
+  // ---------------- forward sweep: tau_i (and D_i) per point ----------------
+  double rad = 0, tau = 1, dr = 0;
+  int nef = N;
+  {
+    constexpr int RP = 4 * ROW_FP;
+    bool open = true;
+    for (int r0 = 0; r0 < npb; r0 += RP) {
+      const int i0 = r0 + role * ROW_FP;
+      const int i1 = i0 + ROW_FP < N ? i0 + ROW_FP : N;
+      PtIn nx{};
+      if (i0 < i1) nx = ld_pt(i0);
+      for (int ip = i0; ip < i1; ip++) {
+        const PtIn x = nx;
+        nx = ld_pt(ip + 1 < i1 ? ip + 1 : ip);
+        const double q = qprod(x.e);
+        Seg v;
+        v.s = -1;  // opaque
+        v.src = 0;
+        if (q > 0) v = segment(x, q);
+        LD((ip - r0) * 2) = v.s;
+        LD((ip - r0) * 2 + 1) = v.src;
+      }
+      __syncthreads();
+      if (role == 0) {
+        const int n = N - r0 < RP ? N - r0 : RP;
+        for (int k = 0; k < n && open; k++) {
+          const double s = LD(k * 2), src = LD(k * 2 + 1);
+          const int ip = r0 + k;
+          if (s < 0) {
+            nef = ip;
+            open = false;
+            break;
+          }
+          SCR(0, ip) = tau;
+          if (J.nscr > 1) SCR(1, ip) = dr;
+          rad += src * (1 - s) * tau;
+          dr = dr * s + src * (1 - s);
+          tau *= s;
+        }
+      }
+      __syncthreads();
+    }
+    if (role == 0) s_nef[lane] = map ? nef : 0;
+    __syncthreads();
+  }
+  const int ne = s_nef[lane];  // points of the lane's reverse sweep
+  int hi = ne;
+  for (int o = 32; o > 0; o >>= 1) hi = max(hi, __shfl_xor(hi, o));
+  hi = __builtin_amdgcn_readfirstlane(hi);
+  const int nround = (hi + ROW_RP - 1) / ROW_RP;
+#define TERM(r, j, k) LD((((r) & 1) * ROW_RP + (j)) * ROW_TERMS + (k))
+#define GZ(r, j, k) LD(N_TERM + (((r) & 1) * ROW_RP + (j)) * 2 + (k))
+
+  if (role >= 2) {
+    // ---------------- the segments' terms and gradients ----------------
+    const int j = role - 2;
+    PtIn nx{};
+    if (hi - 1 - j >= 0) nx = ld_pt(hi - 1 - j);
+    for (int r = 0; r < nround + 2; r++) {
+      const int ip = hi - 1 - (r * ROW_RP + j);
+      if (ip >= 0) {
+        const PtIn x = nx;
+        if (ip >= ROW_RP) nx = ld_pt(ip - ROW_RP);
+        if (ip < ne) {
+          const Seg v = segment(x, qprod(x.e));
+          const double ucoef = 10 * x.p * v.rt * x.ds * (1 / JUR_KB);
+          const double uu = v.bg.du_co2 * (co2 ? x.uc : 0.0) + v.bg.du_h2o * (h2o ? x.uh : 0.0);
+          TERM(r, j, 0) = v.s;
+          TERM(r, j, 1) = v.src;
+          TERM(r, j, 2) = v.dsrc;
+          TERM(r, j, 3) = v.beta;
+          // per d rad / d beta_i: T, p, q_co2, q_h2o
+          TERM(r, j, 4) = v.bg.dt - uu * v.rt;
+          TERM(r, j, 5) = v.bg.dp + uu * v.rp;
+          TERM(r, j, 6) = v.bg.du_co2 * ucoef;
+          TERM(r, j, 7) = v.bg.du_h2o * ucoef + v.bg.dq_h2o;
+        }
+      }
+      __syncthreads();
+    }
+    return;
+  }
+
+  if (role == 1) {
+    // ---------------- the refracted path's reverse march ----------------
+    PathRev<1, true> P;
+    P.xm = xm;
+    P.nlev = atm->np;
+    P.nc = 1;
+    P.kt0 = kt;
+    P.ktstride = (size_t)J.ncol * WAVE;
+    const char *pcg = PATH ? (const char *)(J.pco + J.soff[bl] / ((size_t)nd * J.nscr) * JUR_NPCO) : nullptr;
+    double *pcs = lds + (size_t)(N_TERM + N_GZ) * WAVE;
+    // step k's coefficients into buffer k & 1, which step k + 2 has been read
+    // from (its reads have completed: the memory clobber keeps the compiler
+    // from moving them below the copy, whose LDS write it does not see)
+    auto pc_fetch = [&](int k) {
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      const char *g = pcg + (size_t)k * JUR_NPCO * WAVE * sizeof(double) + lane * 16;
+      char *o = (char *)(pcs + (size_t)(k & 1) * JUR_NPCO * WAVE);
+#pragma unroll
+      for (int i = 0; i < JUR_NPCO / 2; i++)
+        __builtin_amdgcn_global_load_lds((const void *)(g + i * 1024),
+                                         (__attribute__((address_space(3))) void *)(o + i * 1024), 16, 0, 0);
+    };
+    bool pstart = false;
+    double gz_last = 0, gd_last = 0;
+    if (PATH && hi > 0) pc_fetch(hi - 1);
+    for (int r = 0; r < nround + 2; r++) {
+      if (PATH && r >= 2) {
+        for (int j = 0; j < ROW_RP; j++) {
+          const int ip = hi - 1 - ((r - 2) * ROW_RP + j);
+          if (ip < 0) break;
+          // the copy of this step's coefficients has landed in LDS: the
+          // direct-to-LDS loads count as vector memory loads, which the
+          // compiler does not track for LDS reads (the memory clobber keeps
+          // the reads below the wait); then the next step's are sent for
+          asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+          if (ip > 0) pc_fetch(ip - 1);
+          if (ip >= ne) continue;
+          const double gzc = GZ(r, j, 0), gdc = GZ(r, j, 1);
+          if (ip == N - 1) {
+            gz_last = gzc;
+            gd_last = gdc;
+            continue;
+          }
+          if (!pstart) {
+            // the first step reached: the clip of the last step, with point
+            // N-2's d rad / d ds where this is that point
+            double xl[3];
+            for (int i = 0; i < 3; i++) xl[i] = LOSR(L.f_xe + i, N - 1);
+            const double gdm = ip == N - 2 ? gdc : 0.0;
+            P.init(M, tail[ir], xl, &gz_last, &gd_last, &gdm);
+            pstart = true;
+          }
+          const double *cf = pcs + (size_t)(ip & 1) * JUR_NPCO * WAVE + lane;
+          P.template step<1>(ip, N, cf, &gzc, &gdc);
+          if (ip == N - 2) P.template join_clip<1>(cf);
+        }
+      }
+      __syncthreads();
+    }
+    if (PATH && pstart) P.finish();
+    return;
+  }
+
+  // ---------------- wave 0: surface terms and their adjoint seeds ----------------
+  double sfeps = 1.0, wsf = 0;
+  if (M.nsf > 0) {
+    const double x0 = M.sfnu[C.isf], x1 = M.sfnu[C.isf + 1];
+    sfeps = lin(x0, atm->sfeps[C.isf], x1, atm->sfeps[C.isf + 1], nu);
+    wsf = (nu - x0) / (x1 - x0);
+  }
+  const bool surf = ok && M.sftype >= 1 && R.sft > 0;
+  double tb = 0, db = 0, sft_bar = 0, sfeps_bar = 0;
+  if (surf) {
+    double dsrc_sf;
+    const double src_sf = srcfunc_d(M.st, sr_col, R.sft, dsrc_sf);
+    rad += sfeps * src_sf * tau;
+    tb += sfeps * src_sf;
+    sfeps_bar += src_sf * tau;
+    sft_bar = sfeps * tau * dsrc_sf;
+    if (M.sftype >= 2 && sfeps < 1) {
+      rad += dr * tau * (1 - sfeps);
+      tb += dr * (1 - sfeps);
+      db += tau * (1 - sfeps);
+      sfeps_bar -= dr * tau;
+      if (M.sftype >= 3 && R.pad > 0) {
+        const double ks = 6.764e-5 / (2. * JUR_PI) * C.planck_sun * R.rcos;
+        rad += ks * tau * (1 - sfeps) * tau;
+        tb += 2 * ks * tau * (1 - sfeps);
+        sfeps_bar -= ks * tau * tau;
+      }
+    }
+  }
+  if (ok) {
+    rad_out[(size_t)ir * nd + id] = rad;
+    tau_out[(size_t)ir * nd + id] = tau;
+  }
+  // the surface temperature taken from the last LOS point's T
+  const bool sft_los = surf && !(M.nsf > 0 && atm->sft > 0) && N > 0;
+  int lv_sf = 0;
+  double w_sf = 0, gz_sft = 0;
+  if (sft_los) {
+    lv_sf = level_of(atm, LOSR(F_Z, N - 1), -1, w_sf);
+    gz_sft = sft_bar * (atm->t[lv_sf + 1] - atm->t[lv_sf]) / (atm->z[lv_sf + 1] - atm->z[lv_sf]);
+  }
+
+  // ---------------- wave 0: the accumulation's and the chains' reverse ----------------
+  constexpr int NQW = 3 + EM;  // T, p, the window's extinction, every emitter's q
+  int qi[NQW];
+  qi[0] = 1;
+  qi[1] = 0;
+  qi[2] = has_k ? 2 + NG + C.window : -1;
+#pragma unroll
+  for (int g = 0; g < EM; g++) qi[3 + g] = g < ng ? 2 + g : -1;
+  LevelWindow<NQW, (1u << NQW) - 1u, true, PATH> W;
+  int lev = -1;
+  double clz_bar = 0, cldz_bar = 0, clk_bar = 0, Hn = 0;
+  double carry[EM];
+  float trc[EM];
+#pragma unroll
+  for (int g = 0; g < EM; g++) {
+    carry[g] = 0;
+    trc[g] = on[g] && ne > 0 ? (float)trans_of(EPS_AT(g, ne - 1)) : 1.f;
+  }
+  // the point's inputs, loaded one point ahead
+  struct RevIn {
+    double z, p, t, ds, cl, tau, dr, u[EM];
+    float4 d[EM];
+    float em[EM];
+  };
+  auto ld_rev = [&](int ip) {
+    RevIn x;
+    x.z = LOSR(F_Z, ip);
+    x.p = LOSR(F_P, ip);
+    x.t = LOSR(F_T, ip);
+    x.ds = LOSR(F_DS, ip);
+    x.cl = LOSR(f_cl, ip);
+    x.tau = SCR(0, ip);
+    x.dr = J.nscr > 1 ? SCR(1, ip) : 0.0;
+#pragma unroll
+    for (int g = 0; g < EM; g++) {
+      x.u[g] = on[g] ? LOSR(L.f_u + g, ip) : 0.0;
+      x.d[g] = on[g] ? pab[((size_t)g * npb + ip) * WAVE] : make_float4(0.f, 0.f, 0.f, 0.f);
+      x.em[g] = on[g] && ip > 0 ? EPS_AT(g, ip - 1) : 0.f;
+    }
+    return x;
+  };
+  RevIn nx{};
+  if (hi > 0) nx = ld_rev(hi - 1);
+  for (int r = 0; r < nround + 2; r++) {
+    if (r >= 1 && r <= nround) {
+      for (int j = 0; j < ROW_RP; j++) {
+        const int ip = hi - 1 - ((r - 1) * ROW_RP + j);
+        if (ip < 0) break;
+        const RevIn x = nx;
+        if (ip > 0) nx = ld_rev(ip - 1);
+        if (ip >= ne) continue;
+        const double s = TERM(r - 1, j, 0), src = TERM(r - 1, j, 1), dsrc = TERM(r - 1, j, 2);
+        const double beta = TERM(r - 1, j, 3);
+        const double G = x.tau * (tb - src) + db * (x.dr - src);
+        const double src_bar = (1 - s) * (x.tau + db);
+        tb = src * (1 - s) + tb * s;
+        db = db * s;
+        const double H = G * s;
+        const double beta_bar = -H * x.ds;
+        double v[NQW];
+        v[0] = beta_bar * TERM(r - 1, j, 4) + src_bar * dsrc;  // T
+        v[1] = beta_bar * TERM(r - 1, j, 5);                   // p
+        v[2] = beta_bar;                                       // k
+        const double vco2 = beta_bar * TERM(r - 1, j, 6), vh2o = beta_bar * TERM(r - 1, j, 7);
+        // the chains (as k_adj_chains_f32: float reciprocals of T, p and the
+        // transmittance, whose 1e-7 is far below the FP32 lookups')
+        const double rtf = (double)frcp((float)x.t), rpf = (double)frcp((float)x.p);
+        const double ucf = 10 * x.p * rtf * x.ds * (1 / JUR_KB);
+        double vt = 0, vp = 0, gu = 0;  // gu: the chains' d rad / d ds_i through u
+#pragma unroll
+        for (int g = 0; g < EM; g++) {
+          double vq = (g == M.ig_co2 ? vco2 : 0.0) + (g == M.ig_h2o ? vh2o : 0.0);
+          if (on[g]) {
+            const double lam = (Hn - H) * (double)frcp(trc[g]) + carry[g];
+            const double u_bar = lam * x.d[g].w;
+            carry[g] = lam * x.d[g].x;
+            vt += lam * x.d[g].z - u_bar * x.u[g] * rtf;
+            vp += lam * x.d[g].y + u_bar * x.u[g] * rpf;
+            vq += u_bar * ucf;
+            gu += u_bar * x.u[g];
+            trc[g] = (float)(1.0 - (double)x.em[g]);
+          }
+          v[3 + g] = vq;
+        }
+        v[0] += vt;
+        v[1] += vp;
+        Hn = H;
+        double gz = W.add(atm, x.z, lev, v, 1, x.p, xm, qi, kt);
+        if (PATH) {
+          // altitude: the level quantities' slopes, the cloud profile's and
+          // the surface temperature's; segment length: exp(-beta ds) (the
+          // continua's beta does not depend on ds, their u ~ ds cancels their
+          // 1/ds) and the emitters' column densities
+          if (cloud && atm->cldz > 0)
+            gz -= beta_bar * kcl * x.cl * (x.z - atm->clz) / (atm->cldz * atm->cldz);
+          if (ip == N - 1) gz += gz_sft;
+          GZ(r - 1, j, 0) = gz;
+          GZ(r - 1, j, 1) = -H * beta + gu * rcp_d(x.ds);
+        }
+        if (cloud) {
+          clk_bar += beta_bar * x.cl;
+          if (atm->cldz > 0) {
+            const double cl_bar = beta_bar * kcl;
+            const double dz = (x.z - atm->clz) / atm->cldz;
+            clz_bar += cl_bar * x.cl * dz / atm->cldz;
+            cldz_bar += cl_bar * x.cl * dz * dz / atm->cldz;
+          }
+        }
+      }
+    }
+    __syncthreads();
+  }
+  if (!ok || !map) return;
+  W.flush(xm, qi, kt);
+
+  // surface terms (T columns: the path's wave adds to them too)
+  if (surf) {
+    if (M.nsf > 0 && atm->sft > 0) {
+      const int c = xm[JUR_XMAP_SFT];
+      if (c >= 0) KT(c) += sft_bar;
+    } else if (sft_los) {
+      // the surface temperature is the LOS temperature of the last point
+      int c;
+      if ((c = xm[JUR_XMAP_LEV(1, lv_sf)]) >= 0) unsafeAtomicAdd(&KT(c), (1 - w_sf) * sft_bar);
+      if ((c = xm[JUR_XMAP_LEV(1, lv_sf + 1)]) >= 0) unsafeAtomicAdd(&KT(c), w_sf * sft_bar);
+    }
+    if (M.nsf > 0) {
+      int c;
+      if ((c = xm[JUR_XMAP_SFEPS(C.isf)]) >= 0) KT(c) += (1 - wsf) * sfeps_bar;
+      if (C.isf + 1 < NSF && (c = xm[JUR_XMAP_SFEPS(C.isf + 1)]) >= 0) KT(c) += wsf * sfeps_bar;
+    }
+  }
+  if (cloud) {
+    int c;
+    if ((c = xm[JUR_XMAP_CLK(C.icl)]) >= 0) KT(c) += (1 - wcl) * clk_bar;
+    if (C.icl + 1 < NCL && (c = xm[JUR_XMAP_CLK(C.icl + 1)]) >= 0) KT(c) += wcl * clk_bar;
+    if ((c = xm[JUR_XMAP_CLZ]) >= 0) KT(c) += clz_bar;
+    if ((c = xm[JUR_XMAP_CLDZ]) >= 0) KT(c) += cldz_bar;
+  }
+#undef EPS_AT
+#undef SCR
+#undef KT
+#undef LD
+#undef TERM
+#undef GZ
 }
 
 // The reverse sweep over the steps, CH channels per lane (one ray).  With
@@ -2028,44 +2346,28 @@ static void launch_adj(const ModelView &M, const BatchView &B, const LosView &L,
                        const RayInfo *info, const void *tail, int blk0, int nblk, int maxnp, const JacView &J,
                        double *rad, double *tau, hipStream_t s) {
   const int nb8 = padded_blocks(nblk);
-  // small batches (at most two wavefronts per SIMD), FP32 EGA with stored
-  // partials and at most four emitters: the emitter chains and the path
-  // adjoint run in the accumulation's reverse sweep, one pass instead of
-  // three that each last as long as the longest ray's sweep
-  bool one = false;
-  if constexpr (!CGA && sizeof(SF) == sizeof(float))
-    one = E.part && M.ng >= 1 && M.ng <= 4 && (size_t)nb8 * M.nd < 2048;
+  // small batches, FP32 EGA with stored partials and at most four emitters:
+  // one workgroup per row (k_adj_row)
+  bool row = false;
+  if constexpr (!CGA && sizeof(SF) == sizeof(float)) row = E.part && M.ng >= 1 && M.ng <= 4 && nb8 * M.nd < 2048;
   if (PATH) {
-    // reverse-step coefficients of steps 0 .. np - 2 (lane-major for the
-    // one-sweep form)
+    // reverse-step coefficients of steps 0 .. np - 2
     const int nchunk = (maxnp - 1 + PCO_STEPS - 1) / PCO_STEPS;
-    if (nchunk > 0) {
-      if (one)
-        hipLaunchKernelGGL(k_path_coef<true>, dim3(nb8 * nchunk), dim3(WAVE), 0, s, M, B, L, info, blk0, nblk,
-                           nchunk, J);
-      else
-        hipLaunchKernelGGL(k_path_coef<false>, dim3(nb8 * nchunk), dim3(WAVE), 0, s, M, B, L, info, blk0, nblk,
-                           nchunk, J);
-    }
+    if (nchunk > 0)
+      hipLaunchKernelGGL(k_path_coef, dim3(nb8 * nchunk), dim3(WAVE), 0, s, M, B, L, info, blk0, nblk, nchunk, J);
   }
-  bool fused = false;
   if constexpr (!CGA && sizeof(SF) == sizeof(float)) {
-    if (one) {
-      const dim3 grow(nb8 * M.nd), blk(WAVE);
-      const RayTail *tl = (const RayTail *)tail;
-      if (M.ng <= 2)
-        hipLaunchKernelGGL((k_adj_acc<SF, PATH, 2, PATH>), grow, blk, 0, s, M, B, L, E, info, tl, blk0, nblk, J,
-                           rad, tau);
-      else if (M.ng == 3)
-        hipLaunchKernelGGL((k_adj_acc<SF, PATH, 3, PATH>), grow, blk, 0, s, M, B, L, E, info, tl, blk0, nblk, J,
-                           rad, tau);
-      else
-        hipLaunchKernelGGL((k_adj_acc<SF, PATH, 4, PATH>), grow, blk, 0, s, M, B, L, E, info, tl, blk0, nblk, J,
-                           rad, tau);
-      fused = true;
+    if (row) {
+      auto run = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(nb8 * M.nd), dim3(4 * WAVE), 0, s, M, B, L, E, info, (const RayTail *)tail,
+                           blk0, nblk, J, rad, tau);
+      };
+      if (M.ng <= 2) run(k_adj_row<2, PATH>);
+      else if (M.ng == 3) run(k_adj_row<3, PATH>);
+      else run(k_adj_row<4, PATH>);
+      return;
     }
   }
-  if (fused) return;
   hipLaunchKernelGGL((k_adj_acc<SF, PATH>), dim3(nb8 * M.nd), dim3(WAVE), 0, s, M, B, L, E, info,
                      (const RayTail *)tail, blk0, nblk, J, rad, tau);
   if (M.ng > 0) {
