@@ -1765,17 +1765,20 @@ __global__ __launch_bounds__(WAVE) void k_adj_acc(ModelView M, BatchView B, LosV
 // the points (same formulas).
 //   forward: all four waves form the segments' s and src (they do not depend
 //     on each other), wave 0 the running tau, D and radiance;
-//   reverse, in rounds of ROW_RP points, each stage a round behind the one
-//     before: waves 2 and 3 the segment's terms and gradients, wave 0 the
-//     accumulation's adjoint, the emitter chains and the level sums, wave 1
+//   reverse, a point per round, each stage a round behind the one before:
+//     wave 2 the segment's terms and gradients, wave 0 the accumulation's
+//     adjoint and the emitter chains, wave 3 the sums over the levels, wave 1
 //     the reverse march of the refracted path, whose coefficients it copies
 //     into LDS a step ahead.
 // All lanes of the workgroup are at the same point (a lane begins at its own
 // last one), so a step's coefficients are one contiguous copy.  Wave 1 adds
-// to the T and p columns that wave 0 adds to: both add atomically.
-// One wave ran the two sweeps with everything in the reverse one before: 512
-// registers, 1140 vector instructions per point of one wave in series.
-constexpr int ROW_RP = 2;  // points per round: one per producing wave
+// to the T and p columns that wave 3 adds to: both add atomically.
+//
+// Bound by the slowest stage's chain of FP64 operations.  64 x 32 x 12 limb
+// rows: 7.9 ms when one wave ran the two sweeps with everything in the
+// reverse one (512 registers, 1140 vector instructions per point in series),
+// 5.05 ms with the level sums in wave 0 (they change their level pair at most
+// points in some of 64 different profiles: half of that wave's time), 3.8 ms.
 constexpr int ROW_TERMS = 8;
 constexpr int ROW_FP = 8;  // points per wave and round of the forward sweep
 
@@ -1813,11 +1816,13 @@ __global__ __launch_bounds__(4 * WAVE, 2) void k_adj_row(ModelView M, BatchView 
   const double *sr_col = M.sr + (size_t)id * TBLNS;
   const double inv_dst = 1 / (M.st[1] - M.st[0]);
 
-  // LDS: the forward sweep's segments; then the terms [buffer][point][term],
-  // the point values [buffer][point][z, ds] and two steps' coefficients
-  constexpr int N_TERM = 2 * ROW_RP * ROW_TERMS, N_GZ = 2 * ROW_RP * 2, N_PC = PATH ? 2 * JUR_NPCO : 0;
-  constexpr int N_FWD = 4 * ROW_FP * 2;
-  __shared__ double lds[(N_TERM + N_GZ + N_PC > N_FWD ? N_TERM + N_GZ + N_PC : N_FWD) * WAVE];
+  constexpr int NQW = 3 + EM;  // level quantities: T, p, the window's extinction, every emitter's q
+  // LDS: the forward sweep's segments; then, two buffers each, the terms, the
+  // point adjoints (with the rest of d rad / d z_i and d rad / d ds_i), the
+  // path's point values, and two steps' coefficients
+  constexpr int N_TERM = 2 * ROW_TERMS, N_V = 2 * (NQW + 2), N_GZ = 2 * 2, N_PC = PATH ? 2 * JUR_NPCO : 0;
+  constexpr int N_FWD = 4 * ROW_FP * 2, N_REV = N_TERM + N_V + N_GZ + N_PC;
+  __shared__ double lds[(N_REV > N_FWD ? N_REV : N_FWD) * WAVE];
   __shared__ int s_nef[WAVE];
 #define LD(i) lds[(i) * WAVE + lane]
 
@@ -1936,37 +1941,74 @@ __global__ __launch_bounds__(4 * WAVE, 2) void k_adj_row(ModelView M, BatchView 
   int hi = ne;
   for (int o = 32; o > 0; o >>= 1) hi = max(hi, __shfl_xor(hi, o));
   hi = __builtin_amdgcn_readfirstlane(hi);
-  const int nround = (hi + ROW_RP - 1) / ROW_RP;
-#define TERM(r, j, k) LD((((r) & 1) * ROW_RP + (j)) * ROW_TERMS + (k))
-#define GZ(r, j, k) LD(N_TERM + (((r) & 1) * ROW_RP + (j)) * 2 + (k))
+  // round r: point hi - 1 - r in wave 2, the ones after it behind
+  const int nround = hi + 3;
+#define TERM(r, k) LD(((r) & 1) * ROW_TERMS + (k))
+#define VAL(r, k) LD(N_TERM + ((r) & 1) * (NQW + 2) + (k))
+#define GZ(r, k) LD(N_TERM + N_V + ((r) & 1) * 2 + (k))
 
-  if (role >= 2) {
+  if (role == 2) {
     // ---------------- the segments' terms and gradients ----------------
-    const int j = role - 2;
     PtIn nx{};
-    if (hi - 1 - j >= 0) nx = ld_pt(hi - 1 - j);
-    for (int r = 0; r < nround + 2; r++) {
-      const int ip = hi - 1 - (r * ROW_RP + j);
+    if (hi > 0) nx = ld_pt(hi - 1);
+    for (int r = 0; r < nround; r++) {
+      const int ip = hi - 1 - r;
       if (ip >= 0) {
         const PtIn x = nx;
-        if (ip >= ROW_RP) nx = ld_pt(ip - ROW_RP);
+        if (ip > 0) nx = ld_pt(ip - 1);
         if (ip < ne) {
           const Seg v = segment(x, qprod(x.e));
           const double ucoef = 10 * x.p * v.rt * x.ds * (1 / JUR_KB);
           const double uu = v.bg.du_co2 * (co2 ? x.uc : 0.0) + v.bg.du_h2o * (h2o ? x.uh : 0.0);
-          TERM(r, j, 0) = v.s;
-          TERM(r, j, 1) = v.src;
-          TERM(r, j, 2) = v.dsrc;
-          TERM(r, j, 3) = v.beta;
+          TERM(r, 0) = v.s;
+          TERM(r, 1) = v.src;
+          TERM(r, 2) = v.dsrc;
+          TERM(r, 3) = v.beta;
           // per d rad / d beta_i: T, p, q_co2, q_h2o
-          TERM(r, j, 4) = v.bg.dt - uu * v.rt;
-          TERM(r, j, 5) = v.bg.dp + uu * v.rp;
-          TERM(r, j, 6) = v.bg.du_co2 * ucoef;
-          TERM(r, j, 7) = v.bg.du_h2o * ucoef + v.bg.dq_h2o;
+          TERM(r, 4) = v.bg.dt - uu * v.rt;
+          TERM(r, 5) = v.bg.dp + uu * v.rp;
+          TERM(r, 6) = v.bg.du_co2 * ucoef;
+          TERM(r, 7) = v.bg.du_h2o * ucoef + v.bg.dq_h2o;
         }
       }
       __syncthreads();
     }
+    return;
+  }
+
+  if (role == 3) {
+    // ---------------- the sums over the levels ----------------
+    int qi[NQW];
+    qi[0] = 1;
+    qi[1] = 0;
+    qi[2] = has_k ? 2 + NG + C.window : -1;
+#pragma unroll
+    for (int g = 0; g < EM; g++) qi[3 + g] = g < ng ? 2 + g : -1;
+    LevelWindow<NQW, (1u << NQW) - 1u, true, PATH> W;
+    int lev = -1;
+    double zn = hi > 0 ? LOSR(F_Z, hi - 1) : 0, pn = hi > 0 ? LOSR(F_P, hi - 1) : 0;
+    for (int r = 0; r < nround; r++) {
+      const int ip = hi - 1 - (r - 2);
+      if (r >= 2 && ip >= 0) {
+        const double z = zn, p = pn;
+        if (ip > 0) {
+          zn = LOSR(F_Z, ip - 1);
+          pn = LOSR(F_P, ip - 1);
+        }
+        if (ip < ne) {
+          double v[NQW];
+#pragma unroll
+          for (int q = 0; q < NQW; q++) v[q] = VAL(r, q);
+          const double gz = W.add(atm, z, lev, v, 1, p, xm, qi, kt);
+          if (PATH) {
+            GZ(r, 0) = gz + VAL(r, NQW);
+            GZ(r, 1) = VAL(r, NQW + 1);
+          }
+        }
+      }
+      __syncthreads();
+    }
+    if (map) W.flush(xm, qi, kt);
     return;
   }
 
@@ -1979,7 +2021,7 @@ __global__ __launch_bounds__(4 * WAVE, 2) void k_adj_row(ModelView M, BatchView 
     P.kt0 = kt;
     P.ktstride = (size_t)J.ncol * WAVE;
     const char *pcg = PATH ? (const char *)(J.pco + J.soff[bl] / ((size_t)nd * J.nscr) * JUR_NPCO) : nullptr;
-    double *pcs = lds + (size_t)(N_TERM + N_GZ) * WAVE;
+    double *pcs = lds + (size_t)(N_TERM + N_V + N_GZ) * WAVE;
     // step k's coefficients into buffer k & 1, which step k + 2 has been read
     // from (its reads have completed: the memory clobber keeps the compiler
     // from moving them below the copy, whose LDS write it does not see)
@@ -1995,24 +2037,20 @@ __global__ __launch_bounds__(4 * WAVE, 2) void k_adj_row(ModelView M, BatchView 
     bool pstart = false;
     double gz_last = 0, gd_last = 0;
     if (PATH && hi > 0) pc_fetch(hi - 1);
-    for (int r = 0; r < nround + 2; r++) {
-      if (PATH && r >= 2) {
-        for (int j = 0; j < ROW_RP; j++) {
-          const int ip = hi - 1 - ((r - 2) * ROW_RP + j);
-          if (ip < 0) break;
-          // the copy of this step's coefficients has landed in LDS: the
-          // direct-to-LDS loads count as vector memory loads, which the
-          // compiler does not track for LDS reads (the memory clobber keeps
-          // the reads below the wait); then the next step's are sent for
-          asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-          if (ip > 0) pc_fetch(ip - 1);
-          if (ip >= ne) continue;
-          const double gzc = GZ(r, j, 0), gdc = GZ(r, j, 1);
-          if (ip == N - 1) {
-            gz_last = gzc;
-            gd_last = gdc;
-            continue;
-          }
+    for (int r = 0; r < nround; r++) {
+      const int ip = hi - 1 - (r - 3);
+      if (PATH && r >= 3) {
+        // the copy of this step's coefficients has landed in LDS: the
+        // direct-to-LDS loads count as vector memory loads, which the
+        // compiler does not track for LDS reads (the memory clobber keeps
+        // the reads below the wait); then the next step's are sent for
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        if (ip > 0) pc_fetch(ip - 1);
+        const double gzc = GZ(r - 1, 0), gdc = GZ(r - 1, 1);
+        if (ip < ne && ip == N - 1) {
+          gz_last = gzc;
+          gd_last = gdc;
+        } else if (ip < ne) {
           if (!pstart) {
             // the first step reached: the clip of the last step, with point
             // N-2's d rad / d ds where this is that point
@@ -2076,15 +2114,6 @@ __global__ __launch_bounds__(4 * WAVE, 2) void k_adj_row(ModelView M, BatchView 
   }
 
   // ---------------- wave 0: the accumulation's and the chains' reverse ----------------
-  constexpr int NQW = 3 + EM;  // T, p, the window's extinction, every emitter's q
-  int qi[NQW];
-  qi[0] = 1;
-  qi[1] = 0;
-  qi[2] = has_k ? 2 + NG + C.window : -1;
-#pragma unroll
-  for (int g = 0; g < EM; g++) qi[3 + g] = g < ng ? 2 + g : -1;
-  LevelWindow<NQW, (1u << NQW) - 1u, true, PATH> W;
-  int lev = -1;
   double clz_bar = 0, cldz_bar = 0, clk_bar = 0, Hn = 0;
   double carry[EM];
   float trc[EM];
@@ -2118,16 +2147,14 @@ __global__ __launch_bounds__(4 * WAVE, 2) void k_adj_row(ModelView M, BatchView 
   };
   RevIn nx{};
   if (hi > 0) nx = ld_rev(hi - 1);
-  for (int r = 0; r < nround + 2; r++) {
-    if (r >= 1 && r <= nround) {
-      for (int j = 0; j < ROW_RP; j++) {
-        const int ip = hi - 1 - ((r - 1) * ROW_RP + j);
-        if (ip < 0) break;
-        const RevIn x = nx;
-        if (ip > 0) nx = ld_rev(ip - 1);
-        if (ip >= ne) continue;
-        const double s = TERM(r - 1, j, 0), src = TERM(r - 1, j, 1), dsrc = TERM(r - 1, j, 2);
-        const double beta = TERM(r - 1, j, 3);
+  for (int r = 0; r < nround; r++) {
+    const int ip = hi - 1 - (r - 1);
+    if (r >= 1 && ip >= 0) {
+      const RevIn x = nx;
+      if (ip > 0) nx = ld_rev(ip - 1);
+      if (ip < ne) {
+        const double s = TERM(r - 1, 0), src = TERM(r - 1, 1), dsrc = TERM(r - 1, 2);
+        const double beta = TERM(r - 1, 3);
         const double G = x.tau * (tb - src) + db * (x.dr - src);
         const double src_bar = (1 - s) * (x.tau + db);
         tb = src * (1 - s) + tb * s;
@@ -2135,10 +2162,10 @@ __global__ __launch_bounds__(4 * WAVE, 2) void k_adj_row(ModelView M, BatchView 
         const double H = G * s;
         const double beta_bar = -H * x.ds;
         double v[NQW];
-        v[0] = beta_bar * TERM(r - 1, j, 4) + src_bar * dsrc;  // T
-        v[1] = beta_bar * TERM(r - 1, j, 5);                   // p
+        v[0] = beta_bar * TERM(r - 1, 4) + src_bar * dsrc;  // T
+        v[1] = beta_bar * TERM(r - 1, 5);                   // p
         v[2] = beta_bar;                                       // k
-        const double vco2 = beta_bar * TERM(r - 1, j, 6), vh2o = beta_bar * TERM(r - 1, j, 7);
+        const double vco2 = beta_bar * TERM(r - 1, 6), vh2o = beta_bar * TERM(r - 1, 7);
         // the chains (as k_adj_chains_f32: float reciprocals of T, p and the
         // transmittance, whose 1e-7 is far below the FP32 lookups')
         const double rtf = (double)frcp((float)x.t), rpf = (double)frcp((float)x.p);
@@ -2162,17 +2189,17 @@ __global__ __launch_bounds__(4 * WAVE, 2) void k_adj_row(ModelView M, BatchView 
         v[0] += vt;
         v[1] += vp;
         Hn = H;
-        double gz = W.add(atm, x.z, lev, v, 1, x.p, xm, qi, kt);
+#pragma unroll
+        for (int q = 0; q < NQW; q++) VAL(r - 1, q) = v[q];
         if (PATH) {
-          // altitude: the level quantities' slopes, the cloud profile's and
-          // the surface temperature's; segment length: exp(-beta ds) (the
-          // continua's beta does not depend on ds, their u ~ ds cancels their
-          // 1/ds) and the emitters' column densities
-          if (cloud && atm->cldz > 0)
-            gz -= beta_bar * kcl * x.cl * (x.z - atm->clz) / (atm->cldz * atm->cldz);
-          if (ip == N - 1) gz += gz_sft;
-          GZ(r - 1, j, 0) = gz;
-          GZ(r - 1, j, 1) = -H * beta + gu * rcp_d(x.ds);
+          // altitude, beside the level quantities' slopes: the cloud
+          // profile's and the surface temperature's; segment length: exp(-beta
+          // ds) (the continua's beta does not depend on ds, their u ~ ds
+          // cancels their 1/ds) and the emitters' column densities
+          double gz = ip == N - 1 ? gz_sft : 0.0;
+          if (cloud && atm->cldz > 0) gz -= beta_bar * kcl * x.cl * (x.z - atm->clz) / (atm->cldz * atm->cldz);
+          VAL(r - 1, NQW) = gz;
+          VAL(r - 1, NQW + 1) = -H * beta + gu * rcp_d(x.ds);
         }
         if (cloud) {
           clk_bar += beta_bar * x.cl;
@@ -2188,9 +2215,8 @@ __global__ __launch_bounds__(4 * WAVE, 2) void k_adj_row(ModelView M, BatchView 
     __syncthreads();
   }
   if (!ok || !map) return;
-  W.flush(xm, qi, kt);
 
-  // surface terms (T columns: the path's wave adds to them too)
+  // surface terms (T columns: the other waves add to them too)
   if (surf) {
     if (M.nsf > 0 && atm->sft > 0) {
       const int c = xm[JUR_XMAP_SFT];
@@ -2219,6 +2245,7 @@ __global__ __launch_bounds__(4 * WAVE, 2) void k_adj_row(ModelView M, BatchView 
 #undef KT
 #undef LD
 #undef TERM
+#undef VAL
 #undef GZ
 }
 
