@@ -2373,10 +2373,14 @@ static void launch_adj(const ModelView &M, const BatchView &B, const LosView &L,
                        const RayInfo *info, const void *tail, int blk0, int nblk, int maxnp, const JacView &J,
                        double *rad, double *tau, hipStream_t s) {
   const int nb8 = padded_blocks(nblk);
-  // small batches, FP32 EGA with stored partials and at most four emitters:
-  // one workgroup per row (k_adj_row)
+  // FP32 EGA with stored partials and at most four emitters: one workgroup per
+  // row (k_adj_row), up to some 16 rounds of them (512 run at once).  Whole
+  // Jacobian passes, row form against the kernels below: 3072 rows of nadir
+  // paths 20.7 / 23.2 ms, 6144 40.3 / 41.7, 6144 of limb paths 27.4 / 31.0,
+  // but 12,288 of nadir paths 78.0 / 71.0 (the four waves share a CU's
+  // registers with one other workgroup, which hides less of HBM's latency).
   bool row = false;
-  if constexpr (!CGA && sizeof(SF) == sizeof(float)) row = E.part && M.ng >= 1 && M.ng <= 4 && nb8 * M.nd < 2048;
+  if constexpr (!CGA && sizeof(SF) == sizeof(float)) row = E.part && M.ng >= 1 && M.ng <= 4 && nb8 * M.nd < 8192;
   if (PATH) {
     // reverse-step coefficients of steps 0 .. np - 2
     const int nchunk = (maxnp - 1 + PCO_STEPS - 1) / PCO_STEPS;
