@@ -169,71 +169,101 @@ struct LkPart {
   double dep, dp, dt, du;
 };
 
+// The table cell of the point before, whose grids and sizes are read again
+// only when the cell changes (reading them per point is a chain of dependent
+// loads, most of a point's time in small batches).
+struct PartCell {
+  int ipr = -1, j0 = -1, j1 = -1, nt0 = 0, nt1 = 0;
+  bool full = false;
+  double pa = 0, pb = 0, rp = 0, g00 = 0, g01 = 0, g10 = 0, g11 = 0, ta0 = 0, s0 = 0, ta1 = 0, s1 = 0;
+  int nc[4] = {0, 0, 0, 0};
+};
+
 template <bool CGA>
 __device__ __forceinline__ LkPart lookup_partials(const TabView &T, int tix, int npt, int mono, int pdir,
-                                                  double ep, double pq, double tq, double x, int &ipr,
+                                                  double ep, double pq, double tq, double x, PartCell &c,
                                                   int *gi) {
   LkPart d{0, 0, 0, 0};
   const double *pg = T.p + (size_t)tix * T.TP;
-  ipr = (pdir != 0 && ipr >= 0) ? irr_walk(pg, npt, pq, ipr, pdir) : locate_irr(pg, npt, pq);
-  const double pa = pg[ipr], pb = pg[ipr + 1];
-  const int *ntp = T.nt + (size_t)tix * T.TP;
-  const int nt0 = ntp[ipr], nt1 = ntp[ipr + 1];
-  if (nt0 < 2 || nt1 < 2) {
+  bool keep = false;
+  if (c.ipr >= 0 && pdir > 0) keep = (c.ipr == 0 || !(c.pa > pq)) && (c.ipr == npt - 2 || c.pb > pq);
+  if (c.ipr >= 0 && pdir < 0) keep = (c.ipr == 0 || !(c.pa <= pq)) && (c.ipr == npt - 2 || c.pb <= pq);
+  if (!keep) {
+    c.ipr = (pdir != 0 && c.ipr >= 0) ? irr_walk(pg, npt, pq, c.ipr, pdir) : locate_irr(pg, npt, pq);
+    c.pa = pg[c.ipr];
+    c.pb = pg[c.ipr + 1];
+    c.rp = 1 / (c.pb - c.pa);
+    const int *ntp = T.nt + (size_t)tix * T.TP;
+    c.nt0 = ntp[c.ipr];
+    c.nt1 = ntp[c.ipr + 1];
+    const double *tg = T.t + ((size_t)tix * T.TP + c.ipr) * T.TT;
+    c.g00 = tg[0];
+    c.g01 = tg[1];
+    c.g10 = tg[T.TT];
+    c.g11 = tg[T.TT + 1];
+    c.j0 = c.j1 = -1;
+  }
+  if (c.nt0 < 2 || c.nt1 < 2) {
     d.dep = 1;
     return d;
   }
-  const double *tg0 = T.t + ((size_t)tix * T.TP + ipr) * T.TT;
-  int j0 = (int)((tq - tg0[0]) / (tg0[1] - tg0[0]));
-  j0 = j0 < 0 ? 0 : (j0 > nt0 - 2 ? nt0 - 2 : j0);
-  int j1 = (int)((tq - tg0[T.TT]) / (tg0[T.TT + 1] - tg0[T.TT]));
-  j1 = j1 < 0 ? 0 : (j1 > nt1 - 2 ? nt1 - 2 : j1);
-  const size_t c0 = (size_t)tix * T.TP + ipr;
-  int nc[4];
-  nc[0] = T.nu[c0 * T.TT + j0];
-  nc[1] = T.nu[c0 * T.TT + j0 + 1];
-  nc[2] = T.nu[(c0 + 1) * T.TT + j1];
-  nc[3] = T.nu[(c0 + 1) * T.TT + j1 + 1];
-  if (nc[0] < 2 || nc[1] < 2 || nc[2] < 2 || nc[3] < 2) {
+  int j0 = (int)((tq - c.g00) / (c.g01 - c.g00));
+  j0 = j0 < 0 ? 0 : (j0 > c.nt0 - 2 ? c.nt0 - 2 : j0);
+  int j1 = (int)((tq - c.g10) / (c.g11 - c.g10));
+  j1 = j1 < 0 ? 0 : (j1 > c.nt1 - 2 ? c.nt1 - 2 : j1);
+  const size_t c0 = (size_t)tix * T.TP + c.ipr;
+  const size_t col0 = c0 * T.TT + j0, col1 = (c0 + 1) * T.TT + j1;
+  if (j0 != c.j0 || j1 != c.j1) {
+    c.j0 = j0;
+    c.j1 = j1;
+    c.nc[0] = T.nu[col0];
+    c.nc[1] = T.nu[col0 + 1];
+    c.nc[2] = T.nu[col1];
+    c.nc[3] = T.nu[col1 + 1];
+    c.full = c.nc[0] >= 2 && c.nc[1] >= 2 && c.nc[2] >= 2 && c.nc[3] >= 2;
+    c.ta0 = T.t[col0];
+    c.s0 = 1 / (T.t[col0 + 1] - c.ta0);
+    c.ta1 = T.t[col1];
+    c.s1 = 1 / (T.t[col1 + 1] - c.ta1);
+  }
+  if (!c.full) {
     d.dep = 1;
     return d;
   }
+  const double pa = c.pa, pb = c.pb;
   // eps00 = sum_c cw_c e_c is linear in the corner values: every partial is a
   // weighted sum over the corners, accumulated corner by corner
-  const double ta0 = tg0[j0], tb0 = tg0[j0 + 1];
-  const double ta1 = tg0[T.TT + j1], tb1 = tg0[T.TT + j1 + 1];
-  const double s0 = 1 / (tb0 - ta0), s1 = 1 / (tb1 - ta1);
-  const double w0 = (tq - ta0) * s0, w1 = (tq - ta1) * s1;
+  const double s0 = c.s0, s1 = c.s1;
+  const double w0 = (tq - c.ta0) * s0, w1 = (tq - c.ta1) * s1;
   double wp, dwp;
   if (CGA && pq / pa > 0 && pb / pa > 0) {
     const double l = 1 / log(pb / pa);
     wp = log(pq / pa) * l;
     dwp = l / pq;
   } else {
-    dwp = 1 / (pb - pa);
+    dwp = c.rp;
     wp = (pq - pa) * dwp;
   }
   const double q0 = 1 - wp, q1 = wp;
   const double cw[4] = {q0 * (1 - w0), q0 * w0, q1 * (1 - w1), q1 * w1};  // value
   const double tw[4] = {-q0 * s0, q0 * s0, -q1 * s1, q1 * s1};            // d/dT
   const double pw[4] = {-(1 - w0) * dwp, -w0 * dwp, (1 - w1) * dwp, w1 * dwp};  // d/dp
-  const size_t col0 = c0 * T.TT + j0, col1 = (c0 + 1) * T.TT + j1;
   double en = 0;
 #pragma unroll
-  for (int c = 0; c < 4; c++) {
-    const Col col = T.col((c < 2 ? col0 : col1) + (c & 1));
+  for (int k = 0; k < 4; k++) {
+    const Col col = T.col((k < 2 ? col0 : col1) + (k & 1));
     double e, de, du;
     if (CGA) {
-      cga_corner(col, nc[c], mono, x, gi[c], e, du);
+      cga_corner(col, c.nc[k], mono, x, gi[k], e, du);
       de = 0;
     } else {
-      ega_corner(col, nc[c], mono, ep, x, gi[c], e, de, du);
+      ega_corner(col, c.nc[k], mono, ep, x, gi[k], e, de, du);
     }
-    en += cw[c] * e;
-    d.dep += cw[c] * de;
-    d.du += cw[c] * du;
-    d.dt += tw[c] * e;
-    d.dp += pw[c] * e;
+    en += cw[k] * e;
+    d.dep += cw[k] * de;
+    d.du += cw[k] * du;
+    d.dt += tw[k] * e;
+    d.dp += pw[k] * e;
   }
   if (en < 0 || en > 1) return LkPart{0, 0, 0, 0};  // MAX(MIN(eps00, 1), 0) holds it constant
   return d;
@@ -772,18 +802,30 @@ __global__ __launch_bounds__(WAVE) void k_adj_chain(ModelView M, BatchView B, Lo
       return;
     }
   } else {
+  // each point's inputs are loaded one point ahead
+  double Hx = 0, zx = 0, px = 0, tx = 0, dsx = 0, ux = 0;
+  SF ex = SF(0);
+  auto ahead = [&](int i) {
+    Hx = SCR(0, i);
+    zx = LOSR(F_Z, i);
+    px = LOSR(F_P, i);
+    tx = LOSR(F_T, i);
+    dsx = LOSR(F_DS, i);
+    ux = LOSR(fu, i);
+    if (i > 0) ex = EPS_AT(g, i - 1);
+  };
+  if (nef > 0) ahead(nef - 1);
+  PartCell pcell;
   for (int ip = nef - 1; ip >= 0; ip--) {
-    const double H = SCR(0, ip);
+    const double H = Hx, z = zx, p = px, t = tx, ds = dsx, useg = ux;
     double epp = 0, trp = 1;
     float epf = 0.f;  // the stored float path emissivity (FP32 path)
     if (ip > 0) {
-      const SF sp = EPS_AT(g, ip - 1);
-      epp = emis_of(sp);
-      trp = trans_of(sp);
-      epf = (float)sp;
+      epp = emis_of(ex);
+      trp = trans_of(ex);
+      epf = (float)ex;
+      ahead(ip - 1);
     }
-    const double z = LOSR(F_Z, ip), p = LOSR(F_P, ip), t = LOSR(F_T, ip), ds = LOSR(F_DS, ip);
-    const double useg = LOSR(fu, ip);
     const double lam = (Hn - H) / trc + carry;
     double u_bar, p_bar, t_bar;
     if (CGA) {
@@ -791,7 +833,7 @@ __global__ __launch_bounds__(WAVE) void k_adj_chain(ModelView M, BatchView B, Lo
         const double pq = cp / cu, tq = ct / cu;
         const LkPart d = F32 ? lookup_partials_f32<true>(M.tab, tix, npt, mono, pdir, epf, pq, (float)tq, cu,
                                                          ipr, gi)
-                             : lookup_partials<true>(M.tab, tix, npt, mono, pdir, epp, pq, tq, cu, ipr, gi);
+                             : lookup_partials<true>(M.tab, tix, npt, mono, pdir, epp, pq, tq, cu, pcell, gi);
         sU += lam * (d.du - (d.dp * pq + d.dt * tq) / cu);
         sP += lam * d.dp / cu;
         sT += lam * d.dt / cu;
@@ -808,7 +850,7 @@ __global__ __launch_bounds__(WAVE) void k_adj_chain(ModelView M, BatchView B, Lo
     } else {
       const LkPart d = F32 ? lookup_partials_f32<false>(M.tab, tix, npt, mono, pdir, epf, p, (float)t, useg,
                                                         ipr, gi)
-                           : lookup_partials<false>(M.tab, tix, npt, mono, pdir, epp, p, t, useg, ipr, gi);
+                           : lookup_partials<false>(M.tab, tix, npt, mono, pdir, epp, p, t, useg, pcell, gi);
       u_bar = lam * d.du;
       p_bar = lam * d.dp;
       t_bar = lam * d.dt;
