@@ -318,7 +318,9 @@ __device__ __forceinline__ float eps_from_rec_f(const float4 &r, double x) {
 // slope s = deps/du, and a step that leaves the bracket at its upper knot
 // (u_1, e_1) continues from there with the next slope: the part of u_seg
 // beyond the knot is (ep + u_seg s_0 - e_1)/s_0, hence e_1 + that s_1.  No
-// column density is formed, so nothing cancels and nothing needs FP64.
+// column density is formed, so nothing cancels and nothing needs FP64.  The
+// steps return the growth eps - ep: the caller adds it with the rounding error
+// of the last sum carried, since many steps are below half an ulp of ep.
 //
 // ega_step_fast has the three knots k[0..2] from the previous step's bracket
 // g on in hand (a = k[0], k[1]; b = k[2]; g = -1: the bracket between the
@@ -331,16 +333,17 @@ __device__ __forceinline__ float eps_from_rec_f(const float4 &r, double x) {
 template <bool D>
 __device__ __forceinline__ void ega_step_fast(const float4 &a, const float2 &b, float ep, float us, int &g,
                                               float &ec, float &dep, float &deu, bool &ok) {
+  JUR_FP_EXACT  // the multiply-adds as written: every kernel the same bits
   const float s0 = fdiv(a.w - a.y, a.z - a.x);
   const float s1 = fdiv(b.y - a.w, b.x - a.z);
   const float ratio = fdiv(s1, s0);
   const bool up = ep >= a.w;
   const float s = up ? s1 : s0;
-  const float x = ep + us * s;
+  const float x = __builtin_fmaf(us, s, ep);
   const bool in = x < (up ? b.y : a.w);
-  const float y = a.w + (x - a.w) * ratio;
+  const float over = x - a.w, y = __builtin_fmaf(over, ratio, a.w);
   ok = a.y <= ep && (in || (!up && y < b.y));
-  ec = in ? x : y;
+  ec = in ? us * s : __builtin_fmaf(over, ratio, a.w - ep);
   if (D) {
     dep = in ? 1.f : ratio;
     deu = in ? s : s1;
@@ -358,13 +361,14 @@ __device__ __forceinline__ bool ega_above(const float4 &a, const float2 &b, floa
 template <bool D>
 __device__ __forceinline__ float ega_step_above(float u_last, float e_last, float ep, float us, float &dep,
                                                 float &deu) {
+  JUR_FP_EXACT
   const float c = fdiv(__logf(1.f - e_last), u_last);
-  const float ex = __expf(c * us);
   if (D) {
+    const float ex = __expf(c * us);
     deu = ex > 0.f ? -c * (1.f - ep) * ex : 0.f;
     dep = ex;
   }
-  return 1.f - (1.f - ep) * ex;
+  return -(1.f - ep) * expm1f(c * us);
 }
 
 // FP32 path: eps_from_rec_f with its slope.
@@ -388,6 +392,7 @@ __device__ __forceinline__ float eps_rec_f_vs(const float4 &r, double x, float &
 template <bool D>
 __device__ __forceinline__ float ega_step_slow(Col col, int n, float ep, double useg, int &g, float &dep,
                                                float &deu) {
+  JUR_FP_EXACT
   float4 r, r2;
   const int i = col_walk_f<1>(col, n, ep, g, r);
   g = ep < r.y ? -1 : i;
@@ -399,22 +404,21 @@ __device__ __forceinline__ float ega_step_slow(Col col, int n, float ep, double 
   const float2 k2 = below ? make_float2(r.z, r.w) : col.k[i + 2];
   const float x0 = below ? 0.f : r.x, y0 = below ? 0.f : r.y, x1 = below ? r.x : r.z, y1 = below ? r.y : r.w;
   const float s0 = fdiv(y1 - y0, x1 - x0), s1 = fdiv(k2.y - y1, k2.x - x1);
-  const float x = ep + (float)useg * s0;
+  const float x = __builtin_fmaf((float)useg, s0, ep);
   if (x < y1) {
     if (D) {
       dep = 1.f;
       deu = s0;
     }
-    return x;
+    return (float)useg * s0;
   }
-  const float ratio = fdiv(s1, s0);
-  const float y = y1 + (x - y1) * ratio;
-  if (y < k2.y) {
+  const float ratio = fdiv(s1, s0), over = x - y1;
+  if (__builtin_fmaf(over, ratio, y1) < k2.y) {
     if (D) {
       dep = ratio;
       deu = s1;
     }
-    return y;
+    return __builtin_fmaf(over, ratio, y1 - ep);
   }
   // further up: by the column density
   const float su = fdiv(x1 - x0, y1 - y0);
@@ -427,7 +431,7 @@ __device__ __forceinline__ float ega_step_slow(Col col, int n, float ep, double 
     deu = se;
     dep = se * su;
   }
-  return e;
+  return e - ep;
 }
 
 // Reference-order lookups for columns that are not monotone (bisection).

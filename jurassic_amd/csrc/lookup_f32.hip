@@ -6,7 +6,8 @@
 //    The reference's update tau_path *= 1 - eps with eps = 1 - (1 - eps00) /
 //    tau_path makes tau_path exactly 1 - eps00, so eps_path = eps00 carries
 //    no accumulated rounding, and small emissivities keep full relative
-//    precision in float where 1 - tau_path would not.
+//    precision in float where 1 - tau_path would not.  (It is summed with the
+//    rounding error carried; see cell_interp.)
 //  * The emissivity-growth step u_eq = u(eps_path), eps00 = eps(u_eq + u_seg)
 //    runs along the column's piecewise-linear curve (ega_step_fast): inside a
 //    bracket eps00 = eps_path + u_seg deps/du, and across its upper knot it
@@ -82,15 +83,25 @@ __device__ __forceinline__ V pick(const V *v, int c) {
   return c == 0 ? v[0] : (c == 1 ? v[1] : (c == 2 ? v[2] : v[3]));
 }
 
-// The path emissivity from the corners' (linear in T with weights w0, w1 on
-// the cell's two pressures, then in p with wp; MAX(MIN(eps00, 1), 0)) and, with
-// PART, the step's partials d eps_path / d (eps_prev, p, T, u_seg).
-template <bool PART>
+// The path emissivity from the corners' values (linear in T with weights w0,
+// w1 on the cell's two pressures, then in p with wp; MAX(MIN(eps00, 1), 0)):
+// their growths over ep with GROW (EGA), added with the rounding error rest of
+// the last sum (half an ulp of ep per point would be some 1e-6 of it over a
+// path), or the emissivities themselves.  With PART, the step's partials d
+// eps_path / d (eps_prev, p, T, u_seg) (the slopes in T and p are those of
+// either).
+template <bool PART, bool GROW>
 __device__ __forceinline__ float cell_interp(const float *ec, const float *dep, const float *deu, float w0, float w1,
-                                             float wp, float dt0, float dt1, float dwp, float4 &dpart) {
-  const float a = ec[0] + (ec[1] - ec[0]) * w0;
-  const float b = ec[2] + (ec[3] - ec[2]) * w1;
-  float en = a + (b - a) * wp;
+                                             float wp, float dt0, float dt1, float dwp, float ep, float &rest,
+                                             float4 &dpart) {
+  const float a = __builtin_fmaf(ec[1] - ec[0], w0, ec[0]);
+  const float b = __builtin_fmaf(ec[3] - ec[2], w1, ec[2]);
+  float en = __builtin_fmaf(b - a, wp, a);
+  if (GROW) {
+    const float y = en + rest;
+    en = ep + y;
+    rest = y - (en - ep);
+  }
   if constexpr (PART) {
     // the bilinear cell weights and their T and p slopes
     const float q0 = 1.f - wp, q1 = wp;
@@ -108,6 +119,7 @@ __device__ __forceinline__ float cell_interp(const float *ec, const float *dep, 
     // a clamped emissivity is constant
     dpart = (en < 0.f || en > 1.f) ? make_float4(0.f, 0.f, 0.f, 0.f) : make_float4(sdep, sdp, sdt, sdu);
   }
+  if (GROW && (en < 0.f || en > 1.f)) rest = 0.f;
   en = (en < 1.f) ? en : 1.f;
   return (en > 0.f) ? en : 0.f;
 }
@@ -169,7 +181,7 @@ __global__ __launch_bounds__(WAVE, 4) void k_lookup_f32(ModelView M, BatchView B
   const int *nub = T.nu + (size_t)tix * tcols;
   const float2 *knb = T.kn + (size_t)tix * tcols * T.TS;
 
-  float ep = 0.f;
+  float ep = 0.f, rest = 0.f;  // path emissivity and its last sum's rounding error
   double cu = 0, cp = 0, ct = 0;
   constexpr int NC = RL == 1 ? 4 : 1;  // the lane's corners
   int gi[NC];
@@ -298,7 +310,7 @@ __global__ __launch_bounds__(WAVE, 4) void k_lookup_f32(ModelView M, BatchView B
           else g = gi[0];
           float e, de = 0.f, du = 0.f;
           if (!mono) {
-            e = CGA ? col_eps_bis(col, n, cu) : col_eps_bis(col, n, col_u_bis(col, n, ep) + useg);
+            e = CGA ? col_eps_bis(col, n, cu) : col_eps_bis(col, n, col_u_bis(col, n, ep) + useg) - ep;
           } else if (CGA) {
             float4 r;
             g = col_walk_f<0>(col, n, (float)cu, g, r);
@@ -339,7 +351,7 @@ __global__ __launch_bounds__(WAVE, 4) void k_lookup_f32(ModelView M, BatchView B
           wp = (plog && pq * rpa > 0) ? __logf((float)(pq * rpa)) * lpr : (float)(pq - pa) * wp_scale;
         else
           wp = (float)(pq - pa) * wp_scale;
-        ep = cell_interp<PART>(ec, dep, deu, w0, w1, wp, dt0, dt1, wp_scale, dpart);
+        ep = cell_interp<PART, !CGA>(ec, dep, deu, w0, w1, wp, dt0, dt1, wp_scale, ep, rest, dpart);
       } else {
         pn = LOSR(F_P, ipn);
         tn = LOSR(F_T, ipn);
@@ -420,7 +432,7 @@ __global__ __launch_bounds__(WAVE) void k_lookup_f32_cell(ModelView M, BatchView
   const int TT = T.TT, TS = T.TS, gtop = T.TU - 2;
 
   constexpr int NC = RL == 1 ? 4 : 1;  // the lane's corners
-  float ep = 0.f;
+  float ep = 0.f, rest = 0.f;  // path emissivity and its last sum's rounding error
   int gi[NC];
   unsigned ko[NC];  // knot 0 of the corners' columns
 #pragma unroll
@@ -507,7 +519,7 @@ __global__ __launch_bounds__(WAVE) void k_lookup_f32_cell(ModelView M, BatchView
       }
     }
     float4 dpart;
-    ep = cell_interp<PART>(ec, dep, deu, cc.y, cc.z, cc.w, ds.x, ds.y, ds.z, dpart);
+    ep = cell_interp<PART, true>(ec, dep, deu, cc.y, cc.z, cc.w, ds.x, ds.y, ds.z, ep, rest, dpart);
     if (wr) {
       st32(outb, (unsigned)ip * WAVE + ln, ep);
       if (PART) st32(partb, (unsigned)ip * WAVE + ln, dpart);
