@@ -340,7 +340,7 @@ __device__ __forceinline__ LkPart lookup_partials_f32(const TabView &T, int tix,
       e = col_eps_bis_vs(col, n, u + x, se);
       de = se * su;
     } else {
-      e = ep + ega_step_slow<true>(col, n, ep, x, gi[c], de, se);
+      e = ep + ega_step_slow<true>(col, n, ep, 0.f, x, gi[c], de, se);
     }
     ec[c] = e;
     dep += cw[c] * de;

@@ -274,7 +274,7 @@ __global__ __launch_bounds__(WAVE, 4) void k_lookup_f32(ModelView M, BatchView B
         // the corner's column of the table and its knot 0
         auto column = [&](int c) { return (c < 2 ? tq0 + it0 : tq0 + T.TT + it1) + (c & 1); };
         auto knot0 = [&](int c) { return column(c) * T.TS + 1; };
-        const float us = (float)useg;
+        const float us = (float)useg, key = ega_key<PART>(ep, rest);
         float e1[NC], dep1[NC], deu1[NC];
         float4 ka[NC];
         float2 kb[NC];
@@ -296,7 +296,7 @@ __global__ __launch_bounds__(WAVE, 4) void k_lookup_f32(ModelView M, BatchView B
           for (int c = 0; c < NC; c++) {
             bool ok;
             if (CGA) cga_step_fast(ka[c], kb[c], cu, (float)cu, gi[c], e1[c], ok);
-            else ega_step_fast<PART>(ka[c], kb[c], ep, us, gi[c], e1[c], dep1[c], deu1[c], ok);
+            else ega_step_fast<PART>(ka[c], kb[c], ep, rest, key, us, gi[c], e1[c], dep1[c], deu1[c], ok);
             bad |= ok ? 0 : 1 << c;
           }
         }
@@ -317,7 +317,7 @@ __global__ __launch_bounds__(WAVE, 4) void k_lookup_f32(ModelView M, BatchView B
             e = eps_from_rec_f(r, cu);
             if ((float)cu < r.x) g = -1;
           } else {
-            e = ega_step_slow<PART>(col, n, ep, useg, g, de, du);
+            e = ega_step_slow<PART>(col, n, ep, rest, useg, g, de, du);
           }
 #pragma unroll
           for (int q = 0; q < NC; q++)
@@ -469,16 +469,16 @@ __global__ __launch_bounds__(WAVE) void k_lookup_f32_cell(ModelView M, BatchView
     const float4 dn = PART ? ld32(cellb, (ipn * WAVE + ln) * CW + 1) : ds;
     const double un = LOSR(fu, ipn);
     __builtin_amdgcn_sched_barrier(0);
-    const float us = (float)useg;
+    const float us = (float)useg, key = ega_key<PART>(ep, rest);
     float e1[NC], dep1[NC], deu1[NC];
     int bad = 0;
 #pragma unroll
     for (int c = 0; c < NC; c++) {
       bool ok;
       dep1[c] = deu1[c] = 0.f;
-      ega_step_fast<PART>(ka[c], kb[c], ep, us, gi[c], e1[c], dep1[c], deu1[c], ok);
+      ega_step_fast<PART>(ka[c], kb[c], ep, rest, key, us, gi[c], e1[c], dep1[c], deu1[c], ok);
       if (!ok) {
-        if (ega_above(ka[c], kb[c], ep)) e1[c] = ega_step_above<PART>(ka[c].z, ka[c].w, ep, us, dep1[c], deu1[c]);
+        if (ega_above<PART>(ka[c], kb[c], ep, rest)) e1[c] = ega_step_above<PART>(ka[c].z, ka[c].w, ep, us, dep1[c], deu1[c]);
         else bad |= 1 << c;
       }
     }
@@ -490,7 +490,7 @@ __global__ __launch_bounds__(WAVE) void k_lookup_f32_cell(ModelView M, BatchView
       if constexpr (RL == 1) g = pick(gi, c);
       else g = gi[0];
       float de, du;
-      const float e = ega_step_slow<PART>(Col{knb + ((unsigned)q * TS + 1)}, nub[q], ep, useg, g, de, du);
+      const float e = ega_step_slow<PART>(Col{knb + ((unsigned)q * TS + 1)}, nub[q], ep, rest, useg, g, de, du);
 #pragma unroll
       for (int k = 0; k < NC; k++)
         if (k == c) {

@@ -412,3 +412,41 @@ def test_adjoint_path_batch_regimes_agree(gpu):
     k0, k1 = out[0][1], out[1][1]
     assert np.isfinite(k0).all() and np.abs(k0).max() > 0
     np.testing.assert_allclose(k1, k0, rtol=1e-12, atol=1e-12 * np.abs(k0).max())
+
+
+def _device_jacobian(gpu, ctl, batch, precision, torch):
+    """K, radiances and transmittances of a _nadir_batch: ([ray][channel][n],
+    [ray][channel] twice)."""
+    atms, a_d, prof_d, geom_d, nray = batch
+    xm, n = gpu.state_map(ctl, atms[0])
+    rad = torch.zeros(nray, ctl.nd, dtype=torch.float64, device="cuda:0")
+    tau = torch.zeros_like(rad)
+    k = torch.zeros(nray, ctl.nd, n, dtype=torch.float64, device="cuda:0")
+    pmap = torch.zeros(len(atms), dtype=torch.int32, device="cuda:0")
+    ctx = gpu.Context(ctl)
+    try:
+        ctx.jacobian_device(len(atms), a_d.data_ptr(), nray, prof_d.data_ptr(), geom_d.data_ptr(), rad.data_ptr(),
+                            tau.data_ptr(), xm[None, :], pmap.data_ptr(), n, k.data_ptr(), precision=precision)
+        torch.cuda.synchronize()
+    finally:
+        ctx.close()
+    return k.cpu().numpy(), rad.cpu().numpy(), tau.cpu().numpy()
+
+
+def test_fp32_partials_at_knots(gpu):
+    """FP32 K against FP64 K, by state block.  The partials jump where a path
+    meets a knot of a table; one ray here (atmosphere 30, 14 degrees) has a
+    CO2 path 0.8 float ulp from one.  On the wrong side of a knot the slope
+    is off by 1.149^0.2 - 1 = 2.8% (knots a factor 1.149 apart, eps ~ u^0.8)
+    times the corner's weight in its cell: one such ray of the 512 gives
+    0.028 x 0.6 / sqrt(512) = 7e-4 of a block's norm where it begins at the
+    ground, less above.  The bound is 1/20 of that, and some thirty times the
+    rounding of the float partials (1e-6)."""
+    torch = pytest.importorskip("torch")
+    ctl = scenes.nadir_jac_ctl(4)
+    batch = _nadir_batch(ctl, 64, 8, torch)
+    k32, k64 = (_device_jacobian(gpu, ctl, batch, p, torch)[0] for p in (abi.JUR_FP32, abi.JUR_FP64))
+    for b, name in enumerate(["T", "CO2", "H2O", "O3"]):
+        s = slice(81 * b, 81 * b + 81)
+        err = np.linalg.norm(k32[..., s] - k64[..., s]) / np.linalg.norm(k64[..., s])
+        assert err < 3e-5, (name, err)
