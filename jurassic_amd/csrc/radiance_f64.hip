@@ -39,14 +39,16 @@ __global__ __launch_bounds__(WAVE *PW) void k_radiance_f64(ModelView M, BatchVie
   const int lane = threadIdx.x % WAVE;
   const int wv = PW == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
   // lanes without a ray follow the last one (the waves meet at barriers) and
-  // write nothing
+  // write nothing, as do rays that could not be traced, whose atmosphere index
+  // may be out of range: they read the first atmosphere
   const bool live = (blk0 + bl) * WAVE + lane < B.nray;
   const int ir = live ? (blk0 + bl) * WAVE + lane : B.nray - 1;
   RayInfo R = info[ir];
-  const bool write = live && R.status == JUR_OK && wv == 0;
-  if (!live || R.status != JUR_OK) R.np = 0;
+  const bool ok = live && R.status == JUR_OK;
+  const bool write = ok && wv == 0;
+  if (!ok) R.np = 0;
 
-  const atm_t *atm = &B.atm[B.ray_prof[ir]];
+  const atm_t *atm = &B.atm[ok ? B.ray_prof[ir] : 0];
   const ChanInfo C = M.chan[id];
   const double nu = C.nu;
   const double *los = L.los + (size_t)bl * L.cap * L.nfield * WAVE + lane;

@@ -633,3 +633,60 @@ def test_radiance_waves_per_path_agree(gpu, nr):
         for k in (0, n // 2, n - 1):
             r1, t1 = abi.obs_arrays(obss[k], ctl)
             assert np.array_equal(r0, r1) and np.array_equal(t0, t1), (prec, k)
+
+
+@pytest.mark.parametrize("nray", [3, 5600])
+def test_bad_atmosphere_index(gpu, nray):
+    """A device batch whose rays name atmospheres that are not there, with
+    clouds and surface emissivities on (read per ray before any of its
+    points): JUR_ERR_ARG from the forward model and the Jacobian, in batches
+    on several waves per path and on one, and a good call afterwards.  The
+    last ray is a bad one: the lanes behind it in its block follow it."""
+    torch = pytest.importorskip("torch")
+    ctl = scenes.limb_3gas_ctl()
+    ctl.ncl, ctl.nsf, ctl.sftype = 2, 2, 2
+    for i in range(2):
+        ctl.clnu[i], ctl.sfnu[i] = (600.0, 1600.0)[i], (600.0, 1600.0)[i]
+    ctl.rett_zmin, ctl.rett_zmax = -100, 100
+    atms = (abi.atm_t * 2)()
+    for k in range(2):
+        atms[k] = scenes.make_profile_atm(["CO2", "H2O", "O3"], iprof=k)
+        atms[k].clz, atms[k].cldz, atms[k].sft = 8.0, 1.5, 290.0
+        for i in range(2):
+            atms[k].clk[i], atms[k].sfeps[i] = 0.02, 0.8
+    dev = torch.device("cuda:0")
+    a_d = torch.from_numpy(np.frombuffer(bytes(atms), dtype=np.uint8).copy()).to(dev)
+    one = scenes.nadir_geometry(705.0, [20.0])
+    geom = torch.zeros(nray, 7, dtype=torch.float64)
+    for c, key in enumerate(("obsz", "obslon", "obslat", "vpz", "vplon", "vplat")):
+        geom[:, 1 + c] = float(one[key][0])
+    geom = geom.to(dev)
+    good = (torch.arange(nray, dtype=torch.int32) % 2).to(dev)
+    bad = good.clone()
+    bad[0], bad[nray - 1] = -1, 2
+    xm, n = gpu.state_map(ctl, atms[0])
+    pmap = torch.zeros(2, dtype=torch.int32, device=dev)
+    rad = torch.zeros(nray, ctl.nd, dtype=torch.float64, device=dev)
+    tau = torch.zeros_like(rad)
+    k = torch.zeros(3, ctl.nd, n, dtype=torch.float64, device=dev)
+    ctx = gpu.Context(ctl)
+    try:
+        for prec in (abi.JUR_FP64, abi.JUR_FP32):
+            def call(prof):
+                ctx.formod_device(2, a_d.data_ptr(), nray, prof.data_ptr(), geom.data_ptr(), rad.data_ptr(),
+                                  tau.data_ptr(), precision=prec)
+
+            def jac(prof):
+                ctx.jacobian_device(2, a_d.data_ptr(), 3, prof.data_ptr(), geom.data_ptr(), rad.data_ptr(),
+                                    tau.data_ptr(), xm[None, :], pmap.data_ptr(), n, k.data_ptr(), precision=prec)
+            for f in (call, jac) if nray == 3 else (call,):
+                with pytest.raises(gpu.JurassicError) as e:
+                    f(bad)
+                assert e.value.code == abi.JUR_ERR_ARG
+            call(good)
+            torch.cuda.synchronize()
+            assert bool((rad > 0).all()) and bool(torch.isfinite(rad).all())
+            # rays of one atmosphere and geometry agree, the last one too
+            assert bool((rad[nray - 1] == rad[(nray - 1) % 2]).all())
+    finally:
+        ctx.close()
