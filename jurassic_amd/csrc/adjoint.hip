@@ -564,7 +564,15 @@ __device__ __forceinline__ double level_val(const atm_t *atm, int qi, int l) {
   return qi == 0 ? atm->p[l] : (qi == 1 ? atm->t[l] : (qi < 2 + NG ? atm->q[qi - 2][l] : atm->k[qi - 2 - NG][l]));
 }
 
-template <int NQ, unsigned ATOM = 0, bool CCOL = true, bool PATH = false>
+// Quantities in BOX are handed on at a flush: their sums and K columns are put
+// in the lane's slots of a LevelBox, from which another wavefront adds them to
+// the tile.
+struct LevelBox {
+  int *c;     // K columns of the pair's levels, [quantity][2], a wavefront apart
+  double *v;  // their sums
+};
+
+template <int NQ, unsigned ATOM = 0, bool CCOL = true, bool PATH = false, unsigned BOX = 0>
 struct LevelWindow {
   int wa = -1;
   double z0 = 0, z1 = 0, rz = 0, P0 = 0, P1 = 0, rp0 = 0, rp1 = 0;
@@ -572,7 +580,7 @@ struct LevelWindow {
   double acc[NQ][2];
   double sl[NQ];   // PATH: slope of each quantity in the pair (p: of log p, or of p)
   int col[NQ][2];  // K columns of the pair's levels (loaded when the pair is entered)
-  __device__ __forceinline__ void flush(const int *xm, const int *qi, double *kt) {
+  __device__ __forceinline__ void flush(const int *xm, const int *qi, double *kt, LevelBox box = {}) {
     if (wa < 0) return;
 #pragma unroll
     for (int k = 0; k < 2; k++)
@@ -580,6 +588,11 @@ struct LevelWindow {
       for (int q = 0; q < NQ; q++) {
         if (qi[q] < 0) continue;
         const int c = CCOL ? col[q][k] : xm[JUR_XMAP_LEV(qi[q], wa + k)];
+        if (BOX >> q & 1u) {
+          box.c[(2 * q + k) * WAVE] = c;
+          box.v[(2 * q + k) * WAVE] = acc[q][k];
+          continue;
+        }
         if (c < 0) continue;
         if (ATOM >> q & 1u) unsafeAtomicAdd(&kt[(size_t)c * WAVE], acc[q][k]);
         else kt[(size_t)c * WAVE] += acc[q][k];
@@ -589,7 +602,7 @@ struct LevelWindow {
   // weights p/p_level, src/jurassic.c:3685-3706), the others use the LIN
   // weights.
   __device__ __forceinline__ double add(const atm_t *atm, double z, int &lev, const double *v, int qp, double p,
-                                        const int *xm, const int *qi, double *kt) {
+                                        const int *xm, const int *qi, double *kt, LevelBox box = {}) {
     if (!(wa >= 0 && z0 <= z && z < z1)) {
       // the pair locate_irr returns: a neighbour of the current pair (with
       // its clamps at the first and last pair), else a search
@@ -645,7 +658,7 @@ struct LevelWindow {
         }
       }
       if (nl != wa) {
-        flush(xm, qi, kt);
+        flush(xm, qi, kt, box);
         wa = nl;
 #pragma unroll
         for (int q = 0; q < NQ; q++) {
@@ -1284,7 +1297,8 @@ __global__ __launch_bounds__(WAVE) void k_path_coef(ModelView M, BatchView B, Lo
 // of the state, the level window, and the clip of the last step.  Level sums
 // are kept for a window of three levels (the step's LB and the two above)
 // per channel and added to the K tile when the window moves.
-// ATOM: atomic adds, where another wave adds to the same tile row meanwhile.
+// ATOM: atomic adds without return, which do not wait for the tile's value (the
+// wave is the only one that adds to these columns).
 template <int CH, bool ATOM = false>
 struct PathRev {
   const int *xm;
@@ -1813,8 +1827,10 @@ __global__ __launch_bounds__(WAVE) void k_adj_acc(ModelView M, BatchView B, LosV
 //     the reverse march of the refracted path, whose coefficients it copies
 //     into LDS a step ahead.
 // All lanes of the workgroup are at the same point (a lane begins at its own
-// last one), so a step's coefficients are one contiguous copy.  Wave 1 adds
-// to the T and p columns that wave 3 adds to: both add atomically.
+// last one), so a step's coefficients are one contiguous copy.  The T and p
+// columns get the path's sums from wave 1 and the levels' from wave 3, which
+// hands its own to wave 1 (LevelBox): one wave adds them, so K is the same
+// bits on each call.
 //
 // Bound by the slowest stage's chain of FP64 operations.  64 x 32 x 12 limb
 // rows: 7.9 ms when one wave ran the two sweeps with everything in the
@@ -1861,9 +1877,11 @@ __global__ __launch_bounds__(4 * WAVE, 2) void k_adj_row(ModelView M, BatchView 
   constexpr int NQW = 3 + EM;  // level quantities: T, p, the window's extinction, every emitter's q
   // LDS: the forward sweep's segments; then, two buffers each, the terms, the
   // point adjoints (with the rest of d rad / d z_i and d rad / d ds_i), the
-  // path's point values, and two steps' coefficients
-  constexpr int N_TERM = 2 * ROW_TERMS, N_V = 2 * (NQW + 2), N_GZ = 2 * 2, N_PC = PATH ? 2 * JUR_NPCO : 0;
-  constexpr int N_FWD = 4 * ROW_FP * 2, N_REV = N_TERM + N_V + N_GZ + N_PC;
+  // path's point values, the sums over T and p handed to wave 1, and two
+  // steps' coefficients
+  constexpr int N_TERM = 2 * ROW_TERMS, N_V = 2 * (NQW + 2), N_GZ = 2 * 2, N_BOX = PATH ? 2 * 6 : 0;
+  constexpr int N_PC = PATH ? 2 * JUR_NPCO : 0;
+  constexpr int N_FWD = 4 * ROW_FP * 2, N_REV = N_TERM + N_V + N_GZ + N_BOX + N_PC;
   __shared__ double lds[(N_REV > N_FWD ? N_REV : N_FWD) * WAVE];
   __shared__ int s_nef[WAVE];
 #define LD(i) lds[(i) * WAVE + lane]
@@ -1988,6 +2006,11 @@ __global__ __launch_bounds__(4 * WAVE, 2) void k_adj_row(ModelView M, BatchView 
 #define TERM(r, k) LD(((r) & 1) * ROW_TERMS + (k))
 #define VAL(r, k) LD(N_TERM + ((r) & 1) * (NQW + 2) + (k))
 #define GZ(r, k) LD(N_TERM + N_V + ((r) & 1) * 2 + (k))
+  auto box = [&](int r) {
+    double *b = lds + (size_t)(N_TERM + N_V + N_GZ + (r & 1) * 6) * WAVE;
+    return LevelBox{(int *)(b + 4 * WAVE) + lane, b + lane};
+  };
+  constexpr int BOX_EMPTY = -2;  // first column of a box: no flush in this round
 
   if (role == 2) {
     // ---------------- the segments' terms and gradients ----------------
@@ -2026,11 +2049,12 @@ __global__ __launch_bounds__(4 * WAVE, 2) void k_adj_row(ModelView M, BatchView 
     qi[2] = has_k ? 2 + NG + C.window : -1;
 #pragma unroll
     for (int g = 0; g < EM; g++) qi[3 + g] = g < ng ? 2 + g : -1;
-    LevelWindow<NQW, (1u << NQW) - 1u, true, PATH> W;
+    LevelWindow<NQW, (1u << NQW) - 1u, true, PATH, PATH ? 3u : 0u> W;
     int lev = -1;
     double zn = hi > 0 ? LOSR(F_Z, hi - 1) : 0, pn = hi > 0 ? LOSR(F_P, hi - 1) : 0;
     for (int r = 0; r < nround; r++) {
       const int ip = hi - 1 - (r - 2);
+      if (PATH && r >= 2) box(r).c[0] = BOX_EMPTY;
       if (r >= 2 && ip >= 0) {
         const double z = zn, p = pn;
         if (ip > 0) {
@@ -2041,16 +2065,16 @@ __global__ __launch_bounds__(4 * WAVE, 2) void k_adj_row(ModelView M, BatchView 
           double v[NQW];
 #pragma unroll
           for (int q = 0; q < NQW; q++) v[q] = VAL(r, q);
-          const double gz = W.add(atm, z, lev, v, 1, p, xm, qi, kt);
+          const double gz = W.add(atm, z, lev, v, 1, p, xm, qi, kt, box(r));
           if (PATH) {
             GZ(r, 0) = gz + VAL(r, NQW);
             GZ(r, 1) = VAL(r, NQW + 1);
           }
         }
       }
+      if (r == nround - 1 && map) W.flush(xm, qi, kt, box(r));
       __syncthreads();
     }
-    if (map) W.flush(xm, qi, kt);
     return;
   }
 
@@ -2063,7 +2087,17 @@ __global__ __launch_bounds__(4 * WAVE, 2) void k_adj_row(ModelView M, BatchView 
     P.kt0 = kt;
     P.ktstride = (size_t)J.ncol * WAVE;
     const char *pcg = PATH ? (const char *)(J.pco + J.soff[bl] / ((size_t)nd * J.nscr) * JUR_NPCO) : nullptr;
-    double *pcs = lds + (size_t)(N_TERM + N_V + N_GZ) * WAVE;
+    double *pcs = lds + (size_t)(N_TERM + N_V + N_GZ + N_BOX) * WAVE;
+    // the level sums that wave 3 handed on in round r
+    auto add_box = [&](int r) {
+      const LevelBox b = box(r);
+      if (b.c[0] == BOX_EMPTY) return;
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        const int c = b.c[j * WAVE];
+        if (c >= 0) unsafeAtomicAdd(&KT(c), b.v[j * WAVE]);
+      }
+    };
     // step k's coefficients into buffer k & 1, which step k + 2 has been read
     // from (its reads have completed: the memory clobber keeps the compiler
     // from moving them below the copy, whose LDS write it does not see)
@@ -2088,6 +2122,7 @@ __global__ __launch_bounds__(4 * WAVE, 2) void k_adj_row(ModelView M, BatchView 
         // the reads below the wait); then the next step's are sent for
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         if (ip > 0) pc_fetch(ip - 1);
+        add_box(r - 1);
         const double gzc = GZ(r - 1, 0), gdc = GZ(r - 1, 1);
         if (ip < ne && ip == N - 1) {
           gz_last = gzc;
@@ -2109,6 +2144,7 @@ __global__ __launch_bounds__(4 * WAVE, 2) void k_adj_row(ModelView M, BatchView 
       }
       __syncthreads();
     }
+    if (PATH) add_box(nround - 1);
     if (PATH && pstart) P.finish();
     return;
   }
@@ -2153,7 +2189,12 @@ __global__ __launch_bounds__(4 * WAVE, 2) void k_adj_row(ModelView M, BatchView 
   if (sft_los) {
     lv_sf = level_of(atm, LOSR(F_Z, N - 1), -1, w_sf);
     gz_sft = sft_bar * (atm->t[lv_sf + 1] - atm->t[lv_sf]) / (atm->z[lv_sf + 1] - atm->z[lv_sf]);
+    // its T columns, before the other waves add to them (from round 2 on)
+    int c;
+    if (map && (c = xm[JUR_XMAP_LEV(1, lv_sf)]) >= 0) unsafeAtomicAdd(&KT(c), (1 - w_sf) * sft_bar);
+    if (map && (c = xm[JUR_XMAP_LEV(1, lv_sf + 1)]) >= 0) unsafeAtomicAdd(&KT(c), w_sf * sft_bar);
   }
+  __threadfence();
 
   // ---------------- wave 0: the accumulation's and the chains' reverse ----------------
   double clz_bar = 0, cldz_bar = 0, clk_bar = 0, Hn = 0;
@@ -2258,16 +2299,11 @@ __global__ __launch_bounds__(4 * WAVE, 2) void k_adj_row(ModelView M, BatchView 
   }
   if (!ok || !map) return;
 
-  // surface terms (T columns: the other waves add to them too)
+  // surface terms
   if (surf) {
     if (M.nsf > 0 && atm->sft > 0) {
       const int c = xm[JUR_XMAP_SFT];
       if (c >= 0) KT(c) += sft_bar;
-    } else if (sft_los) {
-      // the surface temperature is the LOS temperature of the last point
-      int c;
-      if ((c = xm[JUR_XMAP_LEV(1, lv_sf)]) >= 0) unsafeAtomicAdd(&KT(c), (1 - w_sf) * sft_bar);
-      if ((c = xm[JUR_XMAP_LEV(1, lv_sf + 1)]) >= 0) unsafeAtomicAdd(&KT(c), w_sf * sft_bar);
     }
     if (M.nsf > 0) {
       int c;

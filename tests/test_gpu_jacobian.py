@@ -450,3 +450,21 @@ def test_fp32_partials_at_knots(gpu):
         s = slice(81 * b, 81 * b + 81)
         err = np.linalg.norm(k32[..., s] - k64[..., s]) / np.linalg.norm(k64[..., s])
         assert err < 3e-5, (name, err)
+
+
+@pytest.mark.parametrize("refrac", [0, 1])
+def test_fp32_jacobian_repeats(gpu, refrac):
+    """The FP32 Jacobian of up to four emitters is the same bits on each
+    call, though several waves share a row: every column of K has one wave
+    that adds to it.  Views from nadir to grazing, with the surface
+    temperature taken from the profile (nsf = 0), 512 rows of each kind of
+    atmosphere."""
+    torch = pytest.importorskip("torch")
+    ctl = scenes.nadir_jac_ctl(8)
+    ctl.refrac, ctl.sftype = refrac, 1
+    ctl.retp_zmin, ctl.retp_zmax = -100, 100
+    batch = _nadir_batch(ctl, 64, 8, torch)
+    k0 = _device_jacobian(gpu, ctl, batch, abi.JUR_FP32, torch)[0]
+    assert np.isfinite(k0).all() and np.abs(k0).max() > 0
+    for _ in range(5):
+        assert np.array_equal(_device_jacobian(gpu, ctl, batch, abi.JUR_FP32, torch)[0], k0)
