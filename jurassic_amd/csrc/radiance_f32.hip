@@ -18,9 +18,10 @@
 //   division costs about ten instructions, and radiances move by a few
 //   float ulp.
 //
-// Large batches stream (7.5 ms per 4096 x 32 x 12 limb batch); a small one
-// lasted as long as one path on one wave, 1.16 ms for limb paths of 1530
-// points, and takes 0.15 ms on 16 waves per path.
+// Large batches stream: 3.9 ms per 2048 x 32 x 12 limb batch, on four
+// wavefronts per SIMD (the compiler's own choice of registers leaves three: 4.5
+// ms).  A small one lasted as long as one path on one wave, 1.16 ms for limb
+// paths of 1530 points, and takes 0.15 ms on 16 waves per path.
 #include "jur_device.hpp"
 
 namespace jur {
@@ -28,7 +29,7 @@ namespace jur {
 #define LOSR(f, ip) LOS_AT(los, L, f, ip)
 
 template <int PW>
-__global__ __launch_bounds__(WAVE *PW) void k_radiance_f32(ModelView M, BatchView B, LosView L,
+__global__ __launch_bounds__(WAVE *PW, 4) void k_radiance_f32(ModelView M, BatchView B, LosView L,
                                                        EpsView E, const RayInfo *info, int blk0,
                                                        int nblk, double *rad_out, double *tau_out) {
   const int nd = M.nd, ng = M.ng;
@@ -126,6 +127,9 @@ __global__ __launch_bounds__(WAVE *PW) void k_radiance_f32(ModelView M, BatchVie
   unsigned gmask = 0;
   for (int g = 0; g < ng; g++)
     if (M.tab.np[g * nd + id] >= 30) gmask |= 1u << g;
+
+  // the down-welling sum is used only where the surface reflects
+  const bool refl = M.sftype >= 2 && M.nsf > 0;
 
   PathSum sum;
   float epp[NG];  // path emissivity of each emitter before the segment
@@ -242,7 +246,7 @@ __global__ __launch_bounds__(WAVE *PW) void k_radiance_f32(ModelView M, BatchVie
     const double ed = (double)e, sd = (double)src, d = tau * ed;
     rad += sd * d;
     tau -= d;
-    drefl = drefl - drefl * ed + sd * ed;
+    if (refl) drefl = drefl - drefl * ed + sd * ed;
     load_src(tn);
   }
   PathSum::join<PW>(sum, part, wv, lane,
