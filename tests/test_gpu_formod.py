@@ -611,28 +611,51 @@ def test_level_grids(gpu, oracle, nlev, up, refrac):
 
 @pytest.mark.parametrize("nr", [1, 63, 65])
 def test_radiance_waves_per_path_agree(gpu, nr):
-    """A small batch forms a path's segments on several waves (16 or 8 per
-    path), a large one on one: the same bits for one package of 1, 63 or 65
+    """A small batch forms a path's segments on several waves (FP32 16 or 4,
+    FP64 8), a large one on one: the same bits for one package of 1, 63 or 65
     rays (a block with one lane, one short, two blocks) and for it among
-    copies of itself that fill more blocks than the small launches take."""
+    copies of itself that make 19 blocks x 12 channels (more than the 256
+    workgroups of the FP32 launch with 16 waves, with the rounding to eight
+    blocks) and 100 x 12 (more than the 1024 with 4 and the 512 with 8).  Limb
+    paths and, every other ray, paths to a reflecting surface (emissivity
+    0.8), where the down-welling sum enters the radiance: it moves there by
+    more than 1e-6 with the emissivity."""
     ctl = scenes.limb_3gas_ctl()
-    ctl.sftype = 2
+    ctl.sftype, ctl.nsf = 2, 2
+    ctl.sfnu[0], ctl.sfnu[1] = 600.0, 1600.0
     atm = scenes.make_profile_atm(["CO2", "H2O", "O3"], iprof=2)
-    geom = scenes.limb_geometry(800.0, np.linspace(-5.0, 60.0, nr) if nr > 1 else np.array([11.0]))
-    n = -(-5000 // nr) if nr > 1 else 5000
+    atm.sft = 290.0
+    limb = scenes.limb_geometry(800.0, np.linspace(5.0, 60.0, nr))
+    down = scenes.nadir_geometry(800.0, np.linspace(0.0, 50.0, nr))
+    geom = {k: np.where(np.arange(nr) % 2 == 1, limb[k], down[k]) for k in limb}
     for prec in (abi.JUR_FP64, abi.JUR_FP32):
-        one = scenes.make_obs(geom)
-        gpu.formod(ctl, abi.copy_struct(atm), one, prec)
-        atms, obss = (abi.atm_t * n)(), (abi.obs_t * n)()
-        for k in range(n):
-            atms[k] = atm
-            obss[k] = scenes.make_obs(geom)
-        gpu.formod_batch(ctl, atms, obss, prec)
-        r0, t0 = abi.obs_arrays(one, ctl)
+        ref = {}
+        for eps in (1.0, 0.8):
+            atm.sfeps[0] = atm.sfeps[1] = eps
+            one = scenes.make_obs(geom)
+            gpu.formod(ctl, abi.copy_struct(atm), one, prec)
+            ref[eps] = abi.obs_arrays(one, ctl)
+        r0, t0 = ref[0.8]
         assert np.isfinite(r0).all() and (r0 > 0).any()
-        for k in (0, n // 2, n - 1):
-            r1, t1 = abi.obs_arrays(obss[k], ctl)
-            assert np.array_equal(r0, r1) and np.array_equal(t0, t1), (prec, k)
+        # with an emissivity below 1 the emission falls by (1 - eps) src tau
+        # and the reflection adds (1 - eps) D tau: both enter if the change
+        # is neither zero nor the emission's alone
+        c1, c2 = 1.19104259e-8, 1.43877506
+        nu = np.array([ctl.nu[i] for i in range(ctl.nd)])[:, None]
+        emis = -0.2 * c1 * nu ** 3 / np.expm1(c2 * nu / 290.0) * t0
+        change = r0 - ref[1.0][0]
+        k = np.arange(0, nr, 2)
+        assert (np.abs(change - emis)[:, k].max(axis=1) > 1e-6 * r0[:, k].max(axis=1)).any()
+        for blocks in (19, 100):
+            n = -(-64 * blocks // nr)
+            atms, obss = (abi.atm_t * n)(), (abi.obs_t * n)()
+            for q in range(n):
+                atms[q] = atm
+                obss[q] = scenes.make_obs(geom)
+            gpu.formod_batch(ctl, atms, obss, prec)
+            for q in (0, n // 2, n - 1):
+                r1, t1 = abi.obs_arrays(obss[q], ctl)
+                assert np.array_equal(r0, r1) and np.array_equal(t0, t1), (prec, blocks, q)
 
 
 @pytest.mark.parametrize("nray", [3, 5600])
