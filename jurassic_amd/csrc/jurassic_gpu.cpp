@@ -710,10 +710,10 @@ int forward_pass(jur_ctx *c, const BatchView &B, int precision, const unsigned c
     // radiance kernel reads)
     const bool losf = precision == JUR_FP32 && !jac;
     // FP32 EGA over tables of one grid: each point's cell, located once
-    const bool cells = precision == JUR_FP32 && M.formod != 0 && M.tab.cells;
+    bool cells = precision == JUR_FP32 && M.formod != 0 && M.tab.cells;
     L.ncell = part ? 2 : 1;
-    const size_t los_blk = (size_t)L.nfield * L.cap * WAVE * (sizeof(double) + (losf ? sizeof(float) : 0)) +
-                           (cells ? (size_t)L.ncell * L.cap * WAVE * sizeof(float4) : 0);
+    size_t los_blk = (size_t)L.nfield * L.cap * WAVE * (sizeof(double) + (losf ? sizeof(float) : 0));
+    const size_t cell_blk = (size_t)L.ncell * L.cap * WAVE * sizeof(float4);
     const size_t pt_blk = (size_t)s.nd * s.ng * WAVE * (esz + (part ? sizeof(float4) : 0)) +
                           (jac ? (size_t)s.nd * nscr * WAVE * sizeof(double) : 0) +
                           (dpath ? (size_t)JUR_NPCO * WAVE * sizeof(double) : 0);
@@ -724,6 +724,10 @@ int forward_pass(jur_ctx *c, const BatchView &B, int precision, const unsigned c
       // offset arrays and the alignment of the slices
       const size_t small = (size_t)nblk * (sizeof(int) + 2 * sizeof(size_t)) + 16 * 256;
       budget = pm.cap - pm.used > small ? pm.cap - pm.used - small : 0;
+      // the cells only where a block still fits with them at the full LOS
+      // capacity (half of the budget is for the LOS of a chunk): a call that
+      // fits without them is not refused, and its lookups locate their own
+      cells = cells && std::max(los_blk + cell_blk, budget / 2) + L.cap * pt_blk + 6 * 256 <= budget;
     } else if (budget == 0) {
       // half of the HBM free now (plus what these buffers already hold), at
       // most 96 GiB.  A pass of another kind divides the budget otherwise
@@ -749,6 +753,7 @@ int forward_pass(jur_ctx *c, const BatchView &B, int precision, const unsigned c
             (c->d_kt.n + c->d_scr.n + c->d_pco.n) * sizeof(double);
       budget = std::min(fr / 2, (size_t)96 << 30);
     }
+    if (cells) los_blk += cell_blk;
     // Rays are traced in chunks whose LOS takes at most half the budget; the
     // lookups and the radiance (or adjoint) pass then run over sub-chunks of
     // a chunk sized by the blocks' actual LOS lengths.

@@ -2,8 +2,9 @@
 memory (its work buffers are slices of the library's fixed scratch array),
 against jur_ctx_formod_device on the same batches: bit-identical radiances,
 transmittances and tangent points, FP64 and FP32, on two calls in a row
-(the second smaller), and a clean JUR_ERR_MEM for a batch whose per-ray
-buffers exceed the array, after which calls still work.  Through the C-ABI.
+(the second smaller), a batch that fills the array, and a clean JUR_ERR_MEM
+for a batch whose per-ray buffers exceed it, after which calls still work.
+Through the C-ABI.
 """
 import ctypes as C
 
@@ -95,3 +96,45 @@ def test_noalloc_rejects_batch_beyond_scratch(gpu):
         assert all(np.array_equal(r, g) for r, g in zip(ref, got))
     finally:
         ctx.close()
+
+
+def test_noalloc_full_scratch(gpu):
+    """One limb ray of 211 channels and three emitters: the emissivities of
+    its block's 1531 points are 211 x 3 x 1531 x 64 x 4 B = 248.1 MB, the LOS
+    at its estimated capacity some 20 MB, together within 0.3 MB of the array.
+    The call fits without the lookups' cell records (2.3 MB) and is taken
+    without them, with the same bits (so is one of 210 channels: the rule
+    counts the estimated capacity, not the points)."""
+    torch = pytest.importorskip("torch")
+    dev = torch.device("cuda:0")
+    ng, tp, tt, tu = 3, 30, 2, 4
+    p = np.exp(np.linspace(np.log(0.01), np.log(1100.0), tp))
+    u = np.array([1e15, 1e20, 1e23, 1e27], dtype=np.float32)
+    eps = np.array([1e-8, 1e-4, 0.1, 0.9], dtype=np.float32)
+    atm = scenes.make_profile_atm(["CO2", "H2O", "O3"], iprof=0)
+    a_d = torch.from_numpy(np.frombuffer(bytes(atm), dtype=np.uint8).copy()).to(dev)
+    g = scenes.limb_geometry(800.0, np.array([5.0]))
+    geom = np.array([[0.0] + [float(g[k][0]) for k in ("obsz", "obslon", "obslat", "vpz", "vplon", "vplat")]])
+    batch = (1, a_d, torch.zeros(1, dtype=torch.int32, device=dev), torch.from_numpy(geom).to(dev), 1)
+    for nd in (210, 211):
+        nu = [650.0 + 5.0 * i for i in range(nd)]
+        i32 = torch.int32
+        tabs = dict(np=torch.full((nd, ng), tp, dtype=i32, device=dev),
+                    nt=torch.full((nd, ng, tp), tt, dtype=i32, device=dev),
+                    nu=torch.full((nd, ng, tp, tt), tu, dtype=i32, device=dev),
+                    p=torch.tensor(p, device=dev).expand(nd, ng, tp).contiguous(),
+                    t=torch.tensor([150.0, 350.0], dtype=torch.float64, device=dev).expand(nd, ng, tp, tt).contiguous(),
+                    u=torch.tensor(u, device=dev).expand(nd, ng, tp, tt, tu).contiguous(),
+                    eps=torch.tensor(eps, device=dev).expand(nd, ng, tp, tt, tu).contiguous())
+        off = 5 * np.arange(nd + 1, dtype=np.int32)
+        xs = np.concatenate([v + np.array([-0.6, -0.5, 0.0, 0.5, 0.6]) for v in nu])
+        filt = (off, xs, np.tile(np.array([0.0, 1.0, 1.0, 1.0, 0.0]), nd))
+        ctl = abi.make_ctl(["CO2", "H2O", "O3"], nu[:1], tblbase="-", tblfmt=2)
+        ctx = gpu.Context.from_device_tables(ctl, nu, tabs, filters=filt)
+        try:
+            ref = _run(torch, ctx, ctx.formod_device, batch, abi.JUR_FP32)
+            assert ctx.last_mean_np() == 1531
+            got = _run(torch, ctx, ctx.formod_device_noalloc, batch, abi.JUR_FP32)
+            assert all(np.array_equal(r, v) for r, v in zip(ref, got)), nd
+        finally:
+            ctx.close()
