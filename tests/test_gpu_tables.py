@@ -307,3 +307,47 @@ def test_cells_equal_general(gpu, tmp_path, nprof):
     assert np.array_equal(out[0][0][:, 1:], out[1][0][:, 1:])
     assert np.array_equal(out[0][1][:, 1:], out[1][1][:, 1:])
     np.testing.assert_allclose(out[1][0][:, 0], out[0][0][:, 0], rtol=1e-5)
+
+
+def test_temperature_on_grid_point(gpu, tmp_path):
+    """An atmosphere at a temperature of the tables' grid: the cell is the one
+    that begins there (the reference truncates (T - T_0) / (T_1 - T_0)).  With
+    a spacing of 24.5 K the product with the reciprocal spacing falls short of
+    the quotient at every second point or so, 98 x (1 / 24.5) < 4 among them;
+    the columns at the temperature below have a single knot, so that the cell
+    below holds no data.  FP64 forward model (EGA; the Curtis-Godson mean of a
+    constant is that constant only to rounding) without continua
+    (whose optical depth at one temperature rounds alike at every point: up to
+    1e-11 of a depth of 30) against the oracle."""
+    torch = pytest.importorskip("torch")
+    import oracle as O
+    ctl = _scene_copy(tmp_path, scenes.limb_3gas_ctl(ctm=False), "node")
+    p, _, u = scenes.table_grids()
+    t = 150.0 + 24.5 * np.arange(9)
+    assert int((t[4] - t[0]) * (1 / (t[1] - t[0]))) == 3 and int((t[4] - t[0]) / (t[1] - t[0])) == 4
+    # weak enough that every emitter's path transmittance stays above 1e-3: it
+    # carries some 1e-16 of rounding from each of the ~1000 points (1 - eps00),
+    # so that 1e-10 of it holds
+    eps = scenes.synthetic_eps(p, t, u, 5e-4)
+    for id_ in range(ctl.nd):
+        for ig in range(ctl.ng):
+            fn = scenes.table_name(ctl.tblbase.decode(), ctl.nu[id_], ctl.emitter[ig].value.decode(), 2)
+            with open(fn, "wb") as f:
+                f.write(struct.pack("<i", len(p)) + np.asarray(p, "<f8").tobytes())
+                for ip in range(len(p)):
+                    f.write(struct.pack("<i", len(t)) + t.astype("<f8").tobytes())
+                    for it in range(len(t)):
+                        n = 1 if it == 3 else len(u)
+                        f.write(struct.pack("<i", n) + u[:n].astype("<f4").tobytes() +
+                                eps[ip, it, :n].astype("<f4").tobytes())
+    atm = scenes.make_profile_atm(["CO2", "H2O", "O3"])
+    abi.np_view(atm.t)[:atm.np] = t[4]
+    obs = scenes.make_obs(scenes.limb_geometry(800.0, scenes.limb_tangent_heights()[::4]))
+    ref = abi.copy_struct(obs)
+    O.formod(ctl, abi.copy_struct(atm), ref)
+    r0, t0 = abi.obs_arrays(ref, ctl)
+    assert (t0 < 0.9).any()
+    gpu.formod(ctl, abi.copy_struct(atm), obs, abi.JUR_FP64)
+    r1, t1 = abi.obs_arrays(obs, ctl)
+    np.testing.assert_allclose(r1, r0, rtol=1e-10, atol=0)
+    np.testing.assert_allclose(t1, t0, rtol=1e-10, atol=1e-300)
