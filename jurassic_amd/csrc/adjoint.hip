@@ -2453,10 +2453,17 @@ static void launch_adj(const ModelView &M, const BatchView &B, const LosView &L,
   const int nb8 = padded_blocks(nblk);
   // FP32 EGA with stored partials and at most four emitters: one workgroup per
   // row (k_adj_row), up to some 16 rounds of them (512 run at once).  Whole
-  // Jacobian passes, row form against the kernels below: 3072 rows of nadir
-  // paths 20.7 / 23.2 ms, 6144 40.3 / 41.7, 6144 of limb paths 27.4 / 31.0,
-  // but 12,288 of nadir paths 78.0 / 71.0 (the four waves share a CU's
-  // registers with one other workgroup, which hides less of HBM's latency).
+  // Jacobian passes, row form and the kernels below, ms:
+  //   rows                            3072          6144          7680 / 8064
+  //   nadir, 3 emitters            20.5 / 22.4   40.5 / 40.4   49.8 / 52.1
+  //   nadir, 4 emitters            23.1 / 24.4   44.4 / 45.1   55.5 / 58.5
+  //   nadir, 3, no refraction      14.0 / 14.9   26.7 / 26.6   32.9 / 34.1
+  //   limb, 3 emitters             27.1 / 29.7   51.9 / 55.0   68.4 / 73.4
+  //   limb, 4 emitters             28.9 / 32.2   56.1 / 60.3   75.2 / 80.7
+  //   limb, 3, no refraction                     32.5 / 33.5   42.6 / 43.0
+  // and 78.0 / 71.0 for 12,288 rows of nadir paths (the four waves share a
+  // CU's registers with one other workgroup, which hides less of HBM's
+  // latency).
   bool row = false;
   if constexpr (!CGA && sizeof(SF) == sizeof(float)) row = E.part && M.ng >= 1 && M.ng <= 4 && nb8 * M.nd < 8192;
   if (PATH) {

@@ -554,7 +554,7 @@ def test_lookup_lanes_per_chain_jacobian_agree(gpu):
     atmospheres x 32 tangent heights (T and H2O columns) agree between that
     batch alone (8 ray blocks: four lanes) and inside one of 80 atmospheres
     (40 blocks, more than the four-lane grid's 5120 wavefronts: one lane);
-    both run the one-sweep adjoint."""
+    both run the adjoint with one workgroup per row."""
     torch = pytest.importorskip("torch")
     ctl = scenes.limb_3gas_ctl()
     ctl.rett_zmin, ctl.rett_zmax = -100.0, 100.0
@@ -628,6 +628,7 @@ def test_radiance_waves_per_path_agree(gpu, nr):
     limb = scenes.limb_geometry(800.0, np.linspace(5.0, 60.0, nr))
     down = scenes.nadir_geometry(800.0, np.linspace(0.0, 50.0, nr))
     geom = {k: np.where(np.arange(nr) % 2 == 1, limb[k], down[k]) for k in limb}
+    rads = []
     for prec in (abi.JUR_FP64, abi.JUR_FP32):
         ref = {}
         for eps in (1.0, 0.8):
@@ -644,6 +645,7 @@ def test_radiance_waves_per_path_agree(gpu, nr):
         nu = np.array([ctl.nu[i] for i in range(ctl.nd)])[:, None]
         emis = -0.2 * c1 * nu ** 3 / np.expm1(c2 * nu / 290.0) * t0
         change = r0 - ref[1.0][0]
+        rads.append(r0)
         k = np.arange(0, nr, 2)
         assert (np.abs(change - emis)[:, k].max(axis=1) > 1e-6 * r0[:, k].max(axis=1)).any()
         for blocks in (19, 100):
@@ -656,6 +658,8 @@ def test_radiance_waves_per_path_agree(gpu, nr):
             for q in (0, n // 2, n - 1):
                 r1, t1 = abi.obs_arrays(obss[q], ctl)
                 assert np.array_equal(r0, r1) and np.array_equal(t0, t1), (prec, blocks, q)
+    # FP32 against FP64: some 1e-6 (float segments of ~1000 points)
+    np.testing.assert_allclose(rads[1], rads[0], rtol=1e-5, atol=1e-7 * rads[0].max())
 
 
 @pytest.mark.parametrize("nray", [3, 5600])

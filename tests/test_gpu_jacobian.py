@@ -378,13 +378,14 @@ def _nadir_batch(ctl, nprof, nang, torch):
 
 
 def test_adjoint_path_batch_regimes_agree(gpu):
-    """The adjoint of the refracted path runs two ways: four channels per
-    lane sharing each step's coefficients for large batches, one channel per
-    lane with the next step's inputs loaded ahead for small ones.  The K rows
-    of the same rays agree between a batch of 688 atmospheres x 8 views with
-    96 channels (the first way) and one of its first 64 atmospheres (the
-    second); each lane's arithmetic is its own, so only the T and p columns'
-    order of additions may differ."""
+    """The FP32 Jacobian with the refracted path runs two ways: a workgroup
+    per row (64 rays, channel) below 8192 rows, and above it separate kernels
+    for the accumulation, the emitter chains and the path, the last with four
+    channels per lane sharing each step's coefficients.  The K rows of the
+    same rays agree between a batch of 688 atmospheres x 8 views with 96
+    channels (88 blocks x 96 rows: the separate kernels) and one of its first
+    64 atmospheres (768 rows); the two add a column's terms in different
+    orders."""
     torch = pytest.importorskip("torch")
     ctl = scenes.nadir_jac_ctl(96)
     assert ctl.refrac == 1
@@ -414,9 +415,9 @@ def test_adjoint_path_batch_regimes_agree(gpu):
     np.testing.assert_allclose(k1, k0, rtol=1e-12, atol=1e-12 * np.abs(k0).max())
 
 
-def _device_jacobian(gpu, ctl, batch, precision, torch):
+def _device_jacobian(gpu, ctl, batch, precision, torch, rows=None):
     """K, radiances and transmittances of a _nadir_batch: ([ray][channel][n],
-    [ray][channel] twice)."""
+    [ray][channel] twice); of its first and last `rows` rays if given."""
     atms, a_d, prof_d, geom_d, nray = batch
     xm, n = gpu.state_map(ctl, atms[0])
     rad = torch.zeros(nray, ctl.nd, dtype=torch.float64, device="cuda:0")
@@ -430,7 +431,7 @@ def _device_jacobian(gpu, ctl, batch, precision, torch):
         torch.cuda.synchronize()
     finally:
         ctx.close()
-    return k.cpu().numpy(), rad.cpu().numpy(), tau.cpu().numpy()
+    return tuple((x if rows is None else torch.cat([x[:rows], x[-rows:]])).cpu().numpy() for x in (k, rad, tau))
 
 
 def test_fp32_partials_at_knots(gpu):
@@ -468,3 +469,66 @@ def test_fp32_jacobian_repeats(gpu, refrac):
     assert np.isfinite(k0).all() and np.abs(k0).max() > 0
     for _ in range(5):
         assert np.array_equal(_device_jacobian(gpu, ctl, batch, abi.JUR_FP32, torch)[0], k0)
+
+
+@pytest.mark.parametrize("gases", [1, 3, 4])
+@pytest.mark.parametrize("refrac", [0, 1])
+def test_adjoint_row_form_all_terms(gpu, tmp_path, gases, refrac):
+    """The FP32 Jacobian's two forms (see
+    test_adjoint_path_batch_regimes_agree) with everything that moves K on:
+    a reflecting surface with the sun (sftype 3), surface emissivities and
+    temperature, clouds, an extinction window, p, T and every emitter in the
+    state, one to four emitters.  512 rays of 12 channels alone (96 rows) and
+    tiled 86 times (688 blocks x 12 = 8256 rows): the radiances and every
+    column of K agree, first and last copy, to the rounding of sums of ~1000
+    FP64 terms in different orders (1e-12 of a column's largest entry, times
+    10 for cancellation)."""
+    torch = pytest.importorskip("torch")
+    names = ["CO2", "H2O", "O3", "CH4"][:gases]
+    nus = [650.0 + 60.0 * i for i in range(12)]
+    p, _, u = scenes.table_grids()
+    grids = (p, np.linspace(160.0, 340.0, 8), u[::5])
+    tb = scenes.write_scene_tables(str(tmp_path / "row"), names, nus, grids=grids)
+    ctl = abi.make_ctl(names, nus, tblbase=tb, tblfmt=2, ctm_co2=1, ctm_h2o=1, ctm_n2=1, ctm_o2=1)
+    ctl.refrac, ctl.sftype, ctl.sfsza = refrac, 3, 30.0
+    ctl.ncl, ctl.nsf, ctl.nw = 2, 2, 1
+    ctl.clnu[0], ctl.clnu[1], ctl.sfnu[0], ctl.sfnu[1] = 600.0, 1400.0, 600.0, 1400.0
+    ctl.retp_zmin, ctl.retp_zmax, ctl.rett_zmin, ctl.rett_zmax = -100, 100, -100, 100
+    ctl.retk_zmin[0], ctl.retk_zmax[0] = -100, 100
+    for g in range(gases):
+        ctl.retq_zmin[g], ctl.retq_zmax[g] = -100, 100
+    ctl.ret_clz = ctl.ret_cldz = ctl.ret_clk = ctl.ret_sft = ctl.ret_sfeps = 1
+    _, _, prof_d, geom_d, _ = _nadir_batch(scenes.nadir_jac_ctl(4), 64, 8, torch)
+    atms = (abi.atm_t * 64)()
+    for k in range(64):
+        a = scenes.make_profile_atm(names, iprof=k)
+        a.clz, a.cldz, a.clk[0], a.clk[1] = 8.0, 1.5, 0.02, 0.03
+        a.sft, a.sfeps[0], a.sfeps[1] = 290.0, 0.9, 0.8
+        for ip in range(a.np):
+            a.k[0][ip] = 1e-3 * np.exp(-a.z[ip] / 10)
+        atms[k] = a
+    a_d = torch.from_numpy(np.frombuffer(bytes(atms), dtype=np.uint8).copy()).to("cuda:0")
+    out = []
+    for tiles in (1, 86):
+        batch = (atms, a_d, prof_d.repeat(tiles), geom_d.repeat(tiles, 1).contiguous(), 512 * tiles)
+        k, rad, tau = _device_jacobian(gpu, ctl, batch, abi.JUR_FP32, torch, rows=512)
+        out.append((k, rad, tau))
+    (k0, r0, t0), (k1, r1, t1) = out
+    col = np.abs(k0).max(axis=(0, 1))
+    assert np.isfinite(k0).all() and (col > 0).mean() > 0.95
+    # each column against FP64: a ray on the other side of a knot (a factor 2.0
+    # apart here, eps ~ u^0.8) is off by up to 13%, one such ray of the 512 by
+    # 0.13 / sqrt(512) = 6e-3 of a column's norm, several of them or a ray of
+    # more than its share by some times that; and rounding of the block's
+    # largest column (float partials, 1e-6 of a row, of terms that cancel
+    # down to 1e-2 of theirs)
+    k64 = _device_jacobian(gpu, ctl, (atms, a_d, prof_d, geom_d, 512), abi.JUR_FP64, torch)[0]
+    err, ref = np.linalg.norm(k0[:512] - k64, axis=(0, 1)), np.linalg.norm(k64, axis=(0, 1))
+    nlev = 81 * (3 + gases)
+    top = np.append(np.repeat(ref[:nlev].reshape(-1, 81).max(axis=1), 81), ref[nlev:])
+    assert len(ref) == nlev + 7 and (err <= 3e-2 * ref + 1e-4 * top).all()
+    for c in range(2):  # the first and the last copy
+        np.testing.assert_allclose(r1[c * 512:c * 512 + 512], r0[:512], rtol=1e-12)
+        np.testing.assert_allclose(t1[c * 512:c * 512 + 512], t0[:512], rtol=1e-12, atol=1e-30)
+        err = np.abs(k1[c * 512:c * 512 + 512] - k0[:512]).max(axis=(0, 1))
+        assert (err <= 1e-11 * col).all(), (np.argmax(err / np.maximum(col, 1e-300)), (err / np.maximum(col, 1e-300)).max())
