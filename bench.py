@@ -50,17 +50,19 @@ sys.path.insert(0, ROOT)
 
 METRIC = "radiances/s fwd; Jacobians/s adjoint vs FD; p50/p99 retrieval latency"
 HBM_PEAK = 8.0e12
-# Vector-instruction issue peak of one MI355X: 256 CUs x 2.4 GHz, one wave64
-# VALU instruction per CU per cycle (four SIMD16 units, four cycles each).
+# Vector-instruction issue rate of one MI355X at its nominal clock: 256 CUs x
+# 2.4 GHz, one wave64 VALU instruction per CU per cycle (four SIMD16 units, four
+# cycles each).
 VALU_PEAK = 256 * 2.4e9
-# Counters of one k_lookup_f32 launch at the default workload (4096
-# profiles), from rocprofv3 --pmc runs of this script
-# (profiles/k_lookup_f32_limb_4096x32x12_counters.md): SQ_INSTS_VALU and
+# The lookup kernel of the default workload (FP32 EGA on tables of one grid,
+# large batch) and the counters of one launch at 4096 profiles, from rocprofv3
+# --pmc runs of this script (the profile named here): SQ_INSTS_VALU and
 # SQ_INSTS_VMEM_RD summed over the launch (wave instructions), and HBM bytes
 # = FETCH_SIZE x 2.000 + WRITE_SIZE x 1.000 KiB x 1024 (factors from a 1 GiB
 # device copy under the same counters).  Other workload sizes report null.
-LOOKUP_F32_COUNTERS = {"nprof": 4096, "valu": 3.0198e10, "vmem_rd": 1.3640e9, "hbm_bytes": 39.37e9,
-                       "profile": "profiles/k_lookup_f32_limb_4096x32x12_counters.md"}
+LOOKUP_F32_COUNTERS = {"kernel": "k_lookup_f32_cell<false, 1>", "nprof": 4096, "valu": 1.8676e10,
+                       "vmem_rd": 9.274e8, "hbm_bytes": 80.93e9,
+                       "profile": "profiles/k_lookup_f32_cell_limb_4096x32x12_counters.md"}
 NPROF, NRAY_PER, GASES = 4096, 32, ["CO2", "H2O", "O3"]
 
 
@@ -136,24 +138,26 @@ def cpu_baseline(nsample):
 
 
 def lookup_roofline(nprof, nray, nd, mean_np, kms):
-    """Roofline of the dominant forward kernel, k_lookup_f32 (one launch per
-    pass; its time from HIP events on the library's stream).
+    """Roofline of the dominant forward kernel, the FP32 lookups (one launch
+    per pass; its time from HIP events on the library's stream).
 
     `bound`/`achieved`/`frac` are HBM: the bytes the kernel must move at least
-    (every LOS field it reads once, the tables once, the path-emissivity
-    write) per second of its time, against 8 TB/s; `traffic` is the HBM bytes
-    per launch of the committed counter profile.  The kernel's limiter is
-    vector-instruction issue, reported beside it (`issue`): SQ_INSTS_VALU of
-    the same profile per second of the measured time against VALU_PEAK.  The
-    per-lookup gather model (176 B per (segment, channel, emitter): 4 corners
-    x 2 float brackets of 16 B plus the p and two T brackets, 48 B) is mostly
-    served by L2, so its rate is not an HBM figure."""
+    (each LOS point's cell record, 16 B, and column densities once, the tables
+    once, the path-emissivity write) per second of its time, against 8 TB/s;
+    `traffic` is the HBM bytes per launch of the committed counter profile
+    (every channel's chains read the records and column densities again).
+    What limits the kernel is vector-instruction issue and the L1's lookup
+    rate; the issue is reported beside it (`issue`): SQ_INSTS_VALU of the same
+    profile per second of the measured time against VALU_PEAK.  The per-lookup
+    gather model (120 B per (segment, channel, emitter): 4 corners x 24 B of
+    knots, the cell record and the column density) is mostly served by L1 and
+    L2, so its rate is not an HBM figure."""
     t = kms[1] * 1e-3
     n_chain = nray * mean_np * nd * len(GASES)         # (ray, point, channel, emitter) steps
-    unique = nray * mean_np * (2 + len(GASES)) * 8 + n_chain * 4 + 36 * 40 * 20 * 200 * 16
-    gather = n_chain * 176
+    unique = nray * mean_np * (16 + len(GASES) * 8) + n_chain * 4 + 36 * 40 * 20 * 202 * 8
+    gather = n_chain * 120
     cnt = LOOKUP_F32_COUNTERS if nprof == LOOKUP_F32_COUNTERS["nprof"] else None
-    r = {"kernel": "k_lookup_f32<false, false>", "kernel_ms": kms[1],
+    r = {"kernel": LOOKUP_F32_COUNTERS["kernel"], "kernel_ms": kms[1],
          "kernel_ms_all": {"raytrace": kms[0], "lookup": kms[1], "accumulate": kms[2]},
          "bound": "hbm", "achieved": unique / t / 1e9, "peak": HBM_PEAK / 1e9, "unit": "GB/s",
          "frac": unique / t / HBM_PEAK, "traffic": cnt["hbm_bytes"] if cnt else None}
@@ -167,8 +171,8 @@ def lookup_roofline(nprof, nray, nd, mean_np, kms):
                 "measured_bytes": cnt["hbm_bytes"] if cnt else None,
                 "measured_GBps": cnt["hbm_bytes"] / t / 1e9 if cnt else None,
                 "peak_GBps": HBM_PEAK / 1e9}
-    r["gather_model"] = {"bytes_per_lookup": 176, "bytes_per_launch": gather, "GBps": gather / t / 1e9,
-                         "note": "algorithmic gather bytes; L2 serves most of them, so this rate is "
+    r["gather_model"] = {"bytes_per_lookup": 120, "bytes_per_launch": gather, "GBps": gather / t / 1e9,
+                         "note": "algorithmic gather bytes; L1 and L2 serve most of them, so this rate is "
                                  "not HBM traffic"}
     r["counters_profile"] = cnt["profile"] if cnt else None
     return r

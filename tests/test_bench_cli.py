@@ -24,3 +24,16 @@ def test_help_lists_the_contract_flags():
     assert r.returncode == 0
     for flag in ("--gpus", "--steps", "--warmup", "--serve-lanes", "--serve-path-split"):
         assert flag in r.stdout
+
+
+def test_roofline_names_the_profiled_kernel():
+    """The roofline's counters are those of the kernel it names: the profile
+    that it cites names that kernel, and at the 32.0 ms the launch took under
+    the counters its instructions stay below the nominal issue rate."""
+    import bench
+    r = bench.lookup_roofline(4096, 131072, 12, 890.85, [6.2, 32.0, 8.0])
+    text = open(os.path.join(ROOT, r["counters_profile"])).read()
+    assert r["kernel"] in text
+    assert 0.5 < r["issue"]["frac"] < 1.0
+    assert r["hbm"]["unique_bytes"] < r["hbm"]["measured_bytes"]
+    assert bench.lookup_roofline(64, 2048, 12, 890.85, [6.2, 32.0, 8.0])["counters_profile"] is None
