@@ -539,42 +539,6 @@ __device__ __forceinline__ double col_u(Col col, int n, double x, int mono, int 
   return lin_f(r.y, r.x, r.w, r.z, x);
 }
 
-// Table cell of a (p, T) point: pressure bracket ipr and the temperature
-// brackets it0, it1 of the two pressure levels (intpol_tbl_ega,
-// src/jurassic.c:3826-3832).  ok is false when a temperature row has fewer
-// than two entries (the reference then uses eps = 0).
-struct Cell {
-  int ipr, it0, it1;
-  bool ok;
-  double pa, pb;     // p[ipr], p[ipr+1]
-  double ta0, tb0;   // t[ipr][it0], t[ipr][it0+1]
-  double ta1, tb1;   // t[ipr+1][it1], t[ipr+1][it1+1]
-};
-
-__device__ __forceinline__ Cell locate_cell(const TabView &T, int tix, int npt, double p, double t) {
-  Cell c;
-  const double *pg = T.p + (size_t)tix * T.TP;
-  c.ipr = locate_irr(pg, npt, p);
-  c.pa = pg[c.ipr];
-  c.pb = pg[c.ipr + 1];
-  const int *ntp = T.nt + (size_t)tix * T.TP;
-  const int nt0 = ntp[c.ipr], nt1 = ntp[c.ipr + 1];
-  c.ok = (nt0 >= 2 && nt1 >= 2);
-  c.it0 = c.it1 = 0;
-  c.ta0 = c.tb0 = c.ta1 = c.tb1 = 0;
-  if (c.ok) {
-    const double *tg0 = T.t + ((size_t)tix * T.TP + c.ipr) * T.TT;
-    const double *tg1 = tg0 + T.TT;
-    c.it0 = locate_reg(tg0, nt0, t);
-    c.it1 = locate_reg(tg1, nt1, t);
-    c.ta0 = tg0[c.it0];
-    c.tb0 = tg0[c.it0 + 1];
-    c.ta1 = tg1[c.it1];
-    c.tb1 = tg1[c.it1 + 1];
-  }
-  return c;
-}
-
 // One EGA growth step on one table column, FP64 path: eps(u(x) + u_seg) with
 // the reference's operations (u_from_rec and eps_from_rec; below the first
 // knot their LIN through the origin is the bracket of the column's origin).
@@ -630,11 +594,6 @@ template <int X, typename V>
 __device__ __forceinline__ V quad_xor(V v) {
   return quad_dpp<(0 ^ X) | (1 ^ X) << 2 | (2 ^ X) << 4 | (3 ^ X) << 6>(v);
 }
-
-// Per-(channel, emitter) table constants, loaded once per wavefront.
-struct GasConst {
-  int tix, npt, mono;
-};
 
 // ------------------------------------------------------------------
 // Continua (formod_continua, src/jurassic.c:3075-3117, with ctmco2
@@ -829,17 +788,6 @@ __device__ __forceinline__ bool xcd_block_map(int wg, int G, int nblk, int &blk,
 }
 
 __host__ __device__ __forceinline__ int padded_blocks(int nblk) { return (nblk + 7) & ~7; }
-
-// Contiguous-range remap (kept for kernels without a per-block structure).
-__device__ __forceinline__ int xcd_remap(int wg, int nwg) {
-  constexpr int NX = 8;
-  const int per = nwg / NX, rem = nwg % NX;
-  const int x = wg % NX, k = wg / NX;
-  // XCD x owns logical range [x*per + min(x, rem), ...) of length per + (x < rem)
-  if (k < per) return x * per + (x < rem ? x : rem) + k;
-  // tail ids (k == per) exist only for x < rem
-  return x * per + x + k;
-}
 
 // ------------------------------------------------------------------
 // Sums along a path in chunks of RAD_CH points (the FP32 radiance kernel): each

@@ -254,7 +254,7 @@ struct jur_ctx {
   jur::DevBuf<double> d_p, d_t;
   jur::DevBuf<float2> d_kn;
   int TP = 2, TT = 2, TU = 2, TS = 4;
-  int shared = 0, ref_tix = 0, all_mono = 1, cells = 0;
+  int ref_tix = 0, all_mono = 1, cells = 0;
   size_t table_bytes = 0;
   // model constants
   jur::DevBuf<double> d_st, d_sr, d_clnu, d_sfnu, d_ctm;

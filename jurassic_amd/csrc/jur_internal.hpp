@@ -65,14 +65,12 @@ struct TabView {
   const int *pdir;         // [ng][nd]: +1/-1 strictly ascending/descending p grid,
                            // 0 otherwise (search by bisection)
   int all_mono;            // 1 if mono is 1 for every table with np >= 30
-  int shared;              // 1 if every table with np >= 30 has the same p grid,
-                           // T-grid sizes and T grids (one cell search per
-                           // segment serves all of them)
-  int ref_tix;             // a table holding the shared grids
-  int cells;               // 1 if the tables are shared and all_mono, on a strictly
-                           // monotone p grid, and every row and column of them has
-                           // two entries: a cell is then the same for all of them
+  int cells;               // 1 if every table with np >= 30 has the same, strictly
+                           // monotone p grid and the same T grids, all are
+                           // monotone, and every row and column of them has two
+                           // entries: a cell is then the same for all of them
                            // and never without data
+  int ref_tix;             // a table holding the shared grids
   // column c = (table * TP + p) * TT + T
   __device__ __forceinline__ Col col(size_t c) const { return Col{kn + c * TS + 1}; }
 };

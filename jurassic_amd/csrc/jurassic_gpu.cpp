@@ -270,14 +270,14 @@ static int locate_irr_h(const double *xx, int n, double x) {
 namespace jur {
 
 // Shared grids: every table with np >= 30 has the same p grid, T-row sizes
-// and T grids as the first such table (one cell search per segment then
-// serves all of them).
+// and T grids as the first such table (one cell per LOS point then serves all
+// of them, see TabView::cells).
 static void detect_shared(jur_ctx *c, const std::vector<int> &h_np, const std::vector<int> &h_nt,
                           const std::vector<int> &h_nu, const std::vector<int> &h_pdir,
                           const std::vector<double> &h_p, const std::vector<double> &h_t) {
   const size_t ntab = (size_t)c->s.nd * c->s.ng;
   const int TP = c->TP, TT = c->TT;
-  c->shared = c->cells = 0;
+  c->cells = 0;
   c->ref_tix = 0;
   int ref = -1;
   for (size_t k = 0; k < ntab; k++)
@@ -293,7 +293,6 @@ static void detect_shared(jur_ctx *c, const std::vector<int> &h_np, const std::v
         if (h_t[(k * TP + ip) * TT + it] != h_t[(ref * TP + ip) * TT + it]) same = false;
     }
   }
-  c->shared = same ? 1 : 0;
   c->ref_tix = ref;
   // cells located once for all tables: none without data, columns in 16 bits
   c->cells = same && c->all_mono && h_pdir[ref] != 0 && TP * TT <= 65536;
@@ -615,7 +614,6 @@ static ModelView model_view(const jur_ctx *c) {
   T.kn = c->d_kn.p;
   T.mono = c->d_mono.p;
   T.pdir = c->d_pdir.p;
-  T.shared = c->shared;
   T.ref_tix = c->ref_tix;
   T.all_mono = c->all_mono;
   T.cells = c->cells;
