@@ -576,7 +576,8 @@ __global__ __launch_bounds__(WAVE) void k_ray_finish(ModelView M, BatchView B, L
 // some twenty stores of every step's chain: 1.90 ms for 10 nadir rays (805
 // steps, one emitter) against 0.95 + 0.02 here, 4.27 against 1.93 + 0.04 for
 // 77 x 5 limb rays of three emitters; for 4096 x 32 of them 7.1 against 3.7 +
-// 4.1 ms (bound by the stores).
+// 4.1 ms (bound by the stores).  (The march has since become faster: 0.66, 1.32
+// and 2.6 ms; the points of the large batch take 3.7.)
 constexpr int RP_STEPS = 16;
 
 __global__ __launch_bounds__(WAVE) void k_ray_points(ModelView M, BatchView B, LosView L, const RayInfo *info,
