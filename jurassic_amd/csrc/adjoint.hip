@@ -2189,7 +2189,7 @@ __global__ __launch_bounds__(4 * WAVE, 2) void k_adj_row(ModelView M, BatchView 
   if (sft_los) {
     lv_sf = level_of(atm, LOSR(F_Z, N - 1), -1, w_sf);
     gz_sft = sft_bar * (atm->t[lv_sf + 1] - atm->t[lv_sf]) / (atm->z[lv_sf + 1] - atm->z[lv_sf]);
-    // its T columns, before the other waves add to them (from round 2 on)
+    // its T columns, before the other waves begin to add to them
     int c;
     if (map && (c = xm[JUR_XMAP_LEV(1, lv_sf)]) >= 0) unsafeAtomicAdd(&KT(c), (1 - w_sf) * sft_bar);
     if (map && (c = xm[JUR_XMAP_LEV(1, lv_sf + 1)]) >= 0) unsafeAtomicAdd(&KT(c), w_sf * sft_bar);
